@@ -850,17 +850,27 @@ void prepare(System &S, const EwaldParams &P, EwaldState &E)
     E.chi.ensure(n);
     E.red.ensure(16);
     if (!P.on) return;
+    if (E.planned_n != n) E.dirty = true;   // the choice below depends on it
     if (E.dirty) {
         E.sk_valid = false;
+        E.planned_n = n;
+        E.mesh_on = mesh_suits(n, P, S.geom, E.volume);
         // k-vectors in the reference's loop order (Potentials.f90:1526-1548)
         const double pi = 4.0 * std::atan(1.0);
         double rcl[9];
         for (int q = 0; q < 9; ++q) rcl[q] = 2 * pi * S.geom.inv[q];
         Consts c = consts_of(P, E.volume);
+        for (int q = 0; q < 9; ++q) {
+            E.b[q] = rcl[q];
+            E.f[q] = S.geom.inv[q];
+        }
+        PYSIC_REQUIRE(P.K[0] < 1024 && P.K[1] < 1024 && P.K[2] < 1024, PYSIC_EINVAL,
+                      "at most 1023 reciprocal cells along each axis");
+        if (E.mesh_on) mesh_plan(S, P, E.mesh, E.b, c.inv_eps_2v);
         double kc2 = P.kc * P.kc;
         std::vector<double4> kv;
         std::vector<int4> segs;   // {k1, k2, k3 start | len << 16, first k index}
-        for (int k1 = -P.K[0]; k1 <= P.K[0]; ++k1)
+        for (int k1 = -P.K[0]; k1 <= P.K[0] && !E.mesh_on; ++k1)
             for (int k2 = -P.K[1]; k2 <= P.K[1]; ++k2)
                 for (int k3 = 0; k3 <= P.K[2]; ++k3) {
                     if (k1 == 0 && k2 == 0 && k3 == 0) continue;
@@ -882,12 +892,6 @@ void prepare(System &S, const EwaldParams &P, EwaldState &E)
                     }
                     if (!extend) segs.push_back(make_int4(k1, k2, k3 | (1 << 16), idx));
                 }
-        PYSIC_REQUIRE(P.K[0] < 1024 && P.K[1] < 1024 && P.K[2] < 1024, PYSIC_EINVAL,
-                      "at most 1023 reciprocal cells along each axis");
-        for (int q = 0; q < 9; ++q) {
-            E.b[q] = rcl[q];
-            E.f[q] = S.geom.inv[q];
-        }
         E.nseg = (int)segs.size();
         std::vector<int> plan, flags;
         build_plan(segs, plan, flags);
@@ -940,11 +944,23 @@ Recip recip_of(const EwaldState &E)
     return R;
 }
 
+// Whether there is a reciprocal sum at all.
+bool has_recip(const EwaldState &E) { return E.mesh_on || E.nk > 0; }
+
 // S(k) into E.sk; also leaves the per-atom phase table E.th that
-// recip_atoms reads.
-void structure_factors(System &S, EwaldState &E)
+// recip_atoms reads.  Over the mesh: S(k) as the field's coefficients.
+// placed: the atoms have not moved since the last call.
+void structure_factors(System &S, EwaldState &E, bool placed = false)
 {
     const int n = S.n, nk = E.nk;
+    if (E.mesh_on) {
+        hipEvent_t ev;
+        S.timer.begin("ewald_sk", S.stream, &ev);
+        if (!placed) mesh_place(S, E.mesh, E.f);
+        mesh_structure(S, E.mesh, E.f, E.scaler.p);
+        S.timer.end("ewald_sk", S.stream, ev);
+        return;
+    }
     if (nk == 0) return;
     int stiles = div_up(E.nwaves, EB / 64);
     int nchunk = std::max(1, std::min(div_up(n, EB), div_up(2048, stiles)));
@@ -966,11 +982,29 @@ void structure_factors(System &S, EwaldState &E)
     S.timer.end("ewald_sk", S.stream, ev);
 }
 
+// the virial block partials of a per-atom pass, summed
+void sum_stress(System &S, EwaldState &E, int blocks, double *stress6)
+{
+    k_sum_partials<<<1, EB, 0, S.stream>>>(blocks, 8, 6, E.part.p, E.red.p);
+    HIP_TRY(hipMemcpyAsync(stress6, E.red.p, sizeof(double) * 6, hipMemcpyDeviceToHost, S.stream));
+    HIP_TRY(hipStreamSynchronize(S.stream));
+}
+
 // mode 2: add forces + return stress; mode 3: add into chi.  Needs the
 // structure factors and phase table of the current positions.
 void recip_atoms(System &S, EwaldState &E, int mode, double *stress6)
 {
     const int n = S.n, nk = E.nk;
+    if (E.mesh_on) {
+        const int tiles = div_up(n, EB);
+        E.part.ensure((size_t)tiles * 8);
+        hipEvent_t ev;
+        S.timer.begin(mode == 3 ? "ewald_chi" : "ewald_force", S.stream, &ev);
+        mesh_atoms(S, E.mesh, E.f, E.scaler.p, mode == 2, E.chi.p, E.part.p);
+        S.timer.end(mode == 3 ? "ewald_chi" : "ewald_force", S.stream, ev);
+        if (mode == 2) sum_stress(S, E, tiles, stress6);
+        return;
+    }
     const int atiles = div_up(n, 16 * (EB / 64));
     int nchunk = std::max(1, std::min(E.nwaves, div_up(4096, atiles)));
     const int wchunk = div_up(E.nwaves, nchunk);
@@ -1000,13 +1034,7 @@ void recip_atoms(System &S, EwaldState &E, int mode, double *stress6)
                                                 E.part.p);
     HIP_TRY(hipGetLastError());
     S.timer.end(mode == 3 ? "ewald_chi" : "ewald_force", S.stream, ev);
-    if (mode == 2) {
-        k_sum_partials<<<1, EB, 0, S.stream>>>(ftiles, 8, 6, E.part.p, E.red.p);
-        double h[6];
-        HIP_TRY(hipMemcpyAsync(h, E.red.p, sizeof(double) * 6, hipMemcpyDeviceToHost, S.stream));
-        HIP_TRY(hipStreamSynchronize(S.stream));
-        for (int c = 0; c < 6; ++c) stress6[c] = h[c];
-    }
+    if (mode == 2) sum_stress(S, E, ftiles, stress6);
 }
 
 unsigned long long state_hash(System &S, EwaldState &E)
@@ -1083,7 +1111,8 @@ void real_pass(System &S, const EwaldParams &P, EwaldState &E, int mode, double 
 
 // Electronegativities into E.chi without a host round trip: the charge sum
 // and the background term stay on the device.
-void chi_eval(System &S, const EwaldParams &P, EwaldState &E)
+// placed: the atoms have not moved since the previous evaluation.
+void chi_eval(System &S, const EwaldParams &P, EwaldState &E, bool placed = false)
 {
     const double *bg_dev = nullptr;
     if (P.on) {
@@ -1098,9 +1127,9 @@ void chi_eval(System &S, const EwaldParams &P, EwaldState &E)
         bg_dev = E.red.p + 12;
     }
     real_pass(S, P, E, 3, 0.0, nullptr, bg_dev);
-    if (P.on && E.nk > 0) {
+    if (P.on && has_recip(E)) {
         // the relaxation changes the charges every step: no fingerprint
-        structure_factors(S, E);
+        structure_factors(S, E, placed);
         E.sk_valid = false;
         recip_atoms(S, E, 3, nullptr);
     }
@@ -1128,6 +1157,7 @@ void ewald_release(EwaldState &E)
     E.zw.release();
     E.kpk.release();
     E.hpart.release();
+    mesh_release(E.mesh);
     E.sk_valid = false;
 }
 
@@ -1160,12 +1190,16 @@ double energy_terms(System &S, const EwaldParams &P, EwaldState &E, bool with_se
         charge_sums(S, E, qs);
         e += -qs[1] * c.inv_eps_4pi * c.inv_sig_sqrt2pi;                         // self
         e += -qs[0] * qs[0] * 0.5 * c.inv_eps_2v * P.sigma * P.sigma;            // background
-        if (E.nk > 0) {
+        if (has_recip(E)) {
             current_structure_factors(S, E);
-            int nb = div_up(E.nk, EB);
-            E.part.ensure((size_t)nb);
-            k_recip_energy<<<nb, EB, 0, S.stream>>>(E.nk, E.kvec.p, E.sk.p, E.part.p);
-            k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 1, 1, E.part.p, E.red.p);
+            if (E.mesh_on) {
+                k_sum_partials<<<1, EB, 0, S.stream>>>(E.mesh.nepart, 1, 1, E.mesh.epart.p, E.red.p);
+            } else {
+                int nb = div_up(E.nk, EB);
+                E.part.ensure((size_t)nb);
+                k_recip_energy<<<nb, EB, 0, S.stream>>>(E.nk, E.kvec.p, E.sk.p, E.part.p);
+                k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 1, 1, E.part.p, E.red.p);
+            }
             double er;
             HIP_TRY(hipMemcpyAsync(&er, E.red.p, sizeof(double), hipMemcpyDeviceToHost, S.stream));
             HIP_TRY(hipStreamSynchronize(S.stream));
@@ -1193,7 +1227,7 @@ void ewald_add_forces(System &S, const EwaldParams &P, EwaldState &E, double *st
     double r7[7];
     real_pass(S, P, E, 2, 0.0, r7);
     for (int c = 0; c < 6; ++c) stress[c] = r7[1 + c];
-    if (P.on && E.nk > 0) {
+    if (P.on && has_recip(E)) {
         current_structure_factors(S, E);
         double st[6];
         recip_atoms(S, E, 2, st);
@@ -1224,7 +1258,7 @@ void ewald_relax(System &S, const EwaldParams &P, EwaldState &E, double *rates, 
     const double dt2 = dt * dt, inv_mq = 1.0 / inertia;
     const double future = 1.0 / (1.0 + 0.5 * friction * dt);
     auto dchi_of_q = [&](int update) {
-        chi_eval(S, P, E);
+        chi_eval(S, P, E, update != 0);
         E.part.ensure((size_t)nb * 8);
         k_sum_chi<<<nb, EB, 0, S.stream>>>(n, E.chi.p, E.part.p);
         k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 1, E.part.p, E.red.p);

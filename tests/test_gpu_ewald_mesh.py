@@ -1,0 +1,179 @@
+"""GPU parity of the reciprocal sums over the mesh (mesh.hip), which take over
+from the ion-by-ion sums at 1e8 pairs of an ion and a k-vector.
+
+Reference: the oracle for everything but the reciprocal terms (it is given no
+reciprocal cells), plus the reciprocal sums term by term in numpy's FP64
+(Potentials.f90:1428-2249 as matrix products).
+
+Tolerance 1e-12 of the largest value: a phase 2 pi k.u carries a rounding of
+2 pi K eps = 4e-14 at the largest K = 54 here in either sum, and 25 times that
+covers the mesh's weights and the sums' order.
+"""
+import numpy as np
+import pytest
+
+from helpers import rel_maxnorm
+
+pytestmark = pytest.mark.gpu
+EPS = 0.00552635
+TOL = 1e-12
+
+
+def kcells(cell, kc):
+    rec = 2 * np.pi * np.linalg.inv(cell).T
+    vol = rec[0] @ np.cross(rec[1], rec[2])
+    return [int(kc * np.linalg.norm(np.cross(rec[(a + 1) % 3], rec[(a + 2) % 3])) / vol + 0.5)
+            for a in range(3)]
+
+
+def reciprocal(pos, qs, cell, K, kc, sigma):
+    """(energy, forces, absolute-position virial, field subtracted from chi)."""
+    inv = np.linalg.inv(cell)
+    b = 2 * np.pi * inv.T
+    u = pos @ inv
+    k = [np.arange(-K[0], K[0] + 1), np.arange(-K[1], K[1] + 1), np.arange(0, K[2] + 1)]
+    ex = []
+    for a in range(3):
+        ph = u[:, a:a + 1] * k[a]
+        ex.append(np.exp(2j * np.pi * (ph - np.rint(ph))))
+    inv2v = 1.0 / (2.0 * abs(np.linalg.det(cell)) * EPS)
+    n = len(pos)
+    energy, field, grad = 0.0, np.zeros(n), np.zeros((n, 3))
+    for a, k1 in enumerate(k[0]):
+        kv = (k1 * b[0] + k[1][:, None, None] * b[1] + k[2][None, :, None] * b[2])
+        k2 = (kv * kv).sum(2)
+        on = (k2 < kc * kc) & (k2 > 0)
+        w = np.where(k[2] == 0, 1.0, 2.0)[None, :]
+        c = np.where(on, inv2v * w * np.exp(-sigma ** 2 * k2 / 2) / np.where(on, k2, 1.0), 0.0)
+        e12 = ex[0][:, a:a + 1] * ex[1]
+        s = (qs[:, None] * e12).T @ ex[2]
+        energy += float((c * np.abs(s) ** 2).sum())
+        z = 2.0 * c * s
+        back = ex[2].conj()
+
+        def at(y):
+            return ((back @ y.T) * e12.conj()).sum(1)
+        field += at(z).real
+        for d in range(3):
+            grad[:, d] += (at(z * kv[..., d]) * -1j).real
+    f = -qs[:, None] * grad
+    st = np.array([pos[:, x] @ f[:, y] for x, y in
+                   ((0, 0), (1, 1), (2, 2), (1, 2), (0, 2), (0, 1))])
+    return energy, f, st, field
+
+
+def ions(case):
+    rng = np.random.default_rng(case["seed"])
+    n = case["n"]
+    u = rng.random((n, 3))
+    # a jittered lattice of distinct sites, so that no two ions coincide
+    m = int(np.ceil(n ** (1 / 3)))
+    site = np.array([(i, j, k) for i in range(m) for j in range(m) for k in range(m)])[:n]
+    u = (site + 0.5 + 0.3 * (u - 0.5)) / m * np.array(case.get("part", (1.0, 1.0, 1.0)))
+    u += rng.integers(-case.get("out", 0), case.get("out", 0) + 1, (n, 3))
+    cell = np.array(case["cell"], dtype=float)
+    if cell.ndim == 1:
+        cell = np.diag(cell)
+    q = rng.choice([-1.0, 1.0], n) * rng.uniform(0.5, 2.0, n)
+    scaler = rng.uniform(0.5, 1.5, n) if case.get("scaled") else None
+    return u @ cell, q, cell, scaler
+
+
+CASES = [
+    # a cube, K = 29: tiles of 128 x 120 x 120 points
+    dict(n=3000, cell=(36.0, 36.0, 36.0), kc=5.0, seed=1),
+    # three different axes, K = 48, 24, 12, more ions than one chunk per tile
+    dict(n=9000, cell=(60.0, 30.0, 15.0), kc=5.0, seed=2),
+    # sheared, ions up to three cells outside, scaled charges that do not cancel
+    dict(n=3500, cell=((36.0, 0.0, 0.0), (9.0, 34.0, 0.0), (-7.0, 5.0, 33.0)), kc=5.2, seed=3,
+         out=3, scaled=True),
+    # everything in one corner: empty tiles and crowded ones
+    dict(n=3001, cell=(40.0, 40.0, 40.0), part=(0.3, 0.35, 0.4), kc=4.6, seed=4),
+    # a flat cell: the smallest mesh an axis can have (24 points)
+    dict(n=8000, cell=(68.0, 64.0, 7.0), kc=5.0, seed=5),
+]
+
+
+@pytest.mark.parametrize("k", range(len(CASES)))
+def test_mesh_matches_term_by_term(oracle, k):
+    from pysic_amd.engine import Engine
+    case = CASES[k]
+    pos, q, cell, scaler = ions(case)
+    n, kc, sigma, rc = len(pos), case["kc"], 1.2, 3.0
+    K = kcells(cell, kc)
+    print("mesh case %d: n=%d K=%s" % (k, n, K), flush=True)
+    sp = np.zeros(n, np.int32)
+    eng = Engine(0)
+    eng.create_atoms(sp, pos, charges=q)
+    eng.create_cell(cell)
+    eng.set_potentials(np.zeros((0, 12)))
+    eng.set_bond_order_factors(np.zeros((0, 14)))
+    eng.set_ewald(rc, kc, K, sigma, EPS, scaler=scaler)
+    eng.generate_neighbor_lists(np.full(n, rc + 0.2))
+    nl = oracle.neighbor_list(pos, cell, [1, 1, 1], np.full(n, rc + 0.2))
+    qs = q if scaler is None else q * scaler
+    ew0 = [1, rc, kc, 0, 0, 0, sigma, EPS]
+    none = np.zeros((0, 12))
+
+    def reference(p):
+        args = (sp, p, q, cell, nl, none, None, ew0, scaler)
+        er, fr, sr, field = reciprocal(p, qs, cell, K, kc, sigma)
+        f, s = oracle.evaluate("forces", *args)
+        return (oracle.evaluate("energy", *args) + er, f + fr, s + sr,
+                oracle.evaluate("enegs", *args) - field)
+
+    def compare(p, order):
+        e0, f0, s0, x0 = reference(p)
+        for what in order:
+            if what == "e":
+                assert abs(eng.energy() - e0) <= TOL * abs(e0)
+            elif what == "f":
+                f, s = eng.forces()
+                print("  forces %.1e" % rel_maxnorm(f, f0), flush=True)
+                assert rel_maxnorm(f, f0) <= TOL
+                # the virial sums n terms r F that may cancel
+                assert np.abs(s - s0).max() <= TOL * np.abs(p).max() * np.abs(f0).sum()
+            else:
+                assert rel_maxnorm(eng.electronegativities(), x0) <= TOL
+
+    compare(pos, "efx")
+    # moved ions: nothing of the old places or structure factors is left
+    moved = pos + np.random.default_rng(9).normal(0.0, 0.02, pos.shape)
+    eng.update_coordinates(moved)
+    compare(moved, "fex")
+    eng.close()
+
+
+def test_relaxation_steps_over_the_mesh():
+    """The relaxation keeps the ions' places on the mesh over its steps: its
+    charges are those of the same steps driven from outside, where every
+    electronegativity call places them again."""
+    from pysic_amd.engine import Engine
+    pos, _, cell, _ = ions(CASES[0])
+    n = len(pos)
+    pd = np.array([[2, 1, 0, 0, 10.0, 2.0, 0, 0, -1, 0, 0, 0]])
+    eng = Engine(0)
+    eng.create_atoms(np.zeros(n, np.int32), pos, charges=np.zeros(n))
+    eng.create_cell(cell)
+    eng.set_potentials(pd)
+    eng.set_bond_order_factors(np.zeros((0, 14)))
+    eng.set_ewald(3.0, 5.0, kcells(cell, 5.0), 1.2, EPS)
+    eng.generate_neighbor_lists(np.full(n, 3.2))
+    q0 = np.random.default_rng(3).normal(0.0, 0.1, n)
+    dt, fr = 0.02, 4.0
+    got, rate, steps, _ = eng.relax_charges(q0, np.zeros(n), 4, dt, 1.0, fr, 1e-14)
+    assert steps == 4
+    q, v = q0.copy(), np.zeros(n)
+
+    def force():
+        eng.update_charges(q)
+        x = eng.electronegativities()
+        return x - x.mean()
+    f = force()
+    for _ in range(4):
+        q = q + v * dt + (f - fr * v) * dt * dt
+        v = (1 - 0.5 * fr * dt) * v + 0.5 * f * dt
+        f = force()
+        v = (v + 0.5 * f * dt) / (1 + 0.5 * fr * dt)
+    assert rel_maxnorm(got, q) <= TOL and rel_maxnorm(rate, v) <= TOL
+    eng.close()
