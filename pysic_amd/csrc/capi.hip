@@ -114,15 +114,15 @@ void KernelTimer::reset()
 
 void System::release_all()
 {
-    DBuf<double4> *b4[] = {&pos, &pos2, &mom, &mom2, &frc, &frc2, &out4};
+    DBuf<double4> *b4[] = {&pos, &pos2, &mom, &mom2, &frc, &frc2};
     for (auto *b : b4) b->release();
-    DBuf<double> *bd[] = {&q, &q2, &cut, &cut2, &partial, &totals, &host_stage, &gpartial,
+    DBuf<double> *bd[] = {&q, &q2, &cut, &cut2, &partial, &totals, &gpartial,
                           &gtotals, &atom_ev, &cell_ev};
     for (auto *b : bd) b->release();
     DBuf<int> *bi[] = {&id, &id2, &key, &key2, &wrap, &wrap2, &perm, &cellcount, &cellstart, &cellfill, &scanblk,
                        &prevstart, &dirty, &scanloc, &srow,
                        &nbr, &nimg, &ncnt, &flags, &sj, &simg, &scnt, &cell_of, &first_bin, &atom0,
-                       &bsj, &bsimg, &bscnt, &osj, &osimg, &oscnt, &qc_check};
+                       &bsj, &bsimg, &bscnt, &osj, &osimg, &oscnt, &qc_check, &inv};
     for (auto *b : bi) b->release();
     bG.release();
     oD.release();
@@ -135,6 +135,7 @@ void System::release_all()
     dpmodel.release();
     tables.release();
     cells.release();
+    link.release();
     order_valid = false;
     bins_clean = false;
 }
@@ -143,18 +144,6 @@ void System::release_all()
 // order-restoring helpers
 // ---------------------------------------------------------------------------
 namespace {
-__global__ void k_gather4(int n, const int *__restrict__ id, const double4 *__restrict__ src,
-                          double4 *__restrict__ dst)
-{
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < n) dst[s] = src[id[s]];
-}
-__global__ void k_gather1(int n, const int *__restrict__ id, const double *__restrict__ src,
-                          double *__restrict__ dst)
-{
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < n) dst[s] = src[id[s]];
-}
 __global__ void k_scatter1(int n, const int *__restrict__ id, const double *__restrict__ src,
                            double *__restrict__ dst)
 {
@@ -513,7 +502,8 @@ void compile_model(pysic_ctx *h)
     h->S.model_dirty = false;
 }
 
-void upload_state(pysic_ctx *h, const double *positions, const double *momenta, bool sorted_by_id)
+// New atoms, slot i = atom i.
+void upload_atoms(pysic_ctx *h, const double *positions, const double *momenta)
 {
     System &S = h->S;
     int n = S.n;
@@ -525,53 +515,9 @@ void upload_state(pysic_ctx *h, const double *positions, const double *momenta, 
                pz = momenta ? momenta[3 * i + 2] : 0.0;
         hm[i] = make_double4(px, py, pz, h->masses[i]);
     }
-    if (!sorted_by_id) {
-        HIP_TRY(hipMemcpyAsync(S.pos.p, hp.data(), sizeof(double4) * n, hipMemcpyHostToDevice, S.stream));
-        HIP_TRY(hipMemcpyAsync(S.mom.p, hm.data(), sizeof(double4) * n, hipMemcpyHostToDevice, S.stream));
-    } else {
-        S.out4.ensure(n);
-        HIP_TRY(hipMemcpyAsync(S.out4.p, hp.data(), sizeof(double4) * n, hipMemcpyHostToDevice, S.stream));
-        k_gather4<<<div_up(n, 256), 256, 0, S.stream>>>(n, S.id.p, S.out4.p, S.pos.p);
-        if (momenta) {   // an update without momenta keeps them
-            HIP_TRY(hipMemcpyAsync(S.out4.p, hm.data(), sizeof(double4) * n, hipMemcpyHostToDevice,
-                                   S.stream));
-            k_gather4<<<div_up(n, 256), 256, 0, S.stream>>>(n, S.id.p, S.out4.p, S.mom.p);
-        }
-    }
+    HIP_TRY(hipMemcpyAsync(S.pos.p, hp.data(), sizeof(double4) * n, hipMemcpyHostToDevice, S.stream));
+    HIP_TRY(hipMemcpyAsync(S.mom.p, hm.data(), sizeof(double4) * n, hipMemcpyHostToDevice, S.stream));
     HIP_TRY(hipStreamSynchronize(S.stream));
-}
-
-void upload_scalar(System &S, const double *host, DBuf<double> &dst)
-{
-    int n = S.n;
-    S.host_stage.ensure(n);
-    HIP_TRY(hipMemcpyAsync(S.host_stage.p, host, sizeof(double) * n, hipMemcpyHostToDevice, S.stream));
-    k_gather1<<<div_up(n, 256), 256, 0, S.stream>>>(n, S.id.p, S.host_stage.p, dst.p);
-    HIP_TRY(hipStreamSynchronize(S.stream));
-}
-
-void download_scalar(System &S, const double *src, double *host)
-{
-    int n = S.n;
-    S.host_stage.ensure(n);
-    k_scatter1<<<div_up(n, 256), 256, 0, S.stream>>>(n, S.id.p, src, S.host_stage.p);
-    HIP_TRY(hipMemcpyAsync(host, S.host_stage.p, sizeof(double) * n, hipMemcpyDeviceToHost, S.stream));
-    HIP_TRY(hipStreamSynchronize(S.stream));
-}
-
-void download_vec3(System &S, const double4 *src, double *host)
-{
-    int n = S.n;
-    S.out4.ensure(n);
-    sys_scatter_original(S, src, S.out4.p);
-    std::vector<double4> tmp(n);
-    HIP_TRY(hipMemcpyAsync(tmp.data(), S.out4.p, sizeof(double4) * n, hipMemcpyDeviceToHost, S.stream));
-    HIP_TRY(hipStreamSynchronize(S.stream));
-    for (int i = 0; i < n; ++i) {
-        host[3 * i] = tmp[i].x;
-        host[3 * i + 1] = tmp[i].y;
-        host[3 * i + 2] = tmp[i].z;
-    }
 }
 
 void require_ready(pysic_ctx *h)
@@ -601,16 +547,12 @@ void require_force_flags(int f3)
                   "the dynamics)");
 }
 
-void check_flags(pysic_ctx *h, bool lists_only)
+void check_flags(const int *f)
 {
-    int f[4];
-    nb_read_flags(h->S, f);
     require_range_flag(f[2]);
-    if (!lists_only) {
-        PYSIC_REQUIRE(f[1] == 0, PYSIC_ECAP,
-                      "Tersoff short list overflow: " + std::to_string(f[1]) + " neighbors");
-        require_force_flags(f[3]);
-    }
+    PYSIC_REQUIRE(f[1] == 0, PYSIC_ECAP,
+                  "Tersoff short list overflow: " + std::to_string(f[1]) + " neighbors");
+    require_force_flags(f[3]);
 }
 
 // Neighbor lists for the current positions; grows the capacity on overflow.
@@ -618,7 +560,7 @@ void build_lists(pysic_ctx *h)
 {
     System &S = h->S;
     for (int attempt = 0; attempt < 4; ++attempt) {
-        HIP_TRY(hipMemsetAsync(S.flags.p, 0, sizeof(int) * 4, S.stream));
+        nb_clear_flags(S);
         nb_sort_atoms(S);
         nb_build_lists(S);
         int f[4];
@@ -653,23 +595,27 @@ void tersoff_energy(pysic_ctx *h)
     ts_reduce(S);
 }
 
-// One evaluation for the API path: if an atom had more short neighbors than
-// the variant holds, switch to a variant that holds them and run again.
-void tersoff_checked(pysic_ctx *h, int mode)
+// One evaluation for the API path, waited for: if an atom had more short
+// neighbors than the variant holds, switch to a variant that holds them and
+// run again.  Returns the totals and flags.
+Report tersoff_checked(pysic_ctx *h, int mode)
 {
     System &S = h->S;
+    Report r{};
     for (int attempt = 0; attempt < 2; ++attempt) {
-        HIP_TRY(hipMemsetAsync(S.flags.p, 0, sizeof(int) * 4, S.stream));
+        nb_clear_flags(S);
         if (mode == SITE_ENERGY) tersoff_energy(h);
         else tersoff_forces(h, false, 0.0);
-        int f[4];
-        nb_read_flags(S, f);
-        if (f[1] == 0) break;
-        int v = ts_variant_for_capacity(f[1]);
+        sys_post_report(S, true, false);
+        HIP_TRY(hipStreamSynchronize(S.stream));
+        r = sys_read_report(S);
+        if (r.f[1] == 0) break;
+        int v = ts_variant_for_capacity(r.f[1]);
         PYSIC_REQUIRE(v >= 0, PYSIC_ECAP,
-                      "more short-range neighbors (" + std::to_string(f[1]) + ") than any kernel holds");
+                      "more short-range neighbors (" + std::to_string(r.f[1]) + ") than any kernel holds");
         h->variant = v;
     }
+    return r;
 }
 
 // Forces of every term except Ewald into S.frc; virials into totals[1..6]
@@ -928,12 +874,20 @@ void batch_evaluate(pysic_ctx *h, bool use_graph, bool rebuild)
 
 // Host arrays that become device state are checked before anything changes:
 // a NaN position would bin as a valid one and drop out of every cutoff test.
-void require_finite(const double *x, size_t count, const std::string &what)
+void require_finite(const double *x, size_t count, const char *what)
 {
     if (!x) return;
-    for (size_t k = 0; k < count; ++k)
+    // 0 x is NaN exactly when x is not finite: four running sums without a
+    // branch, and the entry is looked for only when there is one
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    size_t k = 0;
+    for (; k + 4 <= count; k += 4)
+        for (int c = 0; c < 4; ++c) s[c] += 0.0 * x[k + c];
+    for (; k < count; ++k) s[0] += 0.0 * x[k];
+    if (s[0] + s[1] + s[2] + s[3] == 0.0) return;
+    for (k = 0; k < count; ++k)
         PYSIC_REQUIRE(std::isfinite(x[k]), PYSIC_EINVAL,
-                      "non-finite " + what + " (entry " + std::to_string(k) + ")");
+                      std::string("non-finite ") + what + " (entry " + std::to_string(k) + ")");
 }
 
 // Three cell vectors (rows of v) must be finite and span a volume: the bin
@@ -987,6 +941,7 @@ int pysic_create(pysic_ctx **out, int device)
         PYSIC_REQUIRE(device >= 0 && device < count, PYSIC_EINVAL, "no such HIP device");
         HIP_TRY(hipSetDevice(device));
         scratch_setup(device);
+        h->S.device = device;
         HIP_TRY(hipStreamCreate(&h->S.stream));
         h->S.flags.ensure(4);
         HIP_TRY(hipMemset(h->S.flags.p, 0, sizeof(int) * 4));
@@ -1048,7 +1003,7 @@ int pysic_create_atoms(pysic_ctx *h, int n, const double *masses, const double *
     S.pos.ensure(n); S.mom.ensure(n); S.frc.ensure(n); S.q.ensure(n); S.cut.ensure(n); S.id.ensure(n);
     k_iota<<<div_up(n, 256), 256, 0, S.stream>>>(n, S.id.p);
     k_zero4<<<div_up(n, 256), 256, 0, S.stream>>>(n, S.frc.p);
-    upload_state(h, positions, momenta, false);
+    upload_atoms(h, positions, momenta);
     std::vector<double> q(n, 0.0);
     if (charges) q.assign(charges, charges + n);
     HIP_TRY(hipMemcpyAsync(S.q.p, q.data(), sizeof(double) * n, hipMemcpyHostToDevice, S.stream));
@@ -1084,7 +1039,8 @@ int pysic_update_atom_coordinates(pysic_ctx *h, int n, const double *positions, 
                   "update_atom_coordinates: atom count does not match");
     require_finite(positions, 3 * (size_t)n, "position");
     require_finite(momenta, 3 * (size_t)n, "momentum");
-    upload_state(h, positions, momenta, true);
+    sys_upload3(h->S, positions, h->S.pos.p);
+    if (momenta) sys_upload3(h->S, momenta, h->S.mom.p);   // without them: kept
     h->forces_valid = false;
     API_END(h)
 }
@@ -1095,7 +1051,7 @@ int pysic_update_atom_charges(pysic_ctx *h, int n, const double *charges)
     PYSIC_REQUIRE(h->atoms_ready && n == h->S.n && charges, PYSIC_EINVAL,
                   "update_atom_charges: atom count does not match");
     require_finite(charges, (size_t)n, "charge");
-    upload_scalar(h->S, charges, h->S.q);
+    sys_upload1(h->S, charges, h->S.q.p);
     h->forces_valid = false;
     API_END(h)
 }
@@ -1187,7 +1143,7 @@ int pysic_generate_neighbor_lists(pysic_ctx *h, int n, const double *cutoffs)
     h->lists_valid = false;
     h->forces_valid = false;
     h->min_cut = lo;
-    upload_scalar(h->S, cutoffs, h->S.cut);
+    sys_upload1(h->S, cutoffs, h->S.cut.p);
     nb_configure_grid(h->S, mc);
     build_lists(h);
     h->forces_valid = false;
@@ -1244,19 +1200,15 @@ int pysic_calculate_energy(pysic_ctx *h, double *energy)
     System &S = h->S;
     double e = 0.0;
     if (S.model.has_pairs) {
-        tersoff_checked(h, SITE_ENERGY);
-        double t[8];
-        HIP_TRY(hipMemcpyAsync(t, S.totals.p, sizeof(double) * 7, hipMemcpyDeviceToHost, S.stream));
-        HIP_TRY(hipStreamSynchronize(S.stream));
-        check_flags(h, false);
-        e += t[0];
+        const Report r = tersoff_checked(h, SITE_ENERGY);
+        check_flags(r.f);
+        e += r.t[0];
     }
     if (has_gen(S)) {
         pr_eval(S, PAIR_ENERGY, false);
-        double t = 0.0;
-        HIP_TRY(hipMemcpyAsync(&t, S.gtotals.p, sizeof(double), hipMemcpyDeviceToHost, S.stream));
+        sys_post_report(S, false, true);
         HIP_TRY(hipStreamSynchronize(S.stream));
-        e += t;
+        e += sys_read_report(S).g[0];
     }
     if (S.model.has_self || h->ewald.on) e += ewald_eem_energy(S, h->ewald, h->ew);
     *energy = e;
@@ -1377,21 +1329,44 @@ int pysic_calculate_forces(pysic_ctx *h, int n, double *forces, double *stress)
     require_ready(h);
     System &S = h->S;
     PYSIC_REQUIRE(n == S.n && forces && stress, PYSIC_EINVAL, "calculate_forces: bad arguments");
-    double t[8] = {0, 0, 0, 0, 0, 0, 0, 0}, g[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    Report r{};
+    if (S.model.has_pairs && !has_gen(S) && !h->ewald.on) {
+        // the usual case waits once: flags, virial and forces leave together,
+        // and all are formed again if the short lists have to grow
+        int v = -1;
+        for (int attempt = 0; attempt < 2; ++attempt) {
+            nb_clear_flags(S);
+            tersoff_forces(h, false, 0.0);
+            sys_post_report(S, true, false);
+            sys_download3(S, S.frc.p, forces, [&] {
+                r = sys_read_report(S);
+                v = r.f[1] ? ts_variant_for_capacity(r.f[1]) : -1;
+                PYSIC_REQUIRE(r.f[1] == 0 || v >= 0, PYSIC_ECAP,
+                              "more short-range neighbors (" + std::to_string(r.f[1]) +
+                                  ") than any kernel holds");
+                if (v >= 0 && attempt == 0) return false;
+                check_flags(r.f);
+                return true;
+            });
+            if (v < 0) break;
+            h->variant = v;
+        }
+        for (int q = 0; q < 6; ++q) stress[q] = r.t[1 + q];
+        h->forces_valid = true;
+        return PYSIC_OK;
+    }
     local_forces(h);
-    if (S.model.has_pairs)
-        HIP_TRY(hipMemcpyAsync(t, S.totals.p, sizeof(double) * 7, hipMemcpyDeviceToHost, S.stream));
-    if (has_gen(S))
-        HIP_TRY(hipMemcpyAsync(g, S.gtotals.p, sizeof(double) * 7, hipMemcpyDeviceToHost, S.stream));
+    sys_post_report(S, S.model.has_pairs, has_gen(S));
     HIP_TRY(hipStreamSynchronize(S.stream));
-    if (S.model.has_pairs) check_flags(h, false);
-    for (int q = 0; q < 6; ++q) stress[q] = t[1 + q] + g[1 + q];
+    r = sys_read_report(S);
+    if (S.model.has_pairs) check_flags(r.f);
+    for (int q = 0; q < 6; ++q) stress[q] = r.t[1 + q] + r.g[1 + q];
     if (h->ewald.on) {
         double st[6];
         ewald_add_forces(S, h->ewald, h->ew, st);  // adds into S.frc
         for (int q = 0; q < 6; ++q) stress[q] += st[q];
     }
-    download_vec3(S, S.frc.p, forces);
+    sys_download3(S, S.frc.p, forces);
     h->forces_valid = true;
     API_END(h)
 }
@@ -1402,7 +1377,7 @@ int pysic_calculate_electronegativities(pysic_ctx *h, int n, double *enegs)
     require_ready(h);
     PYSIC_REQUIRE(n == h->S.n && enegs, PYSIC_EINVAL, "calculate_electronegativities: bad arguments");
     DBuf<double> &chi = ewald_eem_chi(h->S, h->ewald, h->ew);
-    download_scalar(h->S, chi.p, enegs);
+    sys_download1(h->S, chi.p, enegs);
     API_END(h)
 }
 
@@ -1417,13 +1392,13 @@ int pysic_relax_charges(pysic_ctx *h, int n, double *charges, double *rates, int
                   "relax_charges: bad arguments");
     require_finite(charges, (size_t)n, "charge");
     require_finite(rates, (size_t)n, "charge rate");
-    upload_scalar(S, charges, S.q);
+    sys_upload1(S, charges, S.q.p);
     h->rates.ensure(n);
-    upload_scalar(S, rates, h->rates);
+    sys_upload1(S, rates, h->rates.p);
     ewald_relax(S, h->ewald, h->ew, h->rates.p, n_steps, timestep, inertia, friction, tolerance,
                 steps, error);
-    download_scalar(S, S.q.p, charges);
-    download_scalar(S, h->rates.p, rates);
+    sys_download1(S, S.q.p, charges);
+    sys_download1(S, h->rates.p, rates);
     h->forces_valid = false;
     API_END(h)
 }
@@ -1477,7 +1452,7 @@ int pysic_md_run(pysic_ctx *h, int nsteps, double dt, int rebuild, double *energ
     PYSIC_REQUIRE(f[0] <= S.cap, PYSIC_ECAP,
                   "neighbor list overflow during MD (" + std::to_string(f[0]) +
                       "); raise the capacity and rerun");
-    check_flags(h, false);
+    check_flags(f);
     h->forces_valid = true;
     API_END(h)
 }
@@ -1486,8 +1461,8 @@ int pysic_get_state(pysic_ctx *h, int n, double *positions, double *momenta)
 {
     API_BEGIN(h)
     PYSIC_REQUIRE(h->atoms_ready && n == h->S.n, PYSIC_EINVAL, "get_state: bad arguments");
-    if (positions) download_vec3(h->S, h->S.pos.p, positions);
-    if (momenta) download_vec3(h->S, h->S.mom.p, momenta);
+    if (positions) sys_download3(h->S, h->S.pos.p, positions);
+    if (momenta) sys_download3(h->S, h->S.mom.p, momenta);
     API_END(h)
 }
 
@@ -1657,15 +1632,13 @@ int pysic_get_cell_results(pysic_ctx *h, int ncells, double *energies, double *v
     require_range_flag(f[2]);
     require_force_flags(f[3]);
     std::vector<double> ev((size_t)8 * ncells);
-    HIP_TRY(hipMemcpyAsync(ev.data(), S.cell_ev.p, sizeof(double) * ev.size(),
-                           hipMemcpyDeviceToHost, S.stream));
-    HIP_TRY(hipStreamSynchronize(S.stream));
+    sys_download_plain(S, 8 * ncells, S.cell_ev.p, ev.data());
     for (int c = 0; c < ncells; ++c) {
         if (energies) energies[c] = ev[8 * c];
         if (virials)
             for (int q = 0; q < 6; ++q) virials[6 * c + q] = ev[8 * c + 1 + q];
     }
-    if (forces) download_vec3(S, S.frc.p, forces);
+    if (forces) sys_download3(S, S.frc.p, forces);
     API_END(h)
 }
 
@@ -1928,9 +1901,9 @@ int pysic_mlp_corrector_features(pysic_mlp *m, pysic_ctx *h, int n, const double
         throw;
     }
     System &S = h->S;
-    upload_scalar(S, charges, S.q);
+    sys_upload1(S, charges, S.q.p);
     M.cprev.ensure(n);
-    upload_scalar(S, previous, M.cprev);
+    sys_upload1(S, previous, M.cprev.p);
     h->forces_valid = false;
     DBuf<double> &chi = ewald_eem_chi(S, h->ewald, h->ew);
     M.cfeat.ensure((size_t)n * CORR_NC);
@@ -1944,7 +1917,7 @@ int pysic_mlp_corrector_features(pysic_mlp *m, pysic_ctx *h, int n, const double
     for (int s = 0; s < n; ++s)
         std::memcpy(features + (size_t)id[s] * CORR_NC, f.data() + (size_t)s * CORR_NC,
                     sizeof(double) * CORR_NC);
-    if (enegs) download_scalar(S, chi.p, enegs);
+    if (enegs) sys_download1(S, chi.p, enegs);
     MLP_END(m)
 }
 
@@ -1975,7 +1948,7 @@ int pysic_mlp_warm_start(pysic_mlp *m, pysic_ctx *h, int n, int n_stages, double
         mlp_corrector_stage(S, M, M.ccoef.p + (size_t)k * CORR_NC, chi.p, prev, next, S.stream);
         std::swap(prev, next);
     }
-    download_scalar(S, S.q.p, charges);
+    sys_download1(S, S.q.p, charges);
     MLP_END(m)
 }
 

@@ -36,6 +36,8 @@ struct EwaldState {
     DBuf<double4> kvec;     // kx, ky, kz, coefficient c_k
     DBuf<double2> sk;       // sum q s cos(k.r), sum q s sin(k.r)
     DBuf<double> scaler;    // current (sorted) order
+    int ones = 0;           // scaler holds this many ones (0: something else)
+    DBuf<double> scaler0;   // the caller's scalers, original order
     DBuf<double> chi;       // electronegativities (sorted order)
     DBuf<double> part;      // block partials
     DBuf<double> red;       // reduced scalars
@@ -91,7 +93,8 @@ double ewald_eem_energy(System &S, const EwaldParams &P, EwaldState &E);
 double ewald_standalone_energy(System &S, const EwaldParams &P, EwaldState &E);
 // Adds Ewald forces into S.frc; stress[6] receives the Ewald part.
 void ewald_add_forces(System &S, const EwaldParams &P, EwaldState &E, double *stress);
-// Electronegativities (charge_self + Ewald) into E.chi, sorted order.
+// Electronegativities (charge_self + Ewald) into E.chi, sorted order, queued
+// on the stream.
 DBuf<double> &ewald_eem_chi(System &S, const EwaldParams &P, EwaldState &E);
 // Damped charge dynamics on device; S.q and rates (sorted order) updated.
 void ewald_relax(System &S, const EwaldParams &P, EwaldState &E, double *rates, int n_steps,

@@ -27,6 +27,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 namespace {
 
@@ -840,12 +841,29 @@ Consts consts_of(const EwaldParams &P, double volume)
     return c;
 }
 
+__global__ void k_ones(int n, double *__restrict__ a)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) a[i] = 1.0;
+}
+
+// unit scalers: written when the array is new, larger or held others
+void unit_scaler(System &S, EwaldState &E)
+{
+    if (E.ones >= S.n) return;
+    E.scaler.ensure(S.n);
+    k_ones<<<div_up(S.n, EB), EB, 0, S.stream>>>(S.n, E.scaler.p);
+    HIP_TRY(hipGetLastError());
+    E.ones = S.n;
+}
+
 void prepare(System &S, const EwaldParams &P, EwaldState &E)
 {
     const int n = S.n;
     const double *v = S.geom.v;
     double cr[3] = {v[1] * v[5] - v[2] * v[4], v[2] * v[3] - v[0] * v[5], v[0] * v[4] - v[1] * v[3]};
     E.volume = std::fabs(cr[0] * v[6] + cr[1] * v[7] + cr[2] * v[8]);
+    if (E.scaler.cap < (size_t)n) E.ones = 0;
     E.scaler.ensure(n);
     E.chi.ensure(n);
     E.red.ensure(16);
@@ -907,6 +925,14 @@ void prepare(System &S, const EwaldParams &P, EwaldState &E)
             HIP_TRY(hipMemcpyAsync(E.pflags.p, flags.data(), sizeof(int) * flags.size(),
                                    hipMemcpyHostToDevice, S.stream));
         }
+        if (P.has_scaler) {
+            std::vector<double> sc = P.scaler;
+            sc.resize(n, 1.0);
+            E.scaler0.ensure(n);
+            HIP_TRY(hipMemcpyAsync(E.scaler0.p, sc.data(), sizeof(double) * n,
+                                   hipMemcpyHostToDevice, S.stream));
+            HIP_TRY(hipStreamSynchronize(S.stream));   // before the host vector goes
+        }
         E.nk = (int)kv.size();
         E.kvec.ensure(kv.size());
         E.sk.ensure(kv.size());
@@ -917,21 +943,13 @@ void prepare(System &S, const EwaldParams &P, EwaldState &E)
         E.dirty = false;
     }
     // scaler in the current atom order
-    S.host_stage.ensure(n);
-    std::vector<double> sc = P.scaler;
-    sc.resize(n, 1.0);
-    HIP_TRY(hipMemcpyAsync(S.host_stage.p, sc.data(), sizeof(double) * n, hipMemcpyHostToDevice, S.stream));
-    k_gather_scaler<<<div_up(n, 256), 256, 0, S.stream>>>(n, S.id.p, S.host_stage.p, E.scaler.p);
-    HIP_TRY(hipStreamSynchronize(S.stream));
-}
-
-void ensure_scaler_identity(System &S, EwaldState &E)
-{
-    // used when Ewald is off: chi needs a scaler array anyway
-    std::vector<double> one(S.n, 1.0);
-    E.scaler.ensure(S.n);
-    HIP_TRY(hipMemcpyAsync(E.scaler.p, one.data(), sizeof(double) * S.n, hipMemcpyHostToDevice, S.stream));
-    HIP_TRY(hipStreamSynchronize(S.stream));
+    if (P.has_scaler) {
+        k_gather_scaler<<<div_up(n, 256), 256, 0, S.stream>>>(n, S.id.p, E.scaler0.p, E.scaler.p);
+        HIP_TRY(hipGetLastError());
+        E.ones = 0;
+    } else {
+        unit_scaler(S, E);
+    }
 }
 
 Recip recip_of(const EwaldState &E)
@@ -982,12 +1000,20 @@ void structure_factors(System &S, EwaldState &E, bool placed = false)
     S.timer.end("ewald_sk", S.stream, ev);
 }
 
+// Where the kernels leave what the host wants to see (sys_mail): read after
+// one wait for the stream.
+enum { M_REAL = MAIL_FREE, M_CHARGE = M_REAL + 8, M_DIPOLE = M_CHARGE + 2, M_HASH = M_DIPOLE + 3,
+       M_RECIP, M_STRESS, M_ERROR = M_STRESS + 6, M_END };
+static_assert(M_END <= MAIL_WORDS, "mail words");
+
 // the virial block partials of a per-atom pass, summed
 void sum_stress(System &S, EwaldState &E, int blocks, double *stress6)
 {
-    k_sum_partials<<<1, EB, 0, S.stream>>>(blocks, 8, 6, E.part.p, E.red.p);
-    HIP_TRY(hipMemcpyAsync(stress6, E.red.p, sizeof(double) * 6, hipMemcpyDeviceToHost, S.stream));
+    double *mail = sys_mail(S) + M_STRESS;
+    k_sum_partials<<<1, EB, 0, S.stream>>>(blocks, 8, 6, E.part.p, mail);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(S.stream));
+    for (int c = 0; c < 6; ++c) stress6[c] = mail[c];
 }
 
 // mode 2: add forces + return stress; mode 3: add into chi.  Needs the
@@ -1037,46 +1063,44 @@ void recip_atoms(System &S, EwaldState &E, int mode, double *stress6)
     if (mode == 2) sum_stress(S, E, ftiles, stress6);
 }
 
-unsigned long long state_hash(System &S, EwaldState &E)
+// the state's fingerprint, into the mail
+void post_hash(System &S, EwaldState &E)
 {
     const int nb = div_up(S.n, EB);
-    E.hpart.ensure(nb + 1);
+    E.hpart.ensure(nb);
     k_state_hash<<<nb, EB, 0, S.stream>>>(S.n, S.pos.p, S.q.p, E.scaler.p, E.hpart.p);
-    k_hash_sum<<<1, EB, 0, S.stream>>>(nb, E.hpart.p, E.hpart.p + nb);
+    k_hash_sum<<<1, EB, 0, S.stream>>>(nb, E.hpart.p, (unsigned long long *)(sys_mail(S) + M_HASH));
     HIP_TRY(hipGetLastError());
-    unsigned long long h;
-    HIP_TRY(hipMemcpyAsync(&h, E.hpart.p + nb, sizeof(h), hipMemcpyDeviceToHost, S.stream));
-    HIP_TRY(hipStreamSynchronize(S.stream));
-    return h;
 }
 
-// S(k) and the phase table of the current state.  An energy call followed by
-// a forces call on the same configuration (the usual calculator sequence)
-// computes them once: they are kept while the fingerprint of positions,
-// charges and scalers matches and neither the cell nor the k-vectors changed.
+// S(k) and the phase table of the current state, whose fingerprint has been
+// posted and waited for.  An energy call followed by a forces call on the
+// same configuration (the usual calculator sequence) computes them once:
+// they are kept while the fingerprint of positions, charges and scalers
+// matches and neither the cell nor the k-vectors changed.
 void current_structure_factors(System &S, EwaldState &E)
 {
-    const unsigned long long h = state_hash(S, E);
+    unsigned long long h;
+    std::memcpy(&h, sys_mail(S) + M_HASH, sizeof(h));
     if (E.sk_valid && E.sk_hash == h) return;
     structure_factors(S, E);
     E.sk_hash = h;
     E.sk_valid = true;
 }
 
-// q sums: out[0] = sum q s, out[1] = sum (q s)^2
-void charge_sums(System &S, EwaldState &E, double *out)
+// q sums, into the mail: sum q s, sum (q s)^2
+void post_charge_sums(System &S, EwaldState &E)
 {
     int nb = div_up(S.n, EB);
     E.part.ensure((size_t)nb * 8);
     k_charge_sums<<<nb, EB, 0, S.stream>>>(S.n, S.q.p, E.scaler.p, E.part.p);
-    k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 2, E.part.p, E.red.p);
-    HIP_TRY(hipMemcpyAsync(out, E.red.p, sizeof(double) * 2, hipMemcpyDeviceToHost, S.stream));
-    HIP_TRY(hipStreamSynchronize(S.stream));
+    k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 2, E.part.p, sys_mail(S) + M_CHARGE);
+    HIP_TRY(hipGetLastError());
 }
 
-// real-space + singlet pass; returns the energy (mode 1) or stress (mode 2)
+// real-space + singlet pass; posts the energy (mode 1) and stress (mode 2) sums
 void real_pass(System &S, const EwaldParams &P, EwaldState &E, int mode, double bg_chi,
-               double *out7, const double *bg_dev = nullptr, bool with_self = true)
+               const double *bg_dev = nullptr, bool with_self = true)
 {
     const int n = S.n;
     Consts c = consts_of(P, E.volume);
@@ -1102,10 +1126,9 @@ void real_pass(System &S, const EwaldParams &P, EwaldState &E, int mode, double 
     }
     HIP_TRY(hipGetLastError());
     S.timer.end("ewald_real", S.stream, ev);
-    if (out7) {
-        k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 7, E.part.p, E.red.p);
-        HIP_TRY(hipMemcpyAsync(out7, E.red.p, sizeof(double) * 7, hipMemcpyDeviceToHost, S.stream));
-        HIP_TRY(hipStreamSynchronize(S.stream));
+    if (mode != 3) {
+        k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 7, E.part.p, sys_mail(S) + M_REAL);
+        HIP_TRY(hipGetLastError());
     }
 }
 
@@ -1126,7 +1149,7 @@ void chi_eval(System &S, const EwaldParams &P, EwaldState &E, bool placed = fals
         HIP_TRY(hipGetLastError());
         bg_dev = E.red.p + 12;
     }
-    real_pass(S, P, E, 3, 0.0, nullptr, bg_dev);
+    real_pass(S, P, E, 3, 0.0, bg_dev);
     if (P.on && has_recip(E)) {
         // the relaxation changes the charges every step: no fingerprint
         structure_factors(S, E, placed);
@@ -1143,6 +1166,8 @@ void ewald_release(EwaldState &E)
     E.kvec.release();
     E.sk.release();
     E.scaler.release();
+    E.scaler0.release();
+    E.ones = 0;
     E.chi.release();
     E.part.release();
     E.red.release();
@@ -1168,42 +1193,44 @@ double energy_terms(System &S, const EwaldParams &P, EwaldState &E, bool with_se
                     bool with_dipole)
 {
     prepare(S, P, E);
-    if (!P.on) ensure_scaler_identity(S, E);
-    double r7[7];
-    real_pass(S, P, E, 1, 0.0, r7, nullptr, with_self);
-    double e = r7[0];
-    if (P.on && with_dipole) {
-        // |sum q s r|^2 inv_eps_2v / 3 (Potentials.f90:1563-1565, 1647)
-        Consts c = consts_of(P, E.volume);
-        int nb = div_up(S.n, EB);
-        E.part.ensure((size_t)nb * 8);
-        k_dipole_sums<<<nb, EB, 0, S.stream>>>(S.n, S.pos.p, S.q.p, E.scaler.p, E.part.p);
-        k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 3, E.part.p, E.red.p);
-        double d[3];
-        HIP_TRY(hipMemcpyAsync(d, E.red.p, sizeof(double) * 3, hipMemcpyDeviceToHost, S.stream));
-        HIP_TRY(hipStreamSynchronize(S.stream));
-        e += (d[0] * d[0] + d[1] * d[1] + d[2] * d[2]) * c.inv_eps_2v / 3.0;
+    if (!P.on) unit_scaler(S, E);
+    real_pass(S, P, E, 1, 0.0, nullptr, with_self);
+    if (P.on) {
+        post_charge_sums(S, E);
+        if (with_dipole) {
+            int nb = div_up(S.n, EB);
+            k_dipole_sums<<<nb, EB, 0, S.stream>>>(S.n, S.pos.p, S.q.p, E.scaler.p, E.part.p);
+            k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 3, E.part.p, sys_mail(S) + M_DIPOLE);
+        }
+        if (has_recip(E)) post_hash(S, E);
     }
+    HIP_TRY(hipStreamSynchronize(S.stream));
+    const double *mail = sys_mail(S);
+    double e = mail[M_REAL];
     if (P.on) {
         Consts c = consts_of(P, E.volume);
-        double qs[2];
-        charge_sums(S, E, qs);
+        if (with_dipole) {
+            // |sum q s r|^2 inv_eps_2v / 3 (Potentials.f90:1563-1565, 1647)
+            const double *d = mail + M_DIPOLE;
+            e += (d[0] * d[0] + d[1] * d[1] + d[2] * d[2]) * c.inv_eps_2v / 3.0;
+        }
+        const double *qs = mail + M_CHARGE;
         e += -qs[1] * c.inv_eps_4pi * c.inv_sig_sqrt2pi;                         // self
         e += -qs[0] * qs[0] * 0.5 * c.inv_eps_2v * P.sigma * P.sigma;            // background
         if (has_recip(E)) {
             current_structure_factors(S, E);
+            double *out = sys_mail(S) + M_RECIP;
             if (E.mesh_on) {
-                k_sum_partials<<<1, EB, 0, S.stream>>>(E.mesh.nepart, 1, 1, E.mesh.epart.p, E.red.p);
+                k_sum_partials<<<1, EB, 0, S.stream>>>(E.mesh.nepart, 1, 1, E.mesh.epart.p, out);
             } else {
                 int nb = div_up(E.nk, EB);
                 E.part.ensure((size_t)nb);
                 k_recip_energy<<<nb, EB, 0, S.stream>>>(E.nk, E.kvec.p, E.sk.p, E.part.p);
-                k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 1, 1, E.part.p, E.red.p);
+                k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 1, 1, E.part.p, out);
             }
-            double er;
-            HIP_TRY(hipMemcpyAsync(&er, E.red.p, sizeof(double), hipMemcpyDeviceToHost, S.stream));
+            HIP_TRY(hipGetLastError());
             HIP_TRY(hipStreamSynchronize(S.stream));
-            e += er;
+            e += mail[M_RECIP];
         }
     }
     return e;
@@ -1224,10 +1251,12 @@ double ewald_standalone_energy(System &S, const EwaldParams &P, EwaldState &E)
 void ewald_add_forces(System &S, const EwaldParams &P, EwaldState &E, double *stress)
 {
     prepare(S, P, E);
-    double r7[7];
-    real_pass(S, P, E, 2, 0.0, r7);
-    for (int c = 0; c < 6; ++c) stress[c] = r7[1 + c];
-    if (P.on && has_recip(E)) {
+    real_pass(S, P, E, 2, 0.0);
+    const bool recip = P.on && has_recip(E);
+    if (recip) post_hash(S, E);
+    HIP_TRY(hipStreamSynchronize(S.stream));
+    for (int c = 0; c < 6; ++c) stress[c] = sys_mail(S)[M_REAL + 1 + c];
+    if (recip) {
         current_structure_factors(S, E);
         double st[6];
         recip_atoms(S, E, 2, st);
@@ -1238,9 +1267,8 @@ void ewald_add_forces(System &S, const EwaldParams &P, EwaldState &E, double *st
 DBuf<double> &ewald_eem_chi(System &S, const EwaldParams &P, EwaldState &E)
 {
     prepare(S, P, E);
-    if (!P.on) ensure_scaler_identity(S, E);
+    if (!P.on) unit_scaler(S, E);
     chi_eval(S, P, E);
-    HIP_TRY(hipStreamSynchronize(S.stream));
     return E.chi;
 }
 
@@ -1250,7 +1278,7 @@ void ewald_relax(System &S, const EwaldParams &P, EwaldState &E, double *rates, 
 {
     const int n = S.n;
     prepare(S, P, E);
-    if (!P.on) ensure_scaler_identity(S, E);
+    if (!P.on) unit_scaler(S, E);
     DBuf<double> dchi, mx;
     dchi.ensure(n);
     int nb = div_up(n, EB);
@@ -1264,11 +1292,11 @@ void ewald_relax(System &S, const EwaldParams &P, EwaldState &E, double *rates, 
         k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 1, E.part.p, E.red.p);
         k_relax_finish<<<nb, EB, 0, S.stream>>>(n, E.chi.p, E.red.p, dchi.p, rates, update, future,
                                                 0.5 * inv_mq * dt, mx.p);
-        k_max_partials<<<1, EB, 0, S.stream>>>(nb, mx.p, E.red.p + 8);
-        double err;
-        HIP_TRY(hipMemcpyAsync(&err, E.red.p + 8, sizeof(double), hipMemcpyDeviceToHost, S.stream));
+        double *mail = sys_mail(S) + M_ERROR;
+        k_max_partials<<<1, EB, 0, S.stream>>>(nb, mx.p, mail);
+        HIP_TRY(hipGetLastError());
         HIP_TRY(hipStreamSynchronize(S.stream));
-        return err;
+        return *mail;
     };
     double err = dchi_of_q(0);
     int step = 0;

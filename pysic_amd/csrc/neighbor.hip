@@ -1314,7 +1314,8 @@ void nb_build_lists(System &S)
 
 int nb_read_flags(System &S, int *out4)
 {
-    HIP_TRY(hipMemcpyAsync(out4, S.flags.p, sizeof(int) * 4, hipMemcpyDeviceToHost, S.stream));
+    sys_post_report(S, false, false);
     HIP_TRY(hipStreamSynchronize(S.stream));
+    std::memcpy(out4, sys_read_report(S).f, sizeof(int) * 4);
     return 0;
 }

@@ -5,6 +5,7 @@
 
 #include "common.h"
 
+#include <functional>
 #include <vector>
 
 template <typename T>
@@ -45,8 +46,26 @@ struct KernelTimer {
     void reset();
 };
 
+// A system's end of the transfers (transfer.hip): its block of pinned memory
+// (mail words and two small slots) and the events of up to PAIRS copying
+// threads with two slots each.
+struct HostLink {
+    static constexpr int PAIRS = 4;
+    char *block = nullptr;
+    hipEvent_t done[2 * PAIRS] = {};
+    bool busy[2] = {};           // an upload's kernel may still read the small slot
+    int turn = 0;                // the small slot used last
+    void release();
+};
+// mail: 0..6 totals, 7..13 gtotals, 14..15 the four flags (k_report); from
+// MAIL_FREE on whatever the caller's kernels write
+constexpr int MAIL_WORDS = 64, MAIL_FREE = 16;
+
 struct System {
     hipStream_t stream = nullptr;
+    int device = 0;
+    HostLink link;
+    DBuf<int> inv;              // slot of each original index (transfers)
     int n = 0;
     CellGeom geom{};
 
@@ -90,8 +109,6 @@ struct System {
     int site_grid = 0;          // > 0: persistent site launch with this many blocks
     DBuf<double> totals;        // reduced energy + virial (7 doubles)
 
-    DBuf<double> host_stage;    // scratch for original-order transfers
-    DBuf<double4> out4;
 
     Model model{};
     DBuf<Model> dmodel;
@@ -202,6 +219,26 @@ int bend_blocks(const System &S);
 void bop_eval(System &S, int mode, int blk0, double half_dt, int kick);
 int bop_blocks(const System &S, int mode);
 void bop_chi(System &S, double *chi);
+
+// transfer.hip: per-atom arrays in the caller's order.  Downloads wait for the
+// stream and return with the host array written; uploads return with the host
+// array read and the rest queued on the stream (double4: x, y, z only).
+// `ready` (if given) is asked between the wait and the host array's writing.
+void sys_download3(System &S, const double4 *src, double *host,
+                   const std::function<bool()> &ready = nullptr);
+void sys_download1(System &S, const double *src, double *host);
+void sys_download_plain(System &S, int count, const double *src, double *host);  // device order
+void sys_upload3(System &S, const double *host, double4 *dst);
+void sys_upload1(System &S, const double *host, double *dst);
+// the reduced totals and flags, queued into the mail words; read them after
+// the stream has been waited for
+struct Report {
+    double t[7], g[7];
+    int f[4];
+};
+double *sys_mail(System &S);
+void sys_post_report(System &S, bool tersoff, bool general);
+Report sys_read_report(System &S);
 
 // md.hip
 void md_drift(System &S, double dt, double half_dt);  // p += dt/2 F ; r += dt p/m (no rebuild)
