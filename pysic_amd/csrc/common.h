@@ -209,6 +209,18 @@ __device__ __forceinline__ double recip64(double x)
     return fma(y, e, y);
 }
 
+// 1 / sqrt(x) for a normal x > 0, within an ulp: the hardware estimate and
+// two Newton steps y += y (1 - x y^2) / 2
+__device__ __forceinline__ double rsqrt64(double x)
+{
+    double y = __builtin_amdgcn_rsq(x);
+    double h = 0.5 * y, e = fma(-x * y, y, 1.0);
+    y = fma(h, e, y);
+    h = 0.5 * y;
+    e = fma(-x * y, y, 1.0);
+    return fma(h, e, y);
+}
+
 // sin and cos of (pi/2) x for 0 <= x <= 1.  The angle is moved to
 // w = (pi/2) x - pi/4 in [-pi/4, pi/4], where the Taylor series of sin w
 // (through w^17) and cos w (through w^18) leave a truncation error below
