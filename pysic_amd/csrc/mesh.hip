@@ -89,16 +89,22 @@ __global__ __launch_bounds__(MB) void k_mesh_bin(int n, MeshGeo g, const double4
 }
 
 // Exclusive scan of the tile counts, one block; clears the counts for the
-// next sort and the fill counters for this one.
-__global__ __launch_bounds__(1024) void k_mesh_scan(int nbins, int *__restrict__ count,
-                                                    int *__restrict__ fill,
-                                                    int *__restrict__ start)
+// next sort and the fill counters for this one.  The arrays are padded to
+// whole int4 per thread (scan_room), so a thread's loads are wide and all in
+// flight at once: 27,436 tiles 66 -> 21 us.
+__global__ __launch_bounds__(1024) void k_mesh_scan(int nbins, int per4, int4 *__restrict__ count,
+                                                    int4 *__restrict__ fill,
+                                                    int4 *__restrict__ start,
+                                                    int *__restrict__ last)
 {
     __shared__ int lds[1024];
-    const int t = threadIdx.x, per = (nbins + 1023) / 1024;
-    const int b0 = min(t * per, nbins), b1 = min(b0 + per, nbins);
+    const int t = threadIdx.x;
     int s = 0;
-    for (int b = b0; b < b1; ++b) s += count[b];
+#pragma unroll 8
+    for (int b = t * per4; b < (t + 1) * per4; ++b) {
+        const int4 c = count[b];
+        s += (c.x + c.y) + (c.z + c.w);
+    }
     lds[t] = s;
     __syncthreads();
     for (int d = 1; d < 1024; d <<= 1) {
@@ -108,14 +114,17 @@ __global__ __launch_bounds__(1024) void k_mesh_scan(int nbins, int *__restrict__
         __syncthreads();
     }
     int at = lds[t] - s;
-    for (int b = b0; b < b1; ++b) {
-        const int c = count[b];
-        start[b] = at;
-        count[b] = 0;
-        fill[b] = 0;
-        at += c;
+    const int4 zero = make_int4(0, 0, 0, 0);
+#pragma unroll 8
+    for (int b = t * per4; b < (t + 1) * per4; ++b) {
+        const int4 c = count[b];
+        start[b] = make_int4(at, at + c.x, at + c.x + c.y, at + c.x + c.y + c.z);
+        count[b] = zero;
+        fill[b] = zero;
+        at += (c.x + c.y) + (c.z + c.w);
     }
-    if (t == 1023) start[nbins] = lds[1023];
+    __syncthreads();
+    if (t == 1023) last[nbins] = lds[1023];   // the end of the last tile
 }
 
 __global__ __launch_bounds__(MB) void k_mesh_fill(int n, const int *__restrict__ bin,
@@ -207,20 +216,79 @@ __device__ __forceinline__ void tile_stream(const MeshGeo &g, int tx, int ty, in
     if (s == SLOTS - 1) base[SLOTS] = incl;
 }
 
-// Offset of mesh point p in a window that starts at point g0 (both reduced
-// to the mesh of n points): in the window when below W.
-__device__ __forceinline__ int window_at(int p, int g0, int n)
+// tile origin - window origin on a periodic axis of n points: in 0 .. W - 1
+// when the tile starts inside the window, else negative, and above minus the
+// tile's length exactly when the window starts inside the tile (n >= W + tile,
+// so never both)
+__device__ __forceinline__ int window_rel(int tile0, int g0, int n)
 {
-    const int o = p - g0;
-    return o < 0 ? o + n : o;
+    int o = tile0 - g0;
+    o += o < 0 ? n : 0;
+    return o >= W ? o - n : o;
 }
+
+constexpr int FAR = -100000;   // the rel of an empty place: no window there
+
+// Stream positions c0 .. c0 + 63 of a tile: (rel of each axis, atom), the atom
+// -1 past the end, and which of the 18 bins it came from.
+__device__ __forceinline__ void tile_chunk(const MeshGeo &g, int tx, int ty, int tz, int c0,
+                                           const int *first, const int *base,
+                                           const int4 *__restrict__ at, int4 *s_at, int *s_bin,
+                                           int *slot)
+{
+    const int c = c0 + threadIdx.x;
+    int4 v = make_int4(FAR, FAR, FAR, 0);
+    int bin = -1;
+    if (c < base[SLOTS]) {
+        bin = 0;
+        for (int s = 1; s < SLOTS; ++s) bin = c >= base[s] ? s : bin;
+        const int atom = first[bin] + (c - base[bin]);
+        const int4 o = at[atom];
+        *slot = o.w;
+        v = make_int4(window_rel(tx * TX, o.x, g.n[0]), window_rel(ty * TY, o.y, g.n[1]),
+                      window_rel(tz * TZ, o.z, g.n[2]), atom);
+    }
+    s_at[threadIdx.x] = v;
+    if (s_bin) s_bin[threadIdx.x] = bin;
+}
+
+// A group of 16 atoms in the tile's own coordinates: 16 x, 8 y and 8 z values
+// of each atom's kernel at the tile's points, zero outside its window, so the
+// product loops read them at fixed offsets and compute no index.  Lane L
+// takes entry L % 32 of atoms 2 j + L / 32.  STRIDE doubles a row.
+template <int STRIDE>
+struct Group {
+    double v[8];
+    static __device__ __forceinline__ int axis() { return (threadIdx.x & 31) < 16 ? 0 : (threadIdx.x & 31) < 24 ? 1 : 2; }
+    __device__ __forceinline__ void load(const int4 *s_at, int t, const double *__restrict__ w)
+    {
+        const int e = threadIdx.x & 31, ax = axis(), p = e - (ax == 0 ? 0 : ax == 1 ? 16 : 24);
+        const int *rec = (const int *)(s_at + 16 * t + (threadIdx.x >> 5));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int o = rec[8 * j + ax] + p;
+            const bool in = (unsigned)o < (unsigned)W;
+            const double x = w[(size_t)rec[8 * j + 3] * 48 + 16 * ax + (in ? o : 0)];
+            v[j] = in ? x : 0.0;
+        }
+    }
+    __device__ __forceinline__ void store(double *lds) const
+    {
+        double *row = lds + (threadIdx.x >> 5) * STRIDE + (threadIdx.x & 31);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) row[2 * j * STRIDE] = v[j];
+    }
+};
 
 // Charges to the mesh.  A wave owns a tile of 16 x 8 x 8 points: for atom a
 // the tile gains q_a phi(y) phi(z) (64 rows) times phi(x) (16 columns), so the
 // tile is a (64 x atoms) by (atoms x 16) product: FP64 MFMA 16x16x4, four
-// row blocks of 4 y by 4 z, 4 atoms a step.  Points outside an atom's
-// window carry zeros.  Bound: the matrix pipe; 262,144 ions on 304^3 points
-// need 2.8 times the 16^3 products per ion that no tile could save.
+// row blocks of 4 y by 4 z, 4 atoms a step.  The kernel values of 16 atoms
+// are staged in LDS in the tile's coordinates while the next 16 load.
+// Bound: half the time the matrix pipe (44 steps of 4 products a tile, 126 us
+// in all at its peak), else the wait for the next group's values, which come
+// from L2 or beyond.  262,144 ions, 304^3 points: 302 us with five gathers
+// from global memory a step, 254 staged.
 // Lane L: A row L % 16 (y = L % 4, z = L / 4 % 4) of atom L / 16; B column
 // L % 16 (x) of atom L / 16; D row L / 16 + 4 r in register r.
 __global__ __launch_bounds__(64) void k_mesh_spread(MeshGeo g, const int *__restrict__ start,
@@ -233,55 +301,48 @@ __global__ __launch_bounds__(64) void k_mesh_spread(MeshGeo g, const int *__rest
     __shared__ int first[SLOTS], base[SLOTS + 1];
     __shared__ int4 s_at[64];
     __shared__ double s_q[64];
+    constexpr int STRIDE = 48;   // a step's four rows on alternate halves of the banks
+    __shared__ double s_w[16 * STRIDE];
     const int lane = threadIdx.x, col = lane & 15, kq = lane >> 4;
     const int blk = xcd_block(gridDim.x);
     const int tx = blk % g.nb[0], ty = blk / g.nb[0] % g.nb[1], tz = blk / (g.nb[0] * g.nb[1]);
     tile_stream(g, tx, ty, tz, start, first, base);
     __syncthreads();
     const int total = base[SLOTS];
-    const int px = tx * TX + col, py = ty * TY + (col & 3), pz = tz * TZ + (col >> 2);
+    const double *px = s_w + kq * STRIDE + col, *py = s_w + kq * STRIDE + 16 + (col & 3),
+                 *pz = s_w + kq * STRIDE + 24 + (col >> 2);
     mfma_d4 acc[2][2];
 #pragma unroll
     for (int z = 0; z < 2; ++z)
 #pragma unroll
         for (int y = 0; y < 2; ++y) acc[z][y] = mfma_d4{0.0, 0.0, 0.0, 0.0};
     for (int c0 = 0; c0 < total; c0 += 64) {
-        const int c = c0 + lane;
-        // past the stream: the first atom with no charge
-        int a = first[0], slot = 0;
-        for (int s = 0; s < SLOTS; ++s)
-            if (c >= base[s]) slot = s;
-        const bool there = c < total;
-        if (there) a = first[slot] + (c - base[slot]);
-        else for (int s = 0; s < SLOTS; ++s)
-            if (base[s + 1] > base[s]) a = first[s];
-        const int4 v = at[a];
-        s_at[lane] = make_int4(v.x, v.y, v.z, a);
-        s_q[lane] = there ? q[v.w] * sc[v.w] : 0.0;
+        int slot = -1;
+        tile_chunk(g, tx, ty, tz, c0, first, base, at, s_at, nullptr, &slot);
+        s_q[lane] = slot >= 0 ? q[slot] * sc[slot] : 0.0;
         __syncthreads();
-        const int steps = min(16, (total - c0 + 3) >> 2);
-        for (int t = 0; t < steps; ++t) {
-            const int4 m = s_at[4 * t + kq];
-            const double qa = s_q[4 * t + kq];
-            const double *row = w + (size_t)m.w * 48;
-            const int ox = window_at(px, m.x, g.n[0]);
-            const int oy0 = window_at(py, m.y, g.n[1]);
-            const int oz0 = window_at(pz, m.z, g.n[2]);
-            int oy1 = oy0 + 4, oz1 = oz0 + 4;
-            oy1 -= oy1 >= g.n[1] ? g.n[1] : 0;
-            oz1 -= oz1 >= g.n[2] ? g.n[2] : 0;
-            const double wx = row[min(ox, W - 1)];
-            const double y0 = row[16 + min(oy0, W - 1)], y1 = row[16 + min(oy1, W - 1)];
-            const double z0 = row[32 + min(oz0, W - 1)], z1 = row[32 + min(oz1, W - 1)];
-            const double b = ox < W ? qa * wx : 0.0;
-            const double vy0 = oy0 < W ? y0 : 0.0, vy1 = oy1 < W ? y1 : 0.0;
-            const double vz0 = oz0 < W ? z0 : 0.0, vz1 = oz1 < W ? z1 : 0.0;
-            acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(vy0 * vz0, b, acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(vy1 * vz0, b, acc[0][1], 0, 0, 0);
-            acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(vy0 * vz1, b, acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(vy1 * vz1, b, acc[1][1], 0, 0, 0);
+        const int groups = min(4, (total - c0 + 15) >> 4);
+        Group<STRIDE> v;
+        v.load(s_at, 0, w);
+        for (int t = 0; t < groups; ++t) {
+            if ((lane & 31) < 16) {   // the x values carry the charge
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v.v[j] *= s_q[16 * t + 2 * j + (lane >> 5)];
+            }
+            v.store(s_w);
+            __syncthreads();
+            if (t + 1 < groups) v.load(s_at, t + 1, w);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int o = 4 * k * STRIDE;
+                const double b = px[o], y0 = py[o], y1 = py[o + 4], z0 = pz[o], z1 = pz[o + 4];
+                acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(y0 * z0, b, acc[0][0], 0, 0, 0);
+                acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(y1 * z0, b, acc[0][1], 0, 0, 0);
+                acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(y0 * z1, b, acc[1][0], 0, 0, 0);
+                acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(y1 * z1, b, acc[1][1], 0, 0, 0);
+            }
+            __syncthreads();
         }
-        __syncthreads();
     }
 #pragma unroll
     for (int z = 0; z < 2; ++z)
@@ -291,7 +352,7 @@ __global__ __launch_bounds__(64) void k_mesh_spread(MeshGeo g, const int *__rest
             for (int r = 0; r < 4; ++r) {
                 // row kq + 4 r of the block: y = kq, z = r
                 const size_t Y = ty * TY + 4 * y + kq, Z = tz * TZ + 4 * z + r;
-                mesh[(Z * g.n[1] + Y) * g.n[0] + px] = acc[z][y][r];
+                mesh[(Z * g.n[1] + Y) * g.n[0] + tx * TX + col] = acc[z][y][r];
             }
 }
 
@@ -304,42 +365,84 @@ __global__ __launch_bounds__(64) void k_mesh_spread(MeshGeo g, const int *__rest
 // 16 k by 16 columns of both; lane L: A row L % 16 of point L / 16 (from the
 // table in this order, a coalesced 512 bytes), B column L % 16 of point
 // L / 16.  Bound: the matrix pipe.
+// The table of 4 steps is staged in LDS for the block's four waves, the next
+// 4 steps' table and mesh values loading meanwhile: read by every wave for
+// itself the table alone is 1.2 GB from L2 a pass on 304^3 points.
+// Mesh to k, 304^3 points, K = 74, three axes: 275 -> 245 us; k to mesh 327
+// -> 294 us.
+constexpr int DS = 4;   // steps per staged table
+
+// table values of steps t0 .. t0 + 3 of the wave's tiles: MT double2 a thread
+template <int MT>
+__device__ __forceinline__ void table_load(const double *__restrict__ tab, int m0, int mtiles,
+                                           int steps, int t0, double2 (&v)[MT])
+{
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+        // pair e of the staged block: [sine][tile][step][32 pairs]
+        const int e = j * MB + threadIdx.x;
+        const int p = e & 31, t = t0 + ((e >> 5) & (DS - 1)), m = (e >> 7) % MT, sn = (e >> 7) / MT;
+        const bool on = m0 + m < mtiles && t < steps;
+        const double2 *src = (const double2 *)tab +
+                             (((size_t)sn * mtiles + m0 + (on ? m : 0)) * steps + (on ? t : 0)) * 32 + p;
+        const double2 x = *src;
+        v[j] = on ? x : make_double2(0.0, 0.0);
+    }
+}
+
 template <int MT>
 __global__ __launch_bounds__(MB) void k_dft_forward(int n, int K, int inner, long cols, int steps,
                                                     int mtiles, const double *__restrict__ tab,
                                                     const double *__restrict__ in, long in_size,
                                                     double *__restrict__ out, long out_size)
 {
+    __shared__ double2 s_tab[2][MT * MB];
     const int lane = threadIdx.x & 63, col = lane & 15, kq = lane >> 4;
-    const long c0 = ((long)blockIdx.x * (MB / 64) + (threadIdx.x >> 6)) * 16;
-    if (c0 >= cols) return;   // whole waves; no barrier
-    const long c = c0 + col, cl = c < cols ? c : cols - 1;
+    const long c = ((long)blockIdx.x * (MB / 64) + (threadIdx.x >> 6)) * 16 + col;
+    const long cl = c < cols ? c : cols - 1;   // waves past the columns load the last one
     const int m0 = blockIdx.y * MT;
     const long o = cl / inner, i = cl - o * inner;
     const double *src = in + blockIdx.z * in_size + o * n * inner + i;
-    const double *tc = tab + (size_t)m0 * steps * 64 + lane;
-    const double *tsn = tc + (size_t)mtiles * steps * 64;
     mfma_d4 ac[MT], as[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) ac[m] = as[m] = mfma_d4{0.0, 0.0, 0.0, 0.0};
     const int half = n / 2;
-    auto load = [&](int t, double &x, double &y) {
-        const int p = min(4 * t + kq, half);
-        x = src[(long)p * inner];
-        y = src[(long)(p ? n - p : 0) * inner];
-    };
-    double x, y;
-    load(0, x, y);
-    for (int t = 0; t < steps; ++t) {
-        const double e = x + y, d = x - y;
-        load(t + 1, x, y);
+    double x[DS], y[DS];
+    auto load = [&](int t0) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const bool on = m0 + m < mtiles;
-            const size_t at = ((size_t)(on ? m : 0) * steps + t) * 64;
-            ac[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(tc[at], e, ac[m], 0, 0, 0);
-            as[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(tsn[at], d, as[m], 0, 0, 0);
+        for (int u = 0; u < DS; ++u) {
+            const int p = min(4 * (t0 + u) + kq, half);
+            x[u] = src[(long)p * inner];
+            y[u] = src[(long)(p ? n - p : 0) * inner];
         }
+    };
+    double2 v[MT];
+    table_load<MT>(tab, m0, mtiles, steps, 0, v);
+    load(0);
+    for (int t0 = 0, b = 0; t0 < steps; t0 += DS, b ^= 1) {
+#pragma unroll
+        for (int j = 0; j < MT; ++j) s_tab[b][j * MB + threadIdx.x] = v[j];
+        double e[DS], d[DS];
+#pragma unroll
+        for (int u = 0; u < DS; ++u) {
+            e[u] = x[u] + y[u];
+            d[u] = x[u] - y[u];
+        }
+        __syncthreads();   // also: the other buffer's readers are done
+        if (t0 + DS < steps) {
+            table_load<MT>(tab, m0, mtiles, steps, t0 + DS, v);
+            load(t0 + DS);
+        }
+        const double *tc = (const double *)s_tab[b] + lane;
+#pragma unroll
+        for (int u = 0; u < DS; ++u)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                ac[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(tc[(m * DS + u) * 64], e[u], ac[m],
+                                                             0, 0, 0);
+                as[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(tc[((MT + m) * DS + u) * 64], d[u],
+                                                             as[m], 0, 0, 0);
+            }
     }
     if (c >= cols) return;
     double *oc = out + 2 * blockIdx.z * out_size + o * (K + 1) * inner + i, *os = oc + out_size;
@@ -363,35 +466,52 @@ __global__ __launch_bounds__(MB) void k_dft_inverse(int n, int K, int inner, lon
                                                     const double *__restrict__ in, long in_size,
                                                     double *__restrict__ out, long out_size)
 {
+    __shared__ double2 s_tab[2][MT * MB];
     const int lane = threadIdx.x & 63, col = lane & 15, kq = lane >> 4;
-    const long c0 = ((long)blockIdx.x * (MB / 64) + (threadIdx.x >> 6)) * 16;
-    if (c0 >= cols) return;   // whole waves; no barrier
-    const long c = c0 + col, cl = c < cols ? c : cols - 1;
+    const long c = ((long)blockIdx.x * (MB / 64) + (threadIdx.x >> 6)) * 16 + col;
+    const long cl = c < cols ? c : cols - 1;   // waves past the columns load the last one
     const int m0 = blockIdx.y * MT;
     const long o = cl / inner, i = cl - o * inner;
     const double *src = in + 2 * blockIdx.z * in_size + o * (K + 1) * inner + i;
-    const double *tc = tab + (size_t)m0 * steps * 64 + lane;
-    const double *tsn = tc + (size_t)mtiles * steps * 64;
     mfma_d4 ae[MT], ao[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) ae[m] = ao[m] = mfma_d4{0.0, 0.0, 0.0, 0.0};
-    auto load = [&](int t, double &x, double &y) {
-        const int k = min(4 * t + kq, K);
-        x = src[(long)k * inner];
-        y = src[in_size + (long)k * inner];
-    };
-    double x, y;
-    load(0, x, y);
-    for (int t = 0; t < steps; ++t) {
-        const double a = x, b = y;
-        load(t + 1, x, y);
+    double x[DS], y[DS];
+    auto load = [&](int t0) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const bool on = m0 + m < mtiles;
-            const size_t at = ((size_t)(on ? m : 0) * steps + t) * 64;
-            ae[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(tc[at], a, ae[m], 0, 0, 0);
-            ao[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(tsn[at], b, ao[m], 0, 0, 0);
+        for (int u = 0; u < DS; ++u) {
+            const int k = min(4 * (t0 + u) + kq, K);
+            x[u] = src[(long)k * inner];
+            y[u] = src[in_size + (long)k * inner];
         }
+    };
+    double2 v[MT];
+    table_load<MT>(tab, m0, mtiles, steps, 0, v);
+    load(0);
+    for (int t0 = 0, b = 0; t0 < steps; t0 += DS, b ^= 1) {
+#pragma unroll
+        for (int j = 0; j < MT; ++j) s_tab[b][j * MB + threadIdx.x] = v[j];
+        double e[DS], d[DS];
+#pragma unroll
+        for (int u = 0; u < DS; ++u) {
+            e[u] = x[u];
+            d[u] = y[u];
+        }
+        __syncthreads();   // also: the other buffer's readers are done
+        if (t0 + DS < steps) {
+            table_load<MT>(tab, m0, mtiles, steps, t0 + DS, v);
+            load(t0 + DS);
+        }
+        const double *tc = (const double *)s_tab[b] + lane;
+#pragma unroll
+        for (int u = 0; u < DS; ++u)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                ae[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(tc[(m * DS + u) * 64], e[u], ae[m],
+                                                             0, 0, 0);
+                ao[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(tc[((MT + m) * DS + u) * 64], d[u],
+                                                             ao[m], 0, 0, 0);
+            }
     }
     if (c >= cols) return;
     double *dst = out + blockIdx.z * out_size + o * n * inner + i;
@@ -497,7 +617,13 @@ __global__ __launch_bounds__(MB) void k_mesh_combine(int K1, int K2, int K3,
 // and phi'_z, so one mesh serves all three components (three transforms of
 // i k Phi would cost three inverse transforms).  part[(a * 18 + slot) * NC]
 // takes what this tile gives atom a; every slot is written by one tile.
-// Bound: the matrix pipe, 16 (FORCE: 32) products per 16 atoms and tile.
+// The kernel values of the 16 atoms are staged in LDS as in k_mesh_spread;
+// the sums reuse that space once the values have been read.
+// Bound: 32 products per 16 atoms and tile with FORCE (16 without), 260 us at
+// the matrix pipe's peak for 262,144 ions, and as much again in the FP64
+// contraction, which shares that pipe, and in waiting for values at two waves
+// per SIMD.  Forces of 262,144 ions: 774 us with gathers from global memory,
+// 642 staged.
 template <bool FORCE>
 __global__ __launch_bounds__(64) void k_mesh_field(MeshGeo g, const int *__restrict__ start,
                                                    const int4 *__restrict__ at,
@@ -509,8 +635,11 @@ __global__ __launch_bounds__(64) void k_mesh_field(MeshGeo g, const int *__restr
     constexpr int NC = FORCE ? 3 : 1;
     __shared__ int first[SLOTS], base[SLOTS + 1];
     __shared__ int4 s_at[64];
-    __shared__ int s_slot[64];
-    __shared__ double red[NC * 16 * 17];
+    __shared__ int s_bin[64];
+    constexpr int STRIDE = 36;   // the 16 rows of an A operand spread over the banks
+    constexpr int RED = NC * 16 * 17, VAL = (FORCE ? 2 : 1) * 16 * STRIDE;
+    __shared__ double s_w[RED > VAL ? RED : VAL];   // the sums take the staged values' place
+    double *s_dw = s_w + (FORCE ? 16 * STRIDE : 0), *red = s_w;
     const int lane = threadIdx.x, col = lane & 15, kq = lane >> 4;
     const int blk = xcd_block(gridDim.x);
     const int tx = blk % g.nb[0], ty = blk / g.nb[0] % g.nb[1], tz = blk / (g.nb[0] * g.nb[1]);
@@ -518,7 +647,6 @@ __global__ __launch_bounds__(64) void k_mesh_field(MeshGeo g, const int *__restr
     __syncthreads();
     const int total = base[SLOTS];
     if (total == 0) return;
-    const int py = ty * TY + (col & 3), pz = tz * TZ + (col >> 2);
     // B operands: point x = 4 s + kq of column (y, z) = col of block (bz, by)
     double f[2][2][4];
 #pragma unroll
@@ -527,95 +655,83 @@ __global__ __launch_bounds__(64) void k_mesh_field(MeshGeo g, const int *__restr
         for (int y = 0; y < 2; ++y)
 #pragma unroll
             for (int s = 0; s < 4; ++s)
-                f[z][y][s] = mesh[((size_t)(pz + 4 * z) * g.n[1] + py + 4 * y) * g.n[0] +
-                                  tx * TX + 4 * s + kq];
+                f[z][y][s] = mesh[((size_t)(tz * TZ + (col >> 2) + 4 * z) * g.n[1] + ty * TY +
+                                   (col & 3) + 4 * y) * g.n[0] + tx * TX + 4 * s + kq];
     for (int c0 = 0; c0 < total; c0 += 64) {
-        const int c = c0 + lane;
-        int a = -1, slot = 0;
-        for (int s = 0; s < SLOTS; ++s)
-            if (c >= base[s]) slot = s;
-        if (c < total) a = first[slot] + (c - base[slot]);
-        int4 v = make_int4(0, 0, 0, 0);
-        if (a >= 0) v = at[a];
-        s_at[lane] = make_int4(v.x, v.y, v.z, a);
-        s_slot[lane] = slot;
+        int slot = -1;
+        tile_chunk(g, tx, ty, tz, c0, first, base, at, s_at, s_bin, &slot);
         __syncthreads();
         const int groups = min(4, (total - c0 + 15) >> 4);
+        Group<STRIDE> v, dv;
+        v.load(s_at, 0, w);
+        if (FORCE) dv.load(s_at, 0, dw);
         for (int t = 0; t < groups; ++t) {
-            const int4 m = s_at[16 * t + col];
-            const size_t row = (size_t)max(m.w, 0) * 48;
-            double ax[4], adx[4];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int o = window_at(tx * TX + 4 * s + kq, m.x, g.n[0]);
-                const double x = w[row + min(o, W - 1)];
-                ax[s] = o < W ? x : 0.0;
-                if (FORCE) {
-                    const double dx = dw[row + min(o, W - 1)];
-                    adx[s] = o < W ? dx : 0.0;
-                }
+            v.store(s_w);
+            if (FORCE) dv.store(s_dw);
+            __syncthreads();
+            if (t + 1 < groups) {
+                v.load(s_at, t + 1, w);
+                if (FORCE) dv.load(s_at, t + 1, dw);
             }
             mfma_d4 T[2][2], U[2][2];
 #pragma unroll
             for (int z = 0; z < 2; ++z)
 #pragma unroll
-                for (int y = 0; y < 2; ++y) {
-                    T[z][y] = U[z][y] = mfma_d4{0.0, 0.0, 0.0, 0.0};
-                }
+                for (int y = 0; y < 2; ++y) T[z][y] = U[z][y] = mfma_d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
+            for (int s = 0; s < 4; ++s) {
+                const int o = col * STRIDE + kq + 4 * s;
+                const double ax = s_w[o];
+                const double adx = FORCE ? s_dw[o] : 0.0;
 #pragma unroll
                 for (int z = 0; z < 2; ++z)
 #pragma unroll
                     for (int y = 0; y < 2; ++y) {
-                        T[z][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(ax[s], f[z][y][s], T[z][y],
+                        T[z][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(ax, f[z][y][s], T[z][y],
                                                                        0, 0, 0);
                         if (FORCE)
-                            U[z][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                                adx[s], f[z][y][s], U[z][y], 0, 0, 0);
+                            U[z][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(adx, f[z][y][s],
+                                                                           U[z][y], 0, 0, 0);
                     }
+            }
             // T register r: atom kq + 4 r of the group, column col
+            double out[NC][4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int4 k = s_at[16 * t + kq + 4 * r];
-                const size_t rw = (size_t)max(k.w, 0) * 48;
-                const int oy0 = window_at(py, k.y, g.n[1]), oz0 = window_at(pz, k.z, g.n[2]);
-                int oy1 = oy0 + 4, oz1 = oz0 + 4;
-                oy1 -= oy1 >= g.n[1] ? g.n[1] : 0;
-                oz1 -= oz1 >= g.n[2] ? g.n[2] : 0;
-                const int iy0 = 16 + min(oy0, W - 1), iy1 = 16 + min(oy1, W - 1);
-                const int iz0 = 32 + min(oz0, W - 1), iz1 = 32 + min(oz1, W - 1);
-                const bool by0 = oy0 < W, by1 = oy1 < W, bz0 = oz0 < W, bz1 = oz1 < W;
-                const double ly0 = w[rw + iy0], ly1 = w[rw + iy1];
-                const double lz0 = w[rw + iz0], lz1 = w[rw + iz1];
-                const double y0 = by0 ? ly0 : 0.0, y1 = by1 ? ly1 : 0.0;
-                const double z0 = bz0 ? lz0 : 0.0, z1 = bz1 ? lz1 : 0.0;
+                const int row = (kq + 4 * r) * STRIDE;
+                const int iy0 = row + 16 + (col & 3), iy1 = iy0 + 4;
+                const int iz0 = row + 24 + (col >> 2), iz1 = iz0 + 4;
+                const double y0 = s_w[iy0], y1 = s_w[iy1], z0 = s_w[iz0], z1 = s_w[iz1];
                 const double t0 = fma(T[0][1][r], y1, T[0][0][r] * y0);
                 const double t1 = fma(T[1][1][r], y1, T[1][0][r] * y0);
-                const int at16 = (kq + 4 * r) * 17 + col;
-                if (!FORCE) {
-                    red[at16] = fma(t1, z1, t0 * z0);
+                if constexpr (!FORCE) {
+                    out[0][r] = fma(t1, z1, t0 * z0);
                 } else {
-                    const double my0 = dw[rw + iy0], my1 = dw[rw + iy1];
-                    const double mz0 = dw[rw + iz0], mz1 = dw[rw + iz1];
-                    const double dy0 = by0 ? my0 : 0.0, dy1 = by1 ? my1 : 0.0;
-                    const double dz0 = bz0 ? mz0 : 0.0, dz1 = bz1 ? mz1 : 0.0;
+                    const double dy0 = s_dw[iy0], dy1 = s_dw[iy1];
+                    const double dz0 = s_dw[iz0], dz1 = s_dw[iz1];
                     const double u0 = fma(U[0][1][r], y1, U[0][0][r] * y0);
                     const double u1 = fma(U[1][1][r], y1, U[1][0][r] * y0);
                     const double v0 = fma(T[0][1][r], dy1, T[0][0][r] * dy0);
                     const double v1 = fma(T[1][1][r], dy1, T[1][0][r] * dy0);
-                    red[at16] = fma(u1, z1, u0 * z0);
-                    red[272 + at16] = fma(v1, z1, v0 * z0);
-                    red[544 + at16] = fma(t1, dz1, t0 * dz0);
+                    out[0][r] = fma(u1, z1, u0 * z0);
+                    out[1][r] = fma(v1, z1, v0 * z0);
+                    out[2][r] = fma(t1, dz1, t0 * dz0);
                 }
             }
+            __syncthreads();   // the staged values have been read: their place is red's now
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    red[c * 272 + (kq + 4 * r) * 17 + col] = out[c][r];
             __syncthreads();
             if (lane < 16 * NC) {
-                const int b = 16 * t + (lane & 15), comp = lane >> 4;
                 double s = 0.0;
+#pragma unroll
                 for (int j = 0; j < 16; ++j) s += red[lane * 17 + j];
-                const int ba = s_at[b].w;
-                if (ba >= 0) part[((size_t)ba * SLOTS + s_slot[b]) * NC + comp] = s;
+                const int b = 16 * t + (lane & 15);
+                if (s_bin[b] >= 0)
+                    part[((size_t)s_at[b].w * SLOTS + s_bin[b]) * NC + (lane >> 4)] = s;
             }
             __syncthreads();
         }
@@ -680,6 +796,9 @@ __global__ void k_mesh_zero(int m, int *__restrict__ a)
 // ---- host side ----------------------------------------------------------------
 
 int round_up(int x, int m) { return (x + m - 1) / m * m; }
+
+// ints that k_mesh_scan reads for nbins counts: whole int4 for 1024 threads
+int scan_room(int nbins) { return round_up(nbins, 4096); }
 
 // Fourier transform of the kernel at frequencies k / n, k = 0 .. K, by
 // Gauss-Legendre quadrature in extended precision (the kernel is analytic
@@ -865,10 +984,11 @@ void mesh_plan(System &S, const EwaldParams &P, MeshState &M, const double *b, d
     M.bufa.ensure(std::max(n0 * n1 * n2, 4 * n0 * (M.K[1] + 1) * (M.K[2] + 1)));
     M.bufb.ensure(2 * n0 * n1 * (M.K[2] + 1));
     M.oct.ensure(8 * oct);
-    M.count.ensure(M.nbins);
-    M.fill.ensure(M.nbins);
-    M.start.ensure(M.nbins + 1);
-    k_mesh_zero<<<div_up(M.nbins, 256), 256, 0, S.stream>>>(M.nbins, M.count.p);
+    const int room = scan_room(M.nbins);
+    M.count.ensure(room);
+    M.fill.ensure(room);
+    M.start.ensure(room + 1);
+    k_mesh_zero<<<div_up(room, 256), 256, 0, S.stream>>>(room, M.count.p);
     k_mesh_coef<<<div_up((int)oct, MB), MB, 0, S.stream>>>(
         M.K[0], M.K[1], M.K[2], make_double4(b[0], b[1], b[2], 0), make_double4(b[3], b[4], b[5], 0),
         make_double4(b[6], b[7], b[8], 0), P.kc * P.kc, inv_eps_2v, 0.5 * P.sigma * P.sigma,
@@ -886,7 +1006,8 @@ void mesh_place(System &S, MeshState &M, const double *f)
     M.w.ensure((size_t)n * 48);
     const MeshGeo g = geo_of(M, f);
     k_mesh_bin<<<div_up(n, MB), MB, 0, S.stream>>>(n, g, S.pos.p, M.bin.p, M.count.p);
-    k_mesh_scan<<<1, 1024, 0, S.stream>>>(M.nbins, M.count.p, M.fill.p, M.start.p);
+    k_mesh_scan<<<1, 1024, 0, S.stream>>>(M.nbins, scan_room(M.nbins) / 4096, (int4 *)M.count.p,
+                                          (int4 *)M.fill.p, (int4 *)M.start.p, M.start.p);
     k_mesh_fill<<<div_up(n, MB), MB, 0, S.stream>>>(n, M.bin.p, M.start.p, M.fill.p, M.claim.p);
     k_mesh_order<<<M.nbins, 64, 0, S.stream>>>(M.start.p, M.claim.p, M.order.p);
     const unsigned blocks = (unsigned)(((long)n * 48 + MB - 1) / MB);
