@@ -246,18 +246,59 @@ __global__ void k_scan_blocks(int nb, int *__restrict__ blk, int *__restrict__ o
     if (threadIdx.x == 0) out[m] = carry;
 }
 
+// The whole scan in one block, for at most SCAN_ONE bins, where the pair above
+// is two launches of little work (2,000 bins: 7.5 -> 4.5 us).  The arrays are
+// padded to whole int4 per thread; the block totals that bin_start adds are
+// zeros here.
+constexpr int SCAN_ONE = 1 << 16;
+__global__ __launch_bounds__(1024) void k_scan_one(int per4, int4 *__restrict__ in,
+                                                   int4 *__restrict__ out,
+                                                   int4 *__restrict__ fill, int nblk,
+                                                   int *__restrict__ blk)
+{
+    __shared__ int wsum[16];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int4 zero = make_int4(0, 0, 0, 0);
+    int s = 0;
+#pragma unroll 4
+    for (int b = t * per4; b < (t + 1) * per4; ++b) {
+        const int4 c = in[b];
+        s += (c.x + c.y) + (c.z + c.w);
+    }
+    int incl = s;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int x = __shfl_up(incl, d);
+        if (lane >= d) incl += x;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    if (t < nblk) blk[t] = 0;
+    __syncthreads();
+    int at = incl - s;
+    for (int w = 0; w < wave; ++w) at += wsum[w];
+#pragma unroll 4
+    for (int b = t * per4; b < (t + 1) * per4; ++b) {
+        const int4 c = in[b];
+        out[b] = make_int4(at, at + c.x, at + c.x + c.y, at + c.x + c.y + c.z);
+        in[b] = zero;
+        fill[b] = zero;
+        at += (c.x + c.y) + (c.z + c.w);
+    }
+}
+
 __device__ __forceinline__ int bin_start(int k, const int *__restrict__ loc,
                                          const int *__restrict__ blk)
 {
     return loc[k] + blk[k / SCAN_BLK];
 }
 
-// zero two bin arrays of length m (a kernel, so that graphs hold no memset)
-__global__ void k_fill_int(int m, int *__restrict__ a, int *__restrict__ b)
+// zero three bin arrays of length m (a kernel, so that graphs hold no memset)
+__global__ void k_fill_int(int m, int *__restrict__ a, int *__restrict__ b, int *__restrict__ c)
 {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t < m) a[t] = 0;
     else if (t < 2 * m) b[t - m] = 0;
+    else if (t < 3 * m) c[t - 2 * m] = 0;
 }
 
 __global__ void k_clear_flags(int *__restrict__ flags)
@@ -268,7 +309,7 @@ __global__ void k_clear_flags(int *__restrict__ flags)
 // New slot of the atom in old slot i.  A bin no atom entered or left keeps
 // its atoms in the same order (sorted by original index), so they move as a
 // block: new start + (i - old start).  The atoms of a dirty bin claim slots
-// with atomics and k_cellsort orders them.  all_dirty: every bin is dirty
+// with atomics and k_permute orders them.  all_dirty: every bin is dirty
 // (the old order is not a previous sort's).
 __global__ void k_scatter(int n, const int *__restrict__ key, const int *__restrict__ loc,
                           const int *__restrict__ blk, const int *__restrict__ prevstart,
@@ -285,40 +326,24 @@ __global__ void k_scatter(int n, const int *__restrict__ key, const int *__restr
     else atomicOr(flags + 2, 2);   // an inconsistent sort: reported, never written
 }
 
-// Within each dirty cell, order atoms by original index: the atomic slot
-// claims above are unordered, this makes the whole permutation
-// deterministic (the same as sorting every cell).  Writes the final cell
-// starts and clears the dirty flags for the next sort.
-__global__ void k_cellsort(int ncell, int n, const int *__restrict__ loc,
-                           const int *__restrict__ blk, int *__restrict__ perm,
-                           const int *__restrict__ id, int *__restrict__ dirty, int all_dirty,
-                           int *__restrict__ start)
-{
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncell) return;
-    int a = bin_start(c, loc, blk), b = c + 1 < ncell ? bin_start(c + 1, loc, blk) : n;
-    start[c] = a;
-    if (c == ncell - 1) start[ncell] = n;
-    if (!(all_dirty || dirty[c])) return;
-    dirty[c] = 0;
-    for (int x = a + 1; x < b; ++x) {
-        int v = perm[x];
-        int kv = id[v];
-        int y = x - 1;
-        while (y >= a && id[perm[y]] > kv) {
-            perm[y + 1] = perm[y];
-            --y;
-        }
-        perm[y + 1] = v;
-    }
-}
-
+// Moves every atom to its new slot.  The slots k_scatter claimed within a
+// dirty bin are unordered: the atom's place among the bin's atoms by original
+// index is counted here (each thread reads its bin's indices; a thread per
+// bin sorting them one after another took 1.2 ms for bins of 70 atoms, 114 us
+// for the 13,500 argon atoms' 15; 4 us for 3, in a launch of its own), which
+// makes the whole permutation deterministic, the same as sorting every bin.
+// Threads below nbins also write the final bin starts and clear the dirty
+// flags of the sort before (this sort's are still being read).
 // Forces are not carried: after the drift they are dead until recomputed.
 // QC: move the charges and cutoffs too.  Without it they stay where they
 // are, which is right only while both buffers of each hold one value for
 // every atom (checked before a run that uses it).
 template <class Geo, bool QC>
-__global__ void k_permute(int n, const int *__restrict__ perm, const double4 *__restrict__ pos,
+__global__ void k_permute(int n, int nbins, const int *__restrict__ loc,
+                          const int *__restrict__ blk, const int *__restrict__ perm,
+                          const int *__restrict__ dirty, int *__restrict__ old_dirty,
+                          int all_dirty, int *__restrict__ start,
+                          const double4 *__restrict__ pos,
                           const double4 *__restrict__ mom, const double *__restrict__ q,
                           const double *__restrict__ cut, const int *__restrict__ id,
                           const int *__restrict__ key, const int *__restrict__ wrap,
@@ -327,14 +352,34 @@ __global__ void k_permute(int n, const int *__restrict__ perm, const double4 *__
                           int *__restrict__ id2, int *__restrict__ key2, int *__restrict__ wrap2,
                           Geo geo, float4 *__restrict__ wpos, int *__restrict__ flags)
 {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const CellGeom &g = geo.of(s);   // slot s stays in the cell of slot perm[s]
-    int o = perm[s];
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < nbins) {
+        start[t] = bin_start(t, loc, blk);
+        if (t == nbins - 1) start[nbins] = n;
+        old_dirty[t] = 0;
+    }
+    if (t >= n) return;
+    int o = perm[t];
     if ((unsigned)o >= (unsigned)n) {
         atomicOr(flags + 2, 2);   // an inconsistent sort (reported): keep the slot
-        o = s;
+        o = t;
     }
+    const int k = key[o], ido = id[o];
+    int s = t;
+    if (all_dirty || dirty[k]) {
+        const int a = bin_start(k, loc, blk), b = k + 1 < nbins ? bin_start(k + 1, loc, blk) : n;
+        int rank = 0;
+        for (int x = a; x < b; ++x) {
+            const int m = perm[x];
+            rank += id[(unsigned)m < (unsigned)n ? m : o] < ido ? 1 : 0;
+        }
+        s = a + rank;
+        if (s >= n) {   // only after an inconsistent sort
+            atomicOr(flags + 2, 2);
+            s = t;
+        }
+    }
+    const CellGeom &g = geo.of(s);   // slot s stays in the cell of the atom's old slot
     double4 p = pos[o];
     int w = wrap[o];
     pos2[s] = p;
@@ -343,8 +388,8 @@ __global__ void k_permute(int n, const int *__restrict__ perm, const double4 *__
         q2[s] = q[o];
         cut2[s] = cut[o];
     }
-    id2[s] = id[o];
-    key2[s] = key[o];
+    id2[s] = ido;
+    key2[s] = k;
     wrap2[s] = w;
     // wrapped position in FP32 for the neighbor prefilter
     double wx = img_x(w), wy = img_y(w), wz = img_z(w);
@@ -368,11 +413,8 @@ __global__ void k_permute(int n, const int *__restrict__ perm, const double4 *__
 // any lane of the wave has one, which is almost every candidate; queued,
 // every lane works through its entries together.
 constexpr int NB_QUEUE = 12;
-#ifndef PYSIC_NB_UNIFORM_SPAN
-#define PYSIC_NB_UNIFORM_SPAN 4
-#endif
 
-template <class Geo, bool DENSE>
+template <class Geo>
 __global__ __launch_bounds__(256) void k_neighbors_pf(int n, Geo geo,
                                                       const double4 *__restrict__ pos,
                                                       const float4 *__restrict__ wpos,
@@ -410,26 +452,21 @@ __global__ __launch_bounds__(256) void k_neighbors_pf(int n, Geo geo,
     const float c2sure = (float)c2lim - 2.0f * margin2;
     int count = 0, nq = 0;
     constexpr int SHELL = 1 << 30;  // queue flag: exact test needed (images use bits 0-29)
-    // write out the queued entries, in queue order.  Sparse bins (a few hits
-    // among many candidates): an entry holds the candidate and its bin's
-    // periodic shift, and the pair's image, bin shift + wrap(t) - wrap(s), is
-    // formed here, once per accepted candidate rather than in the scan loop,
-    // where the branch runs whenever any lane of the wave has a hit; the atom
-    // itself at image 0 is dropped here.  Dense bins (most candidates hit):
-    // the image is formed at the hit, as the drain would otherwise reload
-    // each entry's wrap.  Shell entries first pass the exact test.
+    // write out the queued entries, in queue order.  An entry holds the
+    // candidate and its bin's periodic shift, and the pair's image, bin shift
+    // + wrap(t) - wrap(s), is formed here, once per accepted candidate rather
+    // than in the scan loop, where the branch runs whenever any lane of the
+    // wave has a hit; the atom itself at image 0 is dropped here.  Shell
+    // entries first pass the exact test.
     auto drain = [&]() {
         for (int u = 0; u < nq; ++u) {
             const int t = q_slot[u][tid];
             const int q = q_shift[u][tid];
-            int im = q & ~SHELL;
-            if constexpr (!DENSE) {
-                const int wt = __float_as_int(wpos[t].w);
-                const int ox = img_x(im) - wsx + img_x(wt), oy = img_y(im) - wsy + img_y(wt),
-                          oz = img_z(im) - wsz + img_z(wt);
-                if (t == s && ox == 0 && oy == 0 && oz == 0) continue;
-                im = pack_img(ox, oy, oz);
-            }
+            const int sh = q & ~SHELL, wt = __float_as_int(wpos[t].w);
+            const int ox = img_x(sh) - wsx + img_x(wt), oy = img_y(sh) - wsy + img_y(wt),
+                      oz = img_z(sh) - wsz + img_z(wt);
+            if (t == s && ox == 0 && oy == 0 && oz == 0) continue;
+            const int im = pack_img(ox, oy, oz);
             if ((q & SHELL) && !(dot64(separation64(ps, pos[t], im, g.v)) < c2lim)) continue;
             if (count < cap) {
                 nbr[(size_t)count * n + s] = t;
@@ -440,115 +477,46 @@ __global__ __launch_bounds__(256) void k_neighbors_pf(int n, Geo geo,
         nq = 0;
     };
     // FP32 test of every candidate of one bin (row + bx) under the bin's
-    // periodic shift (sx, sy, sz).  UNIFORM: every lane of the wave scans the
-    // same candidates, so a full queue drains every lane's queue at once.
-    auto scan_bin = [&](auto uniform_tag, int row, int bx, int sx, int sy, int sz) {
-        constexpr bool UNIFORM = decltype(uniform_tag)::value;
+    // periodic shift (sx, sy, sz).
+    auto scan_bin = [&](int row, int bx, int sx, int sy, int sz) {
         const float sxf = (float)sx, syf = (float)sy, szf = (float)sz;
         const float shx = sxf * v0x + syf * v1x + szf * v2x - qs.x;
         const float shy = sxf * v0y + syf * v1y + szf * v2y - qs.y;
         const float shz = sxf * v0z + syf * v1z + szf * v2z - qs.z;
         const int sh = pack_img(sx, sy, sz);
-        const int ox0 = sx - wsx, oy0 = sy - wsy, oz0 = sz - wsz;
         const int t1 = start[row + bx + 1];
         for (int t = start[row + bx]; t < t1; ++t) {
             const float4 qt = wpos[t];
             const float fx = qt.x + shx, fy = qt.y + shy, fz = qt.z + shz;
             const float d2f = fx * fx + fy * fy + fz * fz;
-            const bool hit = d2f < c2f;
-            if (UNIFORM) {
-                if (__ballot(hit && nq == NB_QUEUE)) drain();
-            }
-            if (hit) {
-                if (!UNIFORM && nq == NB_QUEUE) drain();
-                const int flag = d2f < c2sure ? 0 : SHELL;
-                if constexpr (DENSE) {
-                    const int wt = __float_as_int(qt.w);
-                    const int ox = ox0 + img_x(wt), oy = oy0 + img_y(wt), oz = oz0 + img_z(wt);
-                    if (!(t == s && ox == 0 && oy == 0 && oz == 0)) {
-                        q_slot[nq][tid] = t;
-                        q_shift[nq][tid] = pack_img(ox, oy, oz) | flag;
-                        ++nq;
-                    }
-                } else {
-                    q_slot[nq][tid] = t;
-                    q_shift[nq][tid] = sh | flag;
-                    ++nq;
-                }
+            if (d2f < c2f) {
+                if (nq == NB_QUEUE) drain();
+                q_slot[nq][tid] = t;
+                q_shift[nq][tid] = sh | (d2f < c2sure ? 0 : SHELL);
+                ++nq;
             }
         }
     };
-    // Wave-uniform scan: when the wave's atoms share one bin row of a
-    // periodic cell at least 3 bins wide on every axis, and span at most
-    // PYSIC_NB_UNIFORM_SPAN + 1 bins of it (dense bins: the union of their
-    // stencils is then at most (SPAN + 3) / 3 times one stencil), every lane
-    // scans that union -- the 9 neighboring rows over x from one bin before
-    // the wave's first bin to one after its last.  Loop bounds
-    // and candidates are then the same for all lanes (scalar loads, no
-    // divergence); the extra candidates lie beyond every lane's cutoff or
-    // are genuine neighbors, and with 3 or more bins per axis no atom image
-    // is reached twice, so the accepted set is the 27-bin stencil's.
-    bool uniform = false;
-    int ux0 = 0, ux1 = 0, uc1 = 0, uc2 = 0;
-    if constexpr (DENSE) {  // one periodic cell, >= 3 bins per axis (checked by the host)
-        {
-            const unsigned long long act = __ballot(1);
-            const int lo = __ffsll((unsigned long long)act) - 1;
-            const int hi = 63 - __clzll((long long)act);
-            // atoms are sorted by bin: the first active lane holds the
-            // wave's lowest bin, the last its highest
-            const int kmin = __builtin_amdgcn_readfirstlane(__shfl(k, lo));
-            const int kmax = __builtin_amdgcn_readfirstlane(__shfl(k, hi));
-            if (kmin / g.dim[0] == kmax / g.dim[0] &&
-                kmax - kmin <= PYSIC_NB_UNIFORM_SPAN) {
-                uniform = true;
-                ux0 = kmin % g.dim[0];
-                ux1 = kmax % g.dim[0];
-                uc1 = (kmin / g.dim[0]) % g.dim[1];
-                uc2 = kmin / (g.dim[0] * g.dim[1]);
-            }
-        }
-    }
-    if (uniform) {
-        for (int dz = -1; dz <= 1; ++dz) {
-            int bz = uc2 + dz, sz = 0;
+    for (int dz = -1; dz <= 1; ++dz) {
+        int bz = c2 + dz, sz = 0;
+        if (g.pbc[2]) {
             if (bz < 0) { bz += g.nc[2]; sz = -1; }
             else if (bz >= g.nc[2]) { bz -= g.nc[2]; sz = 1; }
-            for (int dy = -1; dy <= 1; ++dy) {
-                int by = uc1 + dy, sy = 0;
+        } else if (bz < 0 || bz >= g.dim[2]) continue;
+        for (int dy = -1; dy <= 1; ++dy) {
+            int by = c1 + dy, sy = 0;
+            if (g.pbc[1]) {
                 if (by < 0) { by += g.nc[1]; sy = -1; }
                 else if (by >= g.nc[1]) { by -= g.nc[1]; sy = 1; }
-                const int row = g.dim[0] * (by + g.dim[1] * bz);
-                for (int x = ux0 - 1; x <= ux1 + 1; ++x) {
-                    int bx = x, sx = 0;
+            } else if (by < 0 || by >= g.dim[1]) continue;
+            const int row = g.dim[0] * (by + g.dim[1] * bz);
+            for (int dx = -1; dx <= 1; ++dx) {
+                int bx = c0 + dx, sx = 0;
+                if (g.pbc[0]) {
                     if (bx < 0) { bx += g.nc[0]; sx = -1; }
                     else if (bx >= g.nc[0]) { bx -= g.nc[0]; sx = 1; }
-                    scan_bin(std::true_type{}, row, bx, sx, sy, sz);
-                }
-            }
-        }
-    } else {
-        for (int dz = -1; dz <= 1; ++dz) {
-            int bz = c2 + dz, sz = 0;
-            if (g.pbc[2]) {
-                if (bz < 0) { bz += g.nc[2]; sz = -1; }
-                else if (bz >= g.nc[2]) { bz -= g.nc[2]; sz = 1; }
-            } else if (bz < 0 || bz >= g.dim[2]) continue;
-            for (int dy = -1; dy <= 1; ++dy) {
-                int by = c1 + dy, sy = 0;
-                if (g.pbc[1]) {
-                    if (by < 0) { by += g.nc[1]; sy = -1; }
-                    else if (by >= g.nc[1]) { by -= g.nc[1]; sy = 1; }
-                } else if (by < 0 || by >= g.dim[1]) continue;
-                const int row = g.dim[0] * (by + g.dim[1] * bz);
-                for (int dx = -1; dx <= 1; ++dx) {
-                    int bx = c0 + dx, sx = 0;
-                    if (g.pbc[0]) {
-                        if (bx < 0) { bx += g.nc[0]; sx = -1; }
-                        else if (bx >= g.nc[0]) { bx -= g.nc[0]; sx = 1; }
-                    } else if (bx < 0 || bx >= g.dim[0]) continue;
-                    scan_bin(std::false_type{}, row, bx, sx, sy, sz);
-                }
+                } else if (bx < 0 || bx >= g.dim[0]) continue;
+                scan_bin(row, bx, sx, sy, sz);
             }
         }
     }
@@ -939,6 +907,153 @@ __global__ __launch_bounds__(256) void k_neighbors_group(int n, CellGeom g,
     }
 }
 
+// The lane-parallel scan where one bin on each side suffices (every cell at
+// least as wide as the list radius).  The group's lanes first load the ranges
+// of all 27 bins together (a few per lane) and scan their lengths, so the
+// candidates of the whole stencil are one stream; a lane then takes every
+// G-th of it, U at a time with their loads issued together, and finds each
+// candidate's bin by stepping along the offsets in LDS.  Candidates are
+// tested as in k_neighbors_pf: FP32 wrapped positions first, the exact test
+// in the thin shell.  The stream runs in the per-atom scan's order and the
+// hits are compacted in it, so the lists are k_neighbors_group's, entry by
+// entry.
+// Bound: a chain of three dependent loads (bin ranges, candidates, list
+// stores), where the scan column by column is one of eighteen or more.
+// 5,757 atoms of silicon at 3.5 A: 30.0 -> 10.6 us; 24,576 of SiO2 at 3.55 A:
+// 37.7 -> 14.4; 13,500 of argon at 9.0 A (16 lanes): 65.3 -> 30.
+// Dense bins, 1,048,576 argon atoms: 16 lanes and 2 candidates a lane 1303 us,
+// 8 and 4 1291, 32 and 4 1518; 262,144 ions at 10.5 A: 737, 815, 769.  Blocks
+// of one XCD take consecutive atoms, so the 4-byte stores of neighboring
+// atoms meet in one L2 (1425 us without).
+template <int G, int U>
+__global__ __launch_bounds__(256) void k_neighbors_lanes(int n, CellGeom g,
+                                                         const double4 *__restrict__ pos,
+                                                         const float4 *__restrict__ wpos,
+                                                         const int *__restrict__ key,
+                                                         const int *__restrict__ wrap,
+                                                         const int *__restrict__ start,
+                                                         const double *__restrict__ cut, int cap,
+                                                         float margin2, int *__restrict__ nbr,
+                                                         int *__restrict__ nimg,
+                                                         int *__restrict__ ncnt,
+                                                         int *__restrict__ flags)
+{
+    constexpr int APB = 256 / G, BINS = 27, PER = (BINS + G - 1) / G;
+    __shared__ int s_base[APB][BINS + 1];   // stream position of each bin's first atom
+    __shared__ int s_first[APB][BINS];      // its slot minus that position
+    __shared__ int s_shift[APB][BINS];      // the bin's periodic shift, packed
+    const int a = threadIdx.x / G, l = threadIdx.x % G;
+    const int s = xcd_block(gridDim.x) * APB + a;
+    const bool valid = s < n;
+    const int gbase = ((threadIdx.x & 63) / G) * G;
+    const unsigned long long gmask = (1ull << G) - 1ull, below = (1ull << l) - 1ull;
+    const int k = valid ? key[s] : 0, ws = valid ? wrap[s] : 0;
+    const float4 qs = valid ? wpos[s] : make_float4(0, 0, 0, 0);
+    const double4 ps = valid ? pos[s] : make_double4(0, 0, 0, 0);
+    const double cs = valid ? cut[s] : 0.0, csq = cs * cs;
+    const int c0 = k % g.dim[0], c1 = (k / g.dim[0]) % g.dim[1], c2 = k / (g.dim[0] * g.dim[1]);
+    // ranges of bins l, l + G, ... in (dz, dy, dx) order
+    int first[PER], len[PER], shift[PER];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+        const int b = l + p * G;
+        first[p] = len[p] = shift[p] = 0;
+        if (!valid || b >= BINS) continue;
+        int x[3] = {c0 + b % 3 - 1, c1 + (b / 3) % 3 - 1, c2 + b / 9 - 1}, sh[3] = {0, 0, 0};
+        bool in = true;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (g.pbc[d]) {
+                sh[d] = x[d] < 0 ? -1 : x[d] >= g.nc[d] ? 1 : 0;
+                x[d] -= sh[d] * g.nc[d];
+            } else {
+                in = in && x[d] >= 0 && x[d] < g.dim[d];
+            }
+        }
+        if (!in) continue;
+        const int at = x[0] + g.dim[0] * (x[1] + g.dim[1] * x[2]);
+        first[p] = start[at];
+        len[p] = start[at + 1] - first[p];
+        shift[p] = pack_img(sh[0], sh[1], sh[2]);
+    }
+    int total = 0;
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+        int incl = len[p];
+#pragma unroll
+        for (int d = 1; d < G; d <<= 1) {
+            const int x = __shfl_up(incl, d, G);
+            if (l >= d) incl += x;
+        }
+        const int b = l + p * G, at = total + incl - len[p];
+        if (b < BINS) {
+            s_base[a][b] = at;
+            s_first[a][b] = first[p] - at;
+            s_shift[a][b] = shift[p];
+        }
+        total += __shfl(incl, G - 1, G);
+    }
+    if (l == 0) s_base[a][BINS] = total;
+    __syncthreads();
+    const float v0x = (float)g.v[0], v0y = (float)g.v[1], v0z = (float)g.v[2];
+    const float v1x = (float)g.v[3], v1y = (float)g.v[4], v1z = (float)g.v[5];
+    const float v2x = (float)g.v[6], v2y = (float)g.v[7], v2z = (float)g.v[8];
+    const float c2f = (float)csq + margin2, c2sure = (float)csq - 2.0f * margin2;
+    int bin = 0, next = s_base[a][1], count = 0;
+    // the lanes of a wave leave together: the ballots below are the wave's
+    int longest = total;
+#pragma unroll
+    for (int d = G; d < 64; d <<= 1) longest = max(longest, __shfl_xor(longest, d));
+    for (int t0 = 0; t0 < longest; t0 += G * U) {
+        int slot[U], sh[U];
+        float4 w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int c = t0 + u * G + l;
+            slot[u] = -1;
+            sh[u] = 0;
+            w[u] = make_float4(0, 0, 0, 0);
+            if (c < total) {
+                while (c >= next) next = s_base[a][++bin + 1];
+                slot[u] = s_first[a][bin] + c;
+                sh[u] = s_shift[a][bin];
+                w[u] = wpos[slot[u]];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            bool hit = false;
+            int im = 0;
+            if (slot[u] >= 0) {
+                const int sx = img_x(sh[u]), sy = img_y(sh[u]), sz = img_z(sh[u]);
+                const int wt = __float_as_int(w[u].w);
+                const float fx = (float)sx, fy = (float)sy, fz = (float)sz;
+                const float dx = w[u].x - qs.x + (fx * v0x + fy * v1x + fz * v2x);
+                const float dy = w[u].y - qs.y + (fx * v0y + fy * v1y + fz * v2y);
+                const float dz = w[u].z - qs.z + (fx * v0z + fy * v1z + fz * v2z);
+                const float d2 = dx * dx + dy * dy + dz * dz;
+                if (!(d2 >= c2f)) {   // not a number (beyond FP32): left to the exact test
+                    im = pack_img(sx + img_x(wt) - img_x(ws), sy + img_y(wt) - img_y(ws),
+                                  sz + img_z(wt) - img_z(ws));
+                    hit = d2 < c2sure || dot64(separation64(ps, pos[slot[u]], im, g.v)) < csq;
+                    if (slot[u] == s && im == pack_img(0, 0, 0)) hit = false;
+                }
+            }
+            const unsigned long long gb = (__ballot(hit) >> gbase) & gmask;
+            const int at = count + __popcll(gb & below);
+            if (hit && at < cap) {
+                nbr[(size_t)at * n + s] = slot[u];
+                nimg[(size_t)at * n + s] = im;
+            }
+            count += __popcll(gb);
+        }
+    }
+    if (valid && l == 0) {
+        ncnt[s] = count < cap ? count : cap;
+        if (count > cap) atomicMax(flags, count);
+    }
+}
+
 }  // namespace
 
 // Bins per axis: floor(perpendicular width / max_cut) as in
@@ -1082,10 +1197,14 @@ void nb_swap_state(System &S)
     std::swap(S.key, S.key2);
     std::swap(S.wrap, S.wrap2);
     std::swap(S.cellstart, S.prevstart);
+    std::swap(S.dirty, S.dirty2);
 }
 
-// The counting sort after binning: scan of the bin counts, scatter, per-bin
-// sort by original index, permutation of every per-atom array.
+// bins as k_scan_one reads them: whole int4 for 1024 threads
+static int scan_room(int nbins) { return (nbins + 4095) / 4096 * 4096; }
+
+// The counting sort after binning: scan of the bin counts, scatter, and the
+// permutation of every per-atom array, in each bin by original index.
 static void sort_binned(System &S)
 {
     const int n = S.n;
@@ -1093,22 +1212,25 @@ static void sort_binned(System &S)
     hipStream_t st = S.stream;
     const int nb = div_up(nbins, SCAN_BLK);
     const int all_dirty = S.order_valid ? 0 : 1;
-    k_scan_local<<<nb, SCAN_T, 0, st>>>(nbins, S.cellcount.p, S.scanloc.p, S.scanblk.p,
-                                        S.cellfill.p);
-    k_scan_blocks<<<1, SCAN_T, 0, st>>>(nb, S.scanblk.p, S.scanloc.p, nbins);
+    if (nbins <= SCAN_ONE) {
+        k_scan_one<<<1, 1024, 0, st>>>(scan_room(nbins) / 4096, (int4 *)S.cellcount.p,
+                                       (int4 *)S.scanloc.p, (int4 *)S.cellfill.p, nb, S.scanblk.p);
+    } else {
+        k_scan_local<<<nb, SCAN_T, 0, st>>>(nbins, S.cellcount.p, S.scanloc.p, S.scanblk.p,
+                                            S.cellfill.p);
+        k_scan_blocks<<<1, SCAN_T, 0, st>>>(nb, S.scanblk.p, S.scanloc.p, nbins);
+    }
     // S.cellstart holds the last sort's starts here (the old slot ranges)
     k_scatter<<<div_up(n, 256), 256, 0, st>>>(n, S.key.p, S.scanloc.p, S.scanblk.p,
                                               S.cellstart.p, S.dirty.p, all_dirty, S.cellfill.p,
                                               S.perm.p, S.flags.p);
-    k_cellsort<<<div_up(nbins, 256), 256, 0, st>>>(nbins, n, S.scanloc.p, S.scanblk.p, S.perm.p,
-                                                   S.id.p, S.dirty.p, all_dirty, S.prevstart.p);
     with_geo(S, [&](auto geo) {
         using Geo = decltype(geo);
         auto kern = S.qc_uniform ? k_permute<Geo, false> : k_permute<Geo, true>;
-        kern<<<div_up(n, 256), 256, 0, st>>>(n, S.perm.p, S.pos.p, S.mom.p, S.q.p, S.cut.p, S.id.p,
-                                             S.key.p, S.wrap.p, S.pos2.p, S.mom2.p, S.q2.p,
-                                             S.cut2.p, S.id2.p, S.key2.p, S.wrap2.p, geo,
-                                             S.wpos.p, S.flags.p);
+        kern<<<div_up(std::max(n, nbins), 256), 256, 0, st>>>(
+            n, nbins, S.scanloc.p, S.scanblk.p, S.perm.p, S.dirty.p, S.dirty2.p, all_dirty,
+            S.prevstart.p, S.pos.p, S.mom.p, S.q.p, S.cut.p, S.id.p, S.key.p, S.wrap.p, S.pos2.p,
+            S.mom2.p, S.q2.p, S.cut2.p, S.id2.p, S.key2.p, S.wrap2.p, geo, S.wpos.p, S.flags.p);
     });
     HIP_TRY(hipGetLastError());
     // the new starts went to prevstart, which nb_swap_state makes cellstart
@@ -1122,14 +1244,15 @@ static void ensure_sort_buffers(System &S)
     S.key.ensure(n); S.key2.ensure(n);
     S.wrap.ensure(n); S.wrap2.ensure(n);
     S.perm.ensure(n);
-    const bool fresh = S.cellcount.cap < (size_t)nbins || S.cellfill.cap < (size_t)nbins ||
-                       S.dirty.cap < (size_t)nbins || !S.cellcount.p || !S.dirty.p;
-    S.cellcount.ensure(nbins);
-    S.cellfill.ensure(nbins);
-    S.dirty.ensure(nbins);
+    const size_t room = scan_room(nbins);
+    const bool fresh = S.cellcount.cap < room || S.dirty.cap < room || S.dirty2.cap < room;
+    S.cellcount.ensure(room);
+    S.cellfill.ensure(room);
+    S.dirty.ensure(room);
+    S.dirty2.ensure(room);
     S.cellstart.ensure((size_t)nbins + 1);
     S.prevstart.ensure((size_t)nbins + 1);
-    S.scanloc.ensure((size_t)nbins + 1);
+    S.scanloc.ensure(room + 1);
     S.scanblk.ensure(div_up(nbins, SCAN_BLK) + 1);
     S.pos2.ensure(n); S.mom2.ensure(n); S.q2.ensure(n); S.cut2.ensure(n);
     S.id2.ensure(n);
@@ -1137,7 +1260,8 @@ static void ensure_sort_buffers(System &S)
     S.flags.ensure(4);
     if (fresh || !S.bins_clean) {
         // counts and dirty flags start at zero (a kernel: this may be captured)
-        k_fill_int<<<div_up(2 * nbins, 256), 256, 0, S.stream>>>(nbins, S.cellcount.p, S.dirty.p);
+        k_fill_int<<<div_up(3 * (int)room, 256), 256, 0, S.stream>>>((int)room, S.cellcount.p,
+                                                                     S.dirty.p, S.dirty2.p);
         S.order_valid = false;
         S.bins_clean = true;
     }
@@ -1212,62 +1336,63 @@ void nb_build_lists(System &S)
     double apb = n / interior;  // atoms per bin
     PYSIC_REQUIRE(S.ncells == 0 || S.nb_method == 0 || S.nb_method == 1 || S.nb_method == 5,
                   PYSIC_EINVAL, "a batch of cells takes neighbor method 0, 1 or 5");
-    // the default for one cell below 2^17 atoms is the lane-parallel scan:
-    // one thread per atom would leave most of the chip idle (measured on
-    // 24,576 atoms of SiO2 at 3.55 A: 91 us per thread, 34 us per group)
-    // a cell thinner than the cutoff: the lane-parallel scan, the one that
-    // searches several bins on each side
+    // the default for one cell below 2^17 atoms, and for one with dense bins
+    // at any size, is the lane-parallel scan.  Sparse bins (silicon at 3.5 A):
+    // 64,000 atoms 23 us against 34 with a thread per atom, 140,608 43 against
+    // 38, 1,048,576 271 against 125.  Dense bins: 262,144 ions at 10.5 A 737
+    // against 1915, 1,048,576 argon atoms at 9.0 A 1303 against 1830.
+    // a cell thinner than the cutoff: the lane-parallel scan that searches
+    // several bins on each side
     const bool thin = S.ncells == 0 && (g.reach[0] > 1 || g.reach[1] > 1 || g.reach[2] > 1);
+    const bool sparse = apb * 3.0 <= 10.0;
     const int method =
-        ((S.nb_method == 0 && S.ncells == 0 && n < (1 << 17)) || thin) ? 4 : S.nb_method;
+        ((S.nb_method == 0 && S.ncells == 0 && (n < (1 << 17) || !sparse)) || thin) ? 4
+                                                                                    : S.nb_method;
     bool brick = method == 2 || method == 3;
     hipEvent_t ev;
     S.timer.begin("neighbors", st, &ev);
+    // FP32 prefilter margin: bound on the rounding of the FP32 squared
+    // distance of wrapped positions (|error| per component <= ~1.2e-6 L,
+    // taken 2.5x larger); open axes leave positions unbounded: no
+    // prefilter.  A batch takes the largest cell's bound.
+    auto margin_of = [&](const CellGeom &c) {
+        if (!(c.pbc[0] && c.pbc[1] && c.pbc[2])) return 3.0e38f;
+        double L = 0.0;
+        for (int a = 0; a < 3; ++a)
+            L += std::sqrt(c.v[3 * a] * c.v[3 * a] + c.v[3 * a + 1] * c.v[3 * a + 1] +
+                           c.v[3 * a + 2] * c.v[3 * a + 2]);
+        double delta = 3.0e-6 * L;
+        return (float)(4.0 * std::sqrt(3.0) * S.max_cut * delta + 12.0 * delta * delta);
+    };
     if (method == 0 || method == 5) {
-        // FP32 prefilter margin: bound on the rounding of the FP32 squared
-        // distance of wrapped positions (|error| per component <= ~1.2e-6 L,
-        // taken 2.5x larger); open axes leave positions unbounded: no
-        // prefilter.  A batch takes the largest cell's bound.
         float margin2 = 0.0f;
-        auto margin_of = [&](const CellGeom &c) {
-            if (!(c.pbc[0] && c.pbc[1] && c.pbc[2])) return 3.0e38f;
-            double L = 0.0;
-            for (int a = 0; a < 3; ++a)
-                L += std::sqrt(c.v[3 * a] * c.v[3 * a] + c.v[3 * a + 1] * c.v[3 * a + 1] +
-                               c.v[3 * a + 2] * c.v[3 * a + 2]);
-            double delta = 3.0e-6 * L;
-            return (float)(4.0 * std::sqrt(3.0) * S.max_cut * delta + 12.0 * delta * delta);
-        };
         if (S.ncells == 0) margin2 = margin_of(g);
         for (int c = 0; c < S.ncells; ++c) margin2 = std::max(margin2, margin_of(S.hcells[c]));
-        // dense bins of one periodic cell: the kernel with the wave-uniform
-        // scan (a separate instance: its second scan path costs registers)
-        const bool dense = S.ncells == 0 && g.pbc[0] && g.pbc[1] && g.pbc[2] && g.nc[0] >= 3 &&
-                           g.nc[1] >= 3 && g.nc[2] >= 3 && apb >= 6.0;
         with_geo(S, [&](auto geo) {
             using Geo = decltype(geo);
-            auto go = [&](auto kern) {
-                kern<<<div_up(n, 256), 256, 0, st>>>(n, geo, S.pos.p, S.wpos.p, S.key.p, S.wrap.p,
-                                                     S.cellstart.p, S.cut.p, S.cap, margin2,
-                                                     S.nbr.p, S.nimg.p, S.ncnt.p, S.flags.p);
-            };
-            if constexpr (std::is_same<Geo, GeoOne>::value) {
-                if (dense) go(k_neighbors_pf<Geo, true>);
-                else go(k_neighbors_pf<Geo, false>);
-            } else {
-                go(k_neighbors_pf<Geo, false>);
-            }
+            k_neighbors_pf<Geo><<<div_up(n, 256), 256, 0, st>>>(
+                n, geo, S.pos.p, S.wpos.p, S.key.p, S.wrap.p, S.cellstart.p, S.cut.p, S.cap,
+                margin2, S.nbr.p, S.nimg.p, S.ncnt.p, S.flags.p);
         });
     } else if (method == 4) {
         // lane-parallel scan; wider groups when the bins are dense
-        if (apb * 3.0 <= 10.0)
-            k_neighbors_group<8><<<div_up(n, 256 / 8), 256, 0, st>>>(
-                n, g, S.pos.p, S.key.p, S.wrap.p, S.cellstart.p, S.cut.p, S.cap, S.nbr.p, S.nimg.p,
-                S.ncnt.p, S.flags.p);
-        else
-            k_neighbors_group<32><<<div_up(n, 256 / 32), 256, 0, st>>>(
-                n, g, S.pos.p, S.key.p, S.wrap.p, S.cellstart.p, S.cut.p, S.cap, S.nbr.p, S.nimg.p,
-                S.ncnt.p, S.flags.p);
+        auto go = [&](auto kern, int lanes) {
+            kern<<<div_up(n, 256 / lanes), 256, 0, st>>>(n, g, S.pos.p, S.key.p, S.wrap.p,
+                                                         S.cellstart.p, S.cut.p, S.cap, S.nbr.p,
+                                                         S.nimg.p, S.ncnt.p, S.flags.p);
+        };
+        auto stream = [&](auto kern, int lanes) {
+            kern<<<div_up(n, 256 / lanes), 256, 0, st>>>(
+                n, g, S.pos.p, S.wpos.p, S.key.p, S.wrap.p, S.cellstart.p, S.cut.p, S.cap,
+                margin_of(g), S.nbr.p, S.nimg.p, S.ncnt.p, S.flags.p);
+        };
+        if (thin) {
+            if (sparse) go(k_neighbors_group<8>, 8);
+            else go(k_neighbors_group<32>, 32);
+        } else {
+            if (sparse) stream(k_neighbors_lanes<8, 4>, 8);
+            else stream(k_neighbors_lanes<16, 2>, 16);
+        }
     } else if (!brick) {
         with_geo(S, [&](auto geo) {
             k_neighbors<decltype(geo)><<<div_up(n, 256), 256, 0, st>>>(

@@ -82,7 +82,8 @@ struct System {
     DBuf<float4> wpos;          // wrapped positions, FP32 (neighbor prefilter)
     DBuf<int> cellcount, cellstart, cellfill, scanblk;
     DBuf<int> prevstart;        // the previous sort's cell starts (its slot ranges)
-    DBuf<int> dirty;            // per bin: an atom entered or left it since the last sort
+    DBuf<int> dirty, dirty2;    // per bin: an atom entered or left it since the last sort
+                                // (2: the sort before's, cleared by this one)
     DBuf<int> scanloc;          // cell starts within blocks of 1024 bins
     bool order_valid = false;   // the slot order is the last sort's (key[] holds its bins)
     bool unique_images = false; // no atom reaches two images of another within the list radius
