@@ -48,6 +48,9 @@ struct EwaldState {
     DBuf<double2> wl;       // per-atom exp(2 pi i 16 u3)
     DBuf<double4> zw;       // coefficients of the per-atom sums (plan order)
     DBuf<int> kpk;          // packed (k1, k2, l0) per plan slot
+    DBuf<double> dchi, mx;  // relaxation: differences, their block maxima
+    DBuf<int> stop;         // relaxation of a small system: it has ended
+    hipEvent_t seen[2] = {nullptr, nullptr};   // its last two evaluations' errors are out
     DBuf<unsigned long long> hpart;   // state fingerprint partials
     // sk and th hold the structure factors of the state whose fingerprint
     // is sk_hash

@@ -87,8 +87,8 @@ __global__ __launch_bounds__(EB) void k_real(int n, CellGeom g, const double4 *_
                                              const Model *__restrict__ M, int ewald_on, double rc,
                                              double inv_eps_4pi, double inv_sig_sqrt2,
                                              double inv_sig_sqrt2pi, double inv_sig_sq2,
-                                             double bg_chi, const double *__restrict__ bg_dev,
-                                             int self_on, double *__restrict__ out1,
+                                             double inv_eps_2v, double sigma,
+                                             const double *__restrict__ qsum, int self_on, double *__restrict__ out1,
                                              double4 *__restrict__ frc, double *__restrict__ part)
 {
     constexpr int NBU = 4;
@@ -117,8 +117,8 @@ __global__ __launch_bounds__(EB) void k_real(int n, CellGeom g, const double4 *_
             if (sub == 0) {
                 // self (Potentials.f90:2126) and background (2166) electronegativity
                 const double qs = qi * sc[i];
-                const double bg = bg_dev ? bg_dev[0] : bg_chi;
-                chi += 2.0 * qs * inv_eps_4pi * inv_sig_sqrt2pi + sc[i] * bg;
+                chi += 2.0 * qs * inv_eps_4pi * inv_sig_sqrt2pi;
+                if (MODE == 3) chi += sc[i] * (-inv_eps_2v * (-sigma * sigma * qsum[0]));
             }
             const double inv2perpi = 2.0 * inv_sig_sqrt2pi;
             const double rc2 = rc * rc, lo2 = rc2 * (1.0 - 1e-12), hi2 = rc2 * (1.0 + 1e-12);
@@ -751,31 +751,23 @@ __global__ void k_dipole_sums(int n, const double4 *__restrict__ pos,
     if (threadIdx.x < 3) part[(size_t)blockIdx.x * 8 + threadIdx.x] = r[threadIdx.x][0];
 }
 
-// background electronegativity from the reduced charge sum (same operations
-// as the host form - inv_eps_2v * (-sigma^2 Q), Potentials.f90:2166-2167)
-__global__ void k_background(const double *__restrict__ qsum, double *__restrict__ out,
-                             double inv_eps_2v, double sigma)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) out[0] = -inv_eps_2v * (-sigma * sigma * qsum[0]);
-}
-
-// Deterministic sum of `count` strided partials (component c of stride 8).
-__global__ void k_sum_partials(int count, int stride, int ncomp, const double *__restrict__ part,
-                               double *__restrict__ out)
+// Deterministic sum of `count` strided partials, a block per component (one
+// after another in one block they took 5.4 us for seven, a block each 3).
+__global__ __launch_bounds__(EB) void k_sum_partials(int count, int stride,
+                                                     const double *__restrict__ part,
+                                                     double *__restrict__ out)
 {
     __shared__ double lds[EB];
-    for (int c = 0; c < ncomp; ++c) {
-        double s = 0.0;
-        for (int b = threadIdx.x; b < count; b += EB) s += part[(size_t)b * stride + c];
-        lds[threadIdx.x] = s;
-        __syncthreads();
-        for (int w = EB / 2; w > 0; w >>= 1) {
-            if (threadIdx.x < w) lds[threadIdx.x] += lds[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) out[c] = lds[0];
+    const int c = blockIdx.x;
+    double s = 0.0;
+    for (int b = threadIdx.x; b < count; b += EB) s += part[(size_t)b * stride + c];
+    lds[threadIdx.x] = s;
+    __syncthreads();
+    for (int w = EB / 2; w > 0; w >>= 1) {
+        if (threadIdx.x < w) lds[threadIdx.x] += lds[threadIdx.x + w];
         __syncthreads();
     }
+    if (threadIdx.x == 0) out[c] = lds[0];
 }
 
 __global__ void k_gather_scaler(int n, const int *__restrict__ id, const double *__restrict__ src,
@@ -847,6 +839,84 @@ __global__ void k_sum_chi(int n, const double *__restrict__ chi, double *__restr
         __syncthreads();
     }
     if (threadIdx.x == 0) part[(size_t)blockIdx.x * 8] = red[0];
+}
+
+// The rest of a relaxation step of a small system in one block, where the
+// four kernels above and the next step's k_relax_update and charge sum are
+// little but launches: mean, differences, the rates' second half, the stop
+// test on max(chi - mean) (relaxation.py:449), and, if the relaxation goes on,
+// the next step's charges and rates and their charge sum.  `stop` is set when
+// it does not, and a step queued past that point changes nothing: the host
+// queues step k + 1 before it has seen step k's error.  768 ions: 60 steps
+// 9.6 -> 4.4 ms with this, the smaller chunks of S(k) and no wait between steps.
+constexpr int RELAX_ONE = 8192, RELAX_PER = RELAX_ONE / 1024;
+__global__ __launch_bounds__(1024) void k_relax_tail(int n, const double *__restrict__ chi,
+                                                     double *__restrict__ q,
+                                                     double *__restrict__ rate,
+                                                     const double *__restrict__ sc, int first,
+                                                     int more, double dt, double inv_mq,
+                                                     double friction, double future,
+                                                     double tolerance, int *__restrict__ stop,
+                                                     double *__restrict__ qsum,
+                                                     double *__restrict__ error)
+{
+    __shared__ double lds[16];
+    const int t = threadIdx.x;
+    if (*stop) return;   // the whole block: nobody has written it yet
+    auto reduce = [&](double v, auto op) {
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) v = op(v, __shfl_xor(v, m));
+        __syncthreads();   // the previous reduction has been read
+        if ((t & 63) == 0) lds[t >> 6] = v;
+        __syncthreads();
+        double r = lds[0];
+        for (int w = 1; w < 16; ++w) r = op(r, lds[w]);
+        return r;
+    };
+    auto plus = [](double a, double b) { return a + b; };
+    auto most = [](double a, double b) { return fmax(a, b); };
+    double f[RELAX_PER], r[RELAX_PER], s = 0.0, m = -INFINITY;
+#pragma unroll
+    for (int p = 0; p < RELAX_PER; ++p) {
+        const int i = t + 1024 * p;
+        f[p] = i < n ? chi[i] : 0.0;
+        r[p] = i < n ? rate[i] : 0.0;
+        s += f[p];
+    }
+    const double mean = reduce(s, plus) / n;
+#pragma unroll
+    for (int p = 0; p < RELAX_PER; ++p) {
+        f[p] -= mean;
+        if (!first) r[p] = future * (r[p] + f[p] * (0.5 * inv_mq * dt));
+        if (t + 1024 * p < n) m = fmax(m, f[p]);
+    }
+    const double err = reduce(m, most);
+    // (an error that is not finite is the host's to report: nothing moves on)
+    const bool on = isfinite(err) && (first ? more != 0 : err > tolerance);
+    double sum = 0.0;
+#pragma unroll
+    for (int p = 0; p < RELAX_PER; ++p) {
+        const int i = t + 1024 * p;
+        if (i >= n) continue;
+        if (on && more) {
+            const double x = q[i] + (r[p] * dt + (f[p] - friction * r[p]) * inv_mq * (dt * dt));
+            q[i] = x;
+            r[p] = (1.0 - 0.5 * friction * dt) * r[p] + f[p] * 0.5 * inv_mq * dt;
+            sum += x * sc[i];
+        }
+        rate[i] = r[p];
+    }
+    const double total = reduce(sum, plus);
+    if (t == 0) {
+        *error = err;
+        if (!on) *stop = 1;
+        if (on && more) *qsum = total;
+    }
+}
+
+__global__ void k_clear_stop(int *__restrict__ stop)
+{
+    if (threadIdx.x == 0) *stop = 0;
 }
 
 // ---- host side ----------------------------------------------------------------
@@ -1049,8 +1119,13 @@ void structure_factors(System &S, EwaldState &E, bool placed = false)
         return;
     }
     if (nk == 0) return;
+    // Atom chunks: of at least 256 atoms while that gives 2048 blocks, else down
+    // to 32 until there is a block for every compute unit.  Each chunk costs a
+    // pass over its partial S(k): 768 ions: 80 us in
+    // 256-atom chunks (a few blocks), 18 in 32 (and 8 us for the sum, not 5).
     int stiles = div_up(E.nwaves, EB / 64);
-    int nchunk = std::max(1, std::min(div_up(n, EB), div_up(2048, stiles)));
+    int nchunk = std::max(1, std::max(std::min(div_up(n, EB), div_up(2048, stiles)),
+                                      std::min(div_up(n, 32), div_up(256, stiles))));
     int chunk = div_up(n, nchunk);
     nchunk = div_up(n, chunk);
     E.skpart.ensure((size_t)nchunk * nk);
@@ -1072,14 +1147,14 @@ void structure_factors(System &S, EwaldState &E, bool placed = false)
 // Where the kernels leave what the host wants to see (sys_mail): read after
 // one wait for the stream.
 enum { M_REAL = MAIL_FREE, M_CHARGE = M_REAL + 8, M_DIPOLE = M_CHARGE + 2, M_HASH = M_DIPOLE + 3,
-       M_RECIP, M_STRESS, M_ERROR = M_STRESS + 6, M_END };
+       M_RECIP, M_STRESS, M_ERROR = M_STRESS + 6, M_END = M_ERROR + 2 };
 static_assert(M_END <= MAIL_WORDS, "mail words");
 
 // the virial block partials of a per-atom pass, summed
 void sum_stress(System &S, EwaldState &E, int blocks, double *stress6)
 {
     double *mail = sys_mail(S) + M_STRESS;
-    k_sum_partials<<<1, EB, 0, S.stream>>>(blocks, 8, 6, E.part.p, mail);
+    k_sum_partials<<<6, EB, 0, S.stream>>>(blocks, 8, E.part.p, mail);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(S.stream));
     for (int c = 0; c < 6; ++c) stress6[c] = mail[c];
@@ -1163,13 +1238,13 @@ void post_charge_sums(System &S, EwaldState &E)
     int nb = div_up(S.n, EB);
     E.part.ensure((size_t)nb * 8);
     k_charge_sums<<<nb, EB, 0, S.stream>>>(S.n, S.q.p, E.scaler.p, E.part.p);
-    k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 2, E.part.p, sys_mail(S) + M_CHARGE);
+    k_sum_partials<<<2, EB, 0, S.stream>>>(nb, 8, E.part.p, sys_mail(S) + M_CHARGE);
     HIP_TRY(hipGetLastError());
 }
 
 // real-space + singlet pass; posts the energy (mode 1) and stress (mode 2) sums
-void real_pass(System &S, const EwaldParams &P, EwaldState &E, int mode, double bg_chi,
-               const double *bg_dev = nullptr, bool with_self = true)
+// (mode 3 takes the background's charge sum from E.red)
+void real_pass(System &S, const EwaldParams &P, EwaldState &E, int mode, bool with_self = true)
 {
     const int n = S.n;
     Consts c = consts_of(P, E.volume);
@@ -1182,8 +1257,9 @@ void real_pass(System &S, const EwaldParams &P, EwaldState &E, int mode, double 
     auto launch = [&](auto kern) {
         kern<<<nb, EB, 0, S.stream>>>(n, S.geom, S.pos.p, S.q.p, E.scaler.p, S.nbr.p, S.nimg.p,
                                       S.ncnt.p, S.dmodel.p, P.on, P.rc, c.inv_eps_4pi,
-                                      c.inv_sig_sqrt2, c.inv_sig_sqrt2pi, c.inv_sig_sq2, bg_chi,
-                                      bg_dev, with_self ? 1 : 0, E.chi.p, S.frc.p, E.part.p);
+                                      c.inv_sig_sqrt2, c.inv_sig_sqrt2pi, c.inv_sig_sq2,
+                                      c.inv_eps_2v, P.sigma, E.red.p, with_self ? 1 : 0, E.chi.p,
+                                      S.frc.p, E.part.p);
     };
     auto lanes_of = [&](auto m) {
         constexpr int MODE = decltype(m)::value;
@@ -1201,29 +1277,25 @@ void real_pass(System &S, const EwaldParams &P, EwaldState &E, int mode, double 
     HIP_TRY(hipGetLastError());
     S.timer.end("ewald_real", S.stream, ev);
     if (mode != 3) {
-        k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 7, E.part.p, sys_mail(S) + M_REAL);
+        k_sum_partials<<<7, EB, 0, S.stream>>>(nb, 8, E.part.p, sys_mail(S) + M_REAL);
         HIP_TRY(hipGetLastError());
     }
 }
 
 // Electronegativities into E.chi without a host round trip: the charge sum
-// and the background term stay on the device.
-// placed: the atoms have not moved since the previous evaluation.
-void chi_eval(System &S, const EwaldParams &P, EwaldState &E, bool placed = false)
+// stays on the device (E.red).  placed: the atoms have not moved since the
+// previous evaluation; summed: E.red holds the charge sum already.
+void chi_eval(System &S, const EwaldParams &P, EwaldState &E, bool placed = false,
+              bool summed = false)
 {
-    const double *bg_dev = nullptr;
-    if (P.on) {
+    if (P.on && !summed) {
         int nb = div_up(S.n, EB);
         E.part.ensure((size_t)nb * 8);
         k_charge_sums<<<nb, EB, 0, S.stream>>>(S.n, S.q.p, E.scaler.p, E.part.p);
-        k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 2, E.part.p, E.red.p);
-        Consts c = consts_of(P, E.volume);
-        // - s inv_eps_2v (-sigma^2 Q)  (Potentials.f90:2166-2167)
-        k_background<<<1, 64, 0, S.stream>>>(E.red.p, E.red.p + 12, c.inv_eps_2v, P.sigma);
+        k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, E.part.p, E.red.p);
         HIP_TRY(hipGetLastError());
-        bg_dev = E.red.p + 12;
     }
-    real_pass(S, P, E, 3, 0.0, bg_dev);
+    real_pass(S, P, E, 3);
     if (P.on && has_recip(E)) {
         // the relaxation changes the charges every step: no fingerprint
         structure_factors(S, E, placed);
@@ -1257,6 +1329,13 @@ void ewald_release(EwaldState &E)
     E.kpk.release();
     E.hpart.release();
     mesh_release(E.mesh);
+    E.dchi.release();
+    E.mx.release();
+    E.stop.release();
+    for (hipEvent_t &e : E.seen) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
     E.sk_valid = false;
 }
 
@@ -1268,13 +1347,13 @@ double energy_terms(System &S, const EwaldParams &P, EwaldState &E, bool with_se
 {
     prepare(S, P, E);
     if (!P.on) unit_scaler(S, E);
-    real_pass(S, P, E, 1, 0.0, nullptr, with_self);
+    real_pass(S, P, E, 1, with_self);
     if (P.on) {
         post_charge_sums(S, E);
         if (with_dipole) {
             int nb = div_up(S.n, EB);
             k_dipole_sums<<<nb, EB, 0, S.stream>>>(S.n, S.pos.p, S.q.p, E.scaler.p, E.part.p);
-            k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 3, E.part.p, sys_mail(S) + M_DIPOLE);
+            k_sum_partials<<<3, EB, 0, S.stream>>>(nb, 8, E.part.p, sys_mail(S) + M_DIPOLE);
         }
         if (has_recip(E)) post_hash(S, E);
     }
@@ -1295,12 +1374,12 @@ double energy_terms(System &S, const EwaldParams &P, EwaldState &E, bool with_se
             current_structure_factors(S, E);
             double *out = sys_mail(S) + M_RECIP;
             if (E.mesh_on) {
-                k_sum_partials<<<1, EB, 0, S.stream>>>(E.mesh.nepart, 1, 1, E.mesh.epart.p, out);
+                k_sum_partials<<<1, EB, 0, S.stream>>>(E.mesh.nepart, 1, E.mesh.epart.p, out);
             } else {
                 int nb = div_up(E.nk, EB);
                 E.part.ensure((size_t)nb);
                 k_recip_energy<<<nb, EB, 0, S.stream>>>(E.nk, E.kvec.p, E.sk.p, E.part.p);
-                k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 1, 1, E.part.p, out);
+                k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 1, E.part.p, out);
             }
             HIP_TRY(hipGetLastError());
             HIP_TRY(hipStreamSynchronize(S.stream));
@@ -1325,7 +1404,7 @@ double ewald_standalone_energy(System &S, const EwaldParams &P, EwaldState &E)
 void ewald_add_forces(System &S, const EwaldParams &P, EwaldState &E, double *stress)
 {
     prepare(S, P, E);
-    real_pass(S, P, E, 2, 0.0);
+    real_pass(S, P, E, 2);
     const bool recip = P.on && has_recip(E);
     if (recip) post_hash(S, E);
     HIP_TRY(hipStreamSynchronize(S.stream));
@@ -1353,49 +1432,74 @@ void ewald_relax(System &S, const EwaldParams &P, EwaldState &E, double *rates, 
     const int n = S.n;
     prepare(S, P, E);
     if (!P.on) unit_scaler(S, E);
-    DBuf<double> dchi, mx;
-    dchi.ensure(n);
-    int nb = div_up(n, EB);
-    mx.ensure(nb);
+    const int nb = div_up(n, EB);
     const double dt2 = dt * dt, inv_mq = 1.0 / inertia;
     const double future = 1.0 / (1.0 + 0.5 * friction * dt);
-    auto dchi_of_q = [&](int update) {
-        chi_eval(S, P, E, update != 0);
-        E.part.ensure((size_t)nb * 8);
-        k_sum_chi<<<nb, EB, 0, S.stream>>>(n, E.chi.p, E.part.p);
-        k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, 1, E.part.p, E.red.p);
-        k_relax_finish<<<nb, EB, 0, S.stream>>>(n, E.chi.p, E.red.p, dchi.p, rates, update, future,
-                                                0.5 * inv_mq * dt, mx.p);
-        double *mail = sys_mail(S) + M_ERROR;
-        k_max_partials<<<1, EB, 0, S.stream>>>(nb, mx.p, mail);
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipStreamSynchronize(S.stream));
-        return *mail;
-    };
-    double err = dchi_of_q(0);
+    double *mail = sys_mail(S) + M_ERROR;
     int step = 0;
+    double err = 0.0;
     // the reference tests the signed max(dchi) (relaxation.py:449); a
     // non-finite value means the dynamics ran away (time step too long for
     // the stiffest charge mode, or an indefinite charge Hessian)
     auto check = [&]() {
-        if (!std::isfinite(err)) {
-            dchi.release();
-            mx.release();
-            throw PysicError{PYSIC_ERANGE, "charge relaxation diverged at step " +
-                                               std::to_string(step) +
-                                               " (reduce the time step or raise the inertia)"};
-        }
+        PYSIC_REQUIRE(std::isfinite(err), PYSIC_ERANGE,
+                      "charge relaxation diverged at step " + std::to_string(step) +
+                          " (reduce the time step or raise the inertia)");
     };
+    if (n <= RELAX_ONE) {
+        // Evaluation k (k = 0: of the starting charges) is queued before the
+        // error of k - 1 is known, from the third on: a relaxation of a step
+        // or two would mostly compute the one that is not needed.
+        E.stop.ensure(1);
+        for (hipEvent_t &e : E.seen)
+            if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        k_clear_stop<<<1, 64, 0, S.stream>>>(E.stop.p);
+        auto queue = [&](int k) {
+            chi_eval(S, P, E, k > 0, k > 0);
+            k_relax_tail<<<1, 1024, 0, S.stream>>>(n, E.chi.p, S.q.p, rates, E.scaler.p, k == 0,
+                                                   k < n_steps, dt, inv_mq, friction, future,
+                                                   tolerance, E.stop.p, E.red.p, mail + (k & 1));
+            HIP_TRY(hipGetLastError());
+            HIP_TRY(hipEventRecord(E.seen[k & 1], S.stream));
+        };
+        queue(0);
+        for (int queued = 0;; ++step) {
+            if (queued == step && step < n_steps && step >= 2) queue(++queued);
+            HIP_TRY(hipEventSynchronize(E.seen[step & 1]));
+            err = mail[step & 1];
+            check();
+            if (step == 0) err = 2.0 * tolerance;
+            if (step >= n_steps || !(err > tolerance)) break;
+            if (queued == step) queue(++queued);
+        }
+        *steps = step;
+        *error = err;
+        return;
+    }
+    E.dchi.ensure(n);
+    E.mx.ensure(nb);
+    auto dchi_of_q = [&](int update) {
+        chi_eval(S, P, E, update != 0);
+        E.part.ensure((size_t)nb * 8);
+        k_sum_chi<<<nb, EB, 0, S.stream>>>(n, E.chi.p, E.part.p);
+        k_sum_partials<<<1, EB, 0, S.stream>>>(nb, 8, E.part.p, E.red.p);
+        k_relax_finish<<<nb, EB, 0, S.stream>>>(n, E.chi.p, E.red.p, E.dchi.p, rates, update,
+                                                future, 0.5 * inv_mq * dt, E.mx.p);
+        k_max_partials<<<1, EB, 0, S.stream>>>(nb, E.mx.p, mail);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(S.stream));
+        return *mail;
+    };
+    err = dchi_of_q(0);
     check();
     err = 2.0 * tolerance;
     while (err > tolerance && step < n_steps) {
-        k_relax_update<<<nb, EB, 0, S.stream>>>(n, S.q.p, rates, dchi.p, dt, dt2, inv_mq, friction);
+        k_relax_update<<<nb, EB, 0, S.stream>>>(n, S.q.p, rates, E.dchi.p, dt, dt2, inv_mq,
+                                                friction);
         err = dchi_of_q(1);
         ++step;
         check();
     }
     *steps = step;
     *error = err;
-    dchi.release();
-    mx.release();
 }
