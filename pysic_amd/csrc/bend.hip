@@ -325,34 +325,44 @@ int bend_blocks(const System &S)
     return S.pmodel.nbend > 0 ? div_up(S.n * BG_LANES * BG_PARTS, BB) : 0;
 }
 
-void bend_eval(System &S, int mode, int blk0, double half_dt, int kick)
+// up to the gather: short lists, each vertex's angles, their partials
+void bend_sites(System &S, int mode, int blk0, hipStream_t stream)
 {
-    if (S.pmodel.nbend == 0) return;
     const int n = S.n, nb = div_up(n, BB), na = bend_blocks(S);
     const size_t cap = (size_t)S.cap * n;
     S.bsj.ensure(cap);
     S.bsimg.ensure(cap);
     S.bscnt.ensure(n);
     S.bG.ensure(cap);
-    hipEvent_t ev{};
-    S.timer.begin("bend", S.stream, &ev);
     with_geo(S, [&](auto geo) {
         using Geo = decltype(geo);
-        k_bend_list<Geo><<<nb, BB, 0, S.stream>>>(n, geo, S.pos.p, S.nbr.p, S.nimg.p, S.ncnt.p,
-                                                  S.dpmodel.p, S.bsj.p, S.bsimg.p, S.bscnt.p);
+        k_bend_list<Geo><<<nb, BB, 0, stream>>>(n, geo, S.pos.p, S.nbr.p, S.nimg.p, S.ncnt.p,
+                                                S.dpmodel.p, S.bsj.p, S.bsimg.p, S.bscnt.p);
         auto go = [&](auto kern) {
-            kern<<<na, BB, 0, S.stream>>>(n, geo, S.pos.p, S.id.p, S.dpmodel.p, S.bsj.p,
-                                          S.bsimg.p, S.bscnt.p, S.bG.p, S.gpartial.p, blk0);
+            kern<<<na, BB, 0, stream>>>(n, geo, S.pos.p, S.id.p, S.dpmodel.p, S.bsj.p, S.bsimg.p,
+                                        S.bscnt.p, S.bG.p, S.gpartial.p, blk0);
         };
         if (mode == PAIR_ENERGY) go(k_bend_angles<Geo, PAIR_ENERGY, BG_LANES, BG_PARTS>);
         else if (mode == PAIR_FORCES) go(k_bend_angles<Geo, PAIR_FORCES, BG_LANES, BG_PARTS>);
         else go(k_bend_angles<Geo, PAIR_FORCES_ONLY, BG_LANES, BG_PARTS>);
     });
     HIP_TRY(hipGetLastError());
-    if (mode != PAIR_ENERGY) {
-        k_bend_gather<BG_GATHER_LANES><<<div_up(n * BG_GATHER_LANES, BB), BB, 0, S.stream>>>(
-            n, S.bsj.p, S.bsimg.p, S.bscnt.p, S.bG.p, S.frc.p, S.mom.p, half_dt, kick);
-        HIP_TRY(hipGetLastError());
-    }
+}
+
+void bend_gather(System &S, int mode, double half_dt, int kick)
+{
+    if (mode == PAIR_ENERGY) return;
+    k_bend_gather<BG_GATHER_LANES><<<div_up(S.n * BG_GATHER_LANES, BB), BB, 0, S.stream>>>(
+        S.n, S.bsj.p, S.bsimg.p, S.bscnt.p, S.bG.p, S.frc.p, S.mom.p, half_dt, kick);
+    HIP_TRY(hipGetLastError());
+}
+
+void bend_eval(System &S, int mode, int blk0, double half_dt, int kick)
+{
+    if (S.pmodel.nbend == 0) return;
+    hipEvent_t ev{};
+    S.timer.begin("bend", S.stream, &ev);
+    bend_sites(S, mode, blk0, S.stream);
+    bend_gather(S, mode, half_dt, kick);
     S.timer.end("bend", S.stream, ev);
 }

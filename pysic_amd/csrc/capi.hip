@@ -136,8 +136,32 @@ void System::release_all()
     tables.release();
     cells.release();
     link.release();
+    for (int k = 0; k < 2; ++k) {
+        if (side[k]) (void)hipStreamDestroy(side[k]);
+        if (forked[k]) (void)hipEventDestroy(forked[k]);
+        if (joined[k]) (void)hipEventDestroy(joined[k]);
+        side[k] = nullptr;
+        forked[k] = joined[k] = nullptr;
+    }
     order_valid = false;
     bins_clean = false;
+}
+
+void sys_fork(System &S, int k, bool on)
+{
+    if (!on) return;
+    if (!S.side[k]) HIP_TRY(hipStreamCreate(&S.side[k]));
+    for (hipEvent_t *e : {&S.forked[k], &S.joined[k]})
+        if (!*e) HIP_TRY(hipEventCreateWithFlags(e, hipEventDisableTiming));
+    HIP_TRY(hipEventRecord(S.forked[k], S.stream));
+    HIP_TRY(hipStreamWaitEvent(S.side[k], S.forked[k], 0));
+}
+
+void sys_join(System &S, int k, bool on)
+{
+    if (!on) return;
+    HIP_TRY(hipEventRecord(S.joined[k], S.side[k]));
+    HIP_TRY(hipStreamWaitEvent(S.stream, S.joined[k], 0));
 }
 
 // ---------------------------------------------------------------------------

@@ -29,6 +29,8 @@
 // evaluated only when the model has a step factor.
 #include "system.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int PB = 256;
@@ -414,8 +416,18 @@ __device__ __forceinline__ bool visit(const PairLds<0> &L, int si, int sj, doubl
 // (24,576 atoms of COMB SiO2: 381 us with 1 lane, 209 with 2, 144 with 4,
 // 140 with 8).  Above that, one thread per atom already fills the chip, and
 // each extra block would stage the whole model into LDS once more.
+// The LJ kinds take 8, 4 or 2 lanes up to LJ_LANES_ATOMS / lanes atoms, 4
+// neighbors in flight each, for the same reason: 13,500 argon atoms are 211
+// waves on 1024 SIMDs with a thread each (33.9 us a launch; 11.3 with 8 lanes).
 constexpr int PAIR_LANES_SMALL = 8;
 constexpr int PAIR_LANES_MAX_ATOMS = 1 << 18;
+constexpr int LJ_LANES_ATOMS = 1 << 18;
+int lj_lanes(int n)
+{
+    for (int g = 8; g > 1; g >>= 1)
+        if (n <= LJ_LANES_ATOMS / g) return g;
+    return 1;
+}
 
 template <class Geo, int MODE, int KIND, int G>
 __global__ __launch_bounds__(PB) void k_pairs(int n, Geo geo, const double4 *__restrict__ pos,
@@ -432,7 +444,7 @@ __global__ __launch_bounds__(PB) void k_pairs(int n, Geo geo, const double4 *__r
 {
     constexpr bool FORCE = MODE != PAIR_ENERGY;
     constexpr bool VIR = MODE == PAIR_FORCES;
-    constexpr int NBU = KIND == 0 ? 2 : PYSIC_PAIR_NBU;
+    constexpr int NBU = KIND == 0 ? 2 : G == 1 ? PYSIC_PAIR_NBU : 4;
     __shared__ PairLds<KIND> lds;
     __shared__ double red[7][PB];
     stage(lds, PM);
@@ -1138,8 +1150,8 @@ void pr_eval(System &S, int mode, bool accumulate, double half_dt, int kick)
     PYSIC_REQUIRE(S.dpmodel.p && S.tables.p, PYSIC_ESTATE, "pair model not compiled");
     PYSIC_REQUIRE(S.n > 0, PYSIC_ESTATE, "no atoms");
     const int kind = S.pmodel.lj_only ? (S.model.nspecies == 1 ? 2 : 1) : 0;
-    const bool lanes = kind == 0 && S.n <= PAIR_LANES_MAX_ATOMS;
-    const int nb = div_up(S.n * (lanes ? PAIR_LANES_SMALL : 1), PB);
+    const int lanes = kind != 0 ? lj_lanes(S.n) : S.n <= PAIR_LANES_MAX_ATOMS ? PAIR_LANES_SMALL : 1;
+    const int nb = div_up(S.n * lanes, PB);
     // bond_bend angles, then the bond-order-scaled pairs, add their
     // partials after the pair blocks and their forces after the pair forces
     // (the last of them the half-kick, if asked)
@@ -1148,20 +1160,49 @@ void pr_eval(System &S, int mode, bool accumulate, double half_dt, int kick)
     S.gpartial.ensure((size_t)(nb + bb + ob) * 8);
     S.gtotals.ensure(8);
     S.gpartial_blocks = nb + bb + ob;
+    // The angles and the bond-order passes up to their gathers need nothing of
+    // the pair kernel: on streams of their own they share the chip with it,
+    // which one of them alone leaves half idle at these sizes.  Serially while
+    // the kernels are timed, and for systems that fill the chip.  20 steps of
+    // 24,576 atoms of COMB SiO2 and their state: 7.97 -> 7.30 ms.
+    const bool side = (bb || ob) && !S.timer.on && S.n <= PAIR_LANES_MAX_ATOMS;
+    if (side) {
+        sys_fork(S, 0, bb > 0);
+        sys_fork(S, 1, ob > 0);
+        if (ob) bop_sites(S, mode, nb + bb, S.side[1]);   // the longest chain first
+        if (bb) bend_sites(S, mode, nb, S.side[0]);
+    }
     hipEvent_t ev{};
     const char *name = mode == PAIR_ENERGY ? "pair_energy" : "pair_forces";
     S.timer.begin(name, S.stream, &ev);
     const int pkick = (bb || ob) ? 0 : kick;
     with_geo(S, [&](auto geo) {
         using Geo = decltype(geo);
-        if (kind == 2) launch<Geo, 2, 1>(S, geo, mode, accumulate, half_dt, pkick);
-        else if (kind == 1) launch<Geo, 1, 1>(S, geo, mode, accumulate, half_dt, pkick);
-        else if (lanes) launch<Geo, 0, PAIR_LANES_SMALL>(S, geo, mode, accumulate, half_dt, pkick);
+        auto lj = [&](auto k) {
+            constexpr int KIND = decltype(k)::value;
+            switch (lanes) {
+            case 8: launch<Geo, KIND, 8>(S, geo, mode, accumulate, half_dt, pkick); break;
+            case 4: launch<Geo, KIND, 4>(S, geo, mode, accumulate, half_dt, pkick); break;
+            case 2: launch<Geo, KIND, 2>(S, geo, mode, accumulate, half_dt, pkick); break;
+            default: launch<Geo, KIND, 1>(S, geo, mode, accumulate, half_dt, pkick); break;
+            }
+        };
+        if (kind == 2) lj(std::integral_constant<int, 2>{});
+        else if (kind == 1) lj(std::integral_constant<int, 1>{});
+        else if (lanes > 1)
+            launch<Geo, 0, PAIR_LANES_SMALL>(S, geo, mode, accumulate, half_dt, pkick);
         else launch<Geo, 0, 1>(S, geo, mode, accumulate, half_dt, pkick);
     });
     S.timer.end(name, S.stream, ev);
-    if (bb) bend_eval(S, mode, nb, half_dt, ob ? 0 : kick);
-    if (ob) bop_eval(S, mode, nb + bb, half_dt, kick);
+    if (side) {
+        sys_join(S, 0, bb > 0);
+        sys_join(S, 1, ob > 0);
+        if (bb) bend_gather(S, mode, half_dt, ob ? 0 : kick);
+        if (ob) bop_gather(S, mode, half_dt, kick);
+    } else {
+        if (bb) bend_eval(S, mode, nb, half_dt, ob ? 0 : kick);
+        if (ob) bop_eval(S, mode, nb + bb, half_dt, kick);
+    }
     if (mode != PAIR_FORCES_ONLY) {
         k_pair_totals<<<7, PB, 0, S.stream>>>(nb + bb + ob, S.gpartial.p, S.gtotals.p);
         HIP_TRY(hipGetLastError());
@@ -1194,7 +1235,7 @@ int bop_blocks(const System &S, int mode)
     return mode == PAIR_ENERGY ? nb : 2 * nb;
 }
 
-static void bop_prepare(System &S)
+static void bop_prepare(System &S, hipStream_t stream)
 {
     const int n = S.n;
     const size_t cap = (size_t)S.cap * n;
@@ -1205,30 +1246,28 @@ static void bop_prepare(System &S)
     S.oW.ensure(cap);
     S.oown.ensure(n);
     with_geo(S, [&](auto geo) {
-        k_bop_list<decltype(geo)><<<div_up(n, PB), PB, 0, S.stream>>>(
+        k_bop_list<decltype(geo)><<<div_up(n, PB), PB, 0, stream>>>(
             n, geo, S.pos.p, S.nbr.p, S.nimg.p, S.ncnt.p, S.bmodel.radius, S.osj.p, S.osimg.p,
             S.oscnt.p);
     });
     HIP_TRY(hipGetLastError());
 }
 
-void bop_eval(System &S, int mode, int blk0, double half_dt, int kick)
+// up to the gather: per-slot derivatives and the energy or virial partials
+void bop_sites(System &S, int mode, int blk0, hipStream_t stream)
 {
-    if (!S.bmodel.on) return;
     const int n = S.n, nb = div_up(n * BOP_LANES, PB);
-    hipEvent_t ev{};
-    S.timer.begin("bond_order_pairs", S.stream, &ev);
-    bop_prepare(S);
+    bop_prepare(S, stream);
     with_geo(S, [&](auto geo) {
         using Geo = decltype(geo);
         auto one = [&](auto kern) {
-            kern<<<nb, PB, 0, S.stream>>>(n, geo, S.pos.p, S.id.p, S.dbmodel.p, S.dpmodel.p,
-                                          S.tables.p, S.q.p, S.osj.p, S.osimg.p, S.oscnt.p,
-                                          S.oD.p, S.oW.p, S.oown.p, S.gpartial.p, blk0);
+            kern<<<nb, PB, 0, stream>>>(n, geo, S.pos.p, S.id.p, S.dbmodel.p, S.dpmodel.p,
+                                        S.tables.p, S.q.p, S.osj.p, S.osimg.p, S.oscnt.p, S.oD.p,
+                                        S.oW.p, S.oown.p, S.gpartial.p, blk0);
         };
         auto two = [&](auto kern) {
-            kern<<<nb, PB, 0, S.stream>>>(n, geo, S.pos.p, S.dbmodel.p, S.osj.p, S.osimg.p,
-                                          S.oscnt.p, S.oD.p, S.oW.p, S.gpartial.p, blk0 + nb);
+            kern<<<nb, PB, 0, stream>>>(n, geo, S.pos.p, S.dbmodel.p, S.osj.p, S.osimg.p,
+                                        S.oscnt.p, S.oD.p, S.oW.p, S.gpartial.p, blk0 + nb);
         };
         if (mode == PAIR_ENERGY) {
             one(k_bop_pairs<Geo, PAIR_ENERGY, BOP_LANES>);
@@ -1241,12 +1280,24 @@ void bop_eval(System &S, int mode, int blk0, double half_dt, int kick)
         }
     });
     HIP_TRY(hipGetLastError());
-    if (mode != PAIR_ENERGY) {
-        k_bop_gather<BOP_LANES, false><<<div_up(n * BOP_LANES, PB), PB, 0, S.stream>>>(
-            n, S.osj.p, S.osimg.p, S.oscnt.p, S.oD.p, S.oown.p, S.frc.p, S.mom.p, half_dt, kick,
-            nullptr);
-        HIP_TRY(hipGetLastError());
-    }
+}
+
+void bop_gather(System &S, int mode, double half_dt, int kick)
+{
+    if (mode == PAIR_ENERGY) return;
+    k_bop_gather<BOP_LANES, false><<<div_up(S.n * BOP_LANES, PB), PB, 0, S.stream>>>(
+        S.n, S.osj.p, S.osimg.p, S.oscnt.p, S.oD.p, S.oown.p, S.frc.p, S.mom.p, half_dt, kick,
+        nullptr);
+    HIP_TRY(hipGetLastError());
+}
+
+void bop_eval(System &S, int mode, int blk0, double half_dt, int kick)
+{
+    if (!S.bmodel.on) return;
+    hipEvent_t ev{};
+    S.timer.begin("bond_order_pairs", S.stream, &ev);
+    bop_sites(S, mode, blk0, S.stream);
+    bop_gather(S, mode, half_dt, kick);
     S.timer.end("bond_order_pairs", S.stream, ev);
 }
 
@@ -1254,7 +1305,7 @@ void bop_chi(System &S, double *chi)
 {
     if (!S.bmodel.on) return;
     const int n = S.n, nb = div_up(n * BOP_LANES, PB);
-    bop_prepare(S);
+    bop_prepare(S, S.stream);
     with_geo(S, [&](auto geo) {
         k_bop_pairs<decltype(geo), BOP_CHI, BOP_LANES><<<nb, PB, 0, S.stream>>>(
             n, geo, S.pos.p, S.id.p, S.dbmodel.p, S.dpmodel.p, S.tables.p, S.q.p, S.osj.p,

@@ -63,6 +63,10 @@ constexpr int MAIL_WORDS = 64, MAIL_FREE = 16;
 
 struct System {
     hipStream_t stream = nullptr;
+    // streams for work beside the main stream's, always joined back into it
+    // within the call that forked them (graph capture follows the events)
+    hipStream_t side[2] = {nullptr, nullptr};
+    hipEvent_t forked[2] = {nullptr, nullptr}, joined[2] = {nullptr, nullptr};
     int device = 0;
     HostLink link;
     DBuf<int> inv;              // slot of each original index (transfers)
@@ -214,10 +218,16 @@ void pr_chi(System &S, double *chi);
 // bond_bend angles: energy / virial partials into gpartial blocks
 // [blk0, blk0 + blocks), forces added into frc (then p += half_dt F if kick)
 void bend_eval(System &S, int mode, int blk0, double half_dt, int kick);
+// the same in two parts: everything up to the gather on any stream, the gather
+// (forces and kick) on the main one
+void bend_sites(System &S, int mode, int blk0, hipStream_t stream);
+void bend_gather(System &S, int mode, double half_dt, int kick);
 int bend_blocks(const System &S);
 // bond-order-scaled pair potentials: the same contract as bend_eval, and
 // their share of chi
 void bop_eval(System &S, int mode, int blk0, double half_dt, int kick);
+void bop_sites(System &S, int mode, int blk0, hipStream_t stream);
+void bop_gather(System &S, int mode, double half_dt, int kick);
 int bop_blocks(const System &S, int mode);
 void bop_chi(System &S, double *chi);
 
@@ -240,6 +250,11 @@ struct Report {
 double *sys_mail(System &S);
 void sys_post_report(System &S, bool tersoff, bool general);
 Report sys_read_report(System &S);
+
+// side stream k waits for what the main stream holds now; the main stream
+// waits for what side stream k holds now (nothing if !on)
+void sys_fork(System &S, int k, bool on);
+void sys_join(System &S, int k, bool on);
 
 // md.hip
 void md_drift(System &S, double dt, double half_dt);  // p += dt/2 F ; r += dt p/m (no rebuild)
