@@ -1721,7 +1721,7 @@ void mlp_upload_samples(MlpState &M, long count, const int *samples)
 }
 
 // descriptors of h's system into M.sfeat / M.sspec (current order), on h's stream
-void mlp_system_descriptors(MlpState &M, pysic_ctx *h)
+void mlp_system_descriptors(MlpState &M, pysic_ctx *h, bool keep_near = false)
 {
     PYSIC_REQUIRE(M.configured, PYSIC_ESTATE, "network not configured");
     PYSIC_REQUIRE(h->device == M.device, PYSIC_EINVAL, "network and system live on different GPUs");
@@ -1734,7 +1734,7 @@ void mlp_system_descriptors(MlpState &M, pysic_ctx *h)
     System &S = h->S;
     M.sfeat.ensure((size_t)S.n * MLP_F);
     M.sspec.ensure(S.n);
-    mlp_descriptors(S, M, S.stream);
+    mlp_descriptors(S, M, keep_near, S.stream);
 }
 
 }  // namespace
@@ -1954,7 +1954,7 @@ int pysic_mlp_warm_start(pysic_mlp *m, pysic_ctx *h, int n, int n_stages, double
     PYSIC_REQUIRE(n_stages >= 0 && n_stages <= M.corr_stages, PYSIC_EINVAL,
                   "warm_start: more stages asked for than the corrector holds");
     try {
-        mlp_system_descriptors(M, h);
+        mlp_system_descriptors(M, h, n_stages > 0);
     } catch (const PysicError &e) {
         h->err = e.msg;
         throw;
@@ -1968,7 +1968,7 @@ int pysic_mlp_warm_start(pysic_mlp *m, pysic_ctx *h, int n, int n_stages, double
     h->forces_valid = false;
     double *prev = M.cprev.p, *next = M.cnext.p;
     for (int k = 0; k < n_stages; ++k) {
-        DBuf<double> &chi = ewald_eem_chi(S, h->ewald, h->ew);
+        DBuf<double> &chi = ewald_eem_chi(S, h->ewald, h->ew, k > 0);
         mlp_corrector_stage(S, M, M.ccoef.p + (size_t)k * CORR_NC, chi.p, prev, next, S.stream);
         std::swap(prev, next);
     }

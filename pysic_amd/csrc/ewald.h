@@ -97,8 +97,8 @@ double ewald_standalone_energy(System &S, const EwaldParams &P, EwaldState &E);
 // Adds Ewald forces into S.frc; stress[6] receives the Ewald part.
 void ewald_add_forces(System &S, const EwaldParams &P, EwaldState &E, double *stress);
 // Electronegativities (charge_self + Ewald) into E.chi, sorted order, queued
-// on the stream.
-DBuf<double> &ewald_eem_chi(System &S, const EwaldParams &P, EwaldState &E);
+// on the stream.  placed: the atoms have not moved since the previous call.
+DBuf<double> &ewald_eem_chi(System &S, const EwaldParams &P, EwaldState &E, bool placed = false);
 // Damped charge dynamics on device; S.q and rates (sorted order) updated.
 void ewald_relax(System &S, const EwaldParams &P, EwaldState &E, double *rates, int n_steps,
                  double dt, double inertia, double friction, double tolerance, int *steps,

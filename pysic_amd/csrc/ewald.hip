@@ -1417,11 +1417,11 @@ void ewald_add_forces(System &S, const EwaldParams &P, EwaldState &E, double *st
     }
 }
 
-DBuf<double> &ewald_eem_chi(System &S, const EwaldParams &P, EwaldState &E)
+DBuf<double> &ewald_eem_chi(System &S, const EwaldParams &P, EwaldState &E, bool placed)
 {
     prepare(S, P, E);
     if (!P.on) unit_scaler(S, E);
-    chi_eval(S, P, E);
+    chi_eval(S, P, E, placed);
     return E.chi;
 }
 

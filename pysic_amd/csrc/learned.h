@@ -95,12 +95,15 @@ struct MlpState {
     int corr_stages = 0;
     DBuf<double> ccoef;          // [corr_stages][CORR_NC]
     DBuf<double> cprev, cnext;   // d of the previous stage, current order (ping-pong)
+    DBuf<int2> near;             // [n][128] neighbors within rc: j << 2 | species, FP32 r
+    DBuf<int> nnear;             // their number, which may be larger
     DBuf<double> cfeat;          // [n][CORR_NC] corrector features, current order
     void release_all();
 };
 
 // mlp.hip launchers (all on m.stream unless a stream is given)
-void mlp_descriptors(System &S, const MlpState &m, hipStream_t st);      // -> m.sfeat, m.sspec
+// -> m.sfeat, m.sspec; keep_near: and m.near, m.nnear for mlp_corrector_stage
+void mlp_descriptors(System &S, MlpState &m, bool keep_near, hipStream_t st);
 void mlp_pack(MlpState &m);                                             // P -> W (BF16)
 void mlp_forward(MlpState &m, int count, const int *order, const float *feat, const int *spec,
                  float *y, hipStream_t st);
@@ -114,6 +117,6 @@ void mlp_neutral_charges(System &S, MlpState &m, const float *y, double *prev, h
 // corrector features of chi and prev on S (current order) into m.cfeat
 void mlp_corrector_features(System &S, MlpState &m, const double *chi, const double *prev,
                             hipStream_t st);
-// one corrector stage: S.q += dq, next = dq
+// one corrector stage: S.q += dq, next = dq, over the neighbors of the last mlp_descriptors
 void mlp_corrector_stage(System &S, const MlpState &m, const double *coef, const double *chi,
                          const double *prev, double *next, hipStream_t st);

@@ -5,7 +5,7 @@
 // then runs unchanged to its tolerance.  The network and descriptors are
 // defined in learned.h.
 //
-//  * k_descriptors: one thread per atom over its full neighbor list
+//  * k_descriptors: eight lanes per atom over its full neighbor list
 //    (separations in FP64 as the force kernels form them, Gaussians in FP32);
 //  * k_forward: one thread per sample, all BF16 weights staged in LDS
 //    (12.4 KB, read as wave-wide broadcasts), products by v_dot2_f32_bf16 on
@@ -44,6 +44,76 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c)
                                            __builtin_bit_cast(bf16x2_t, b), c, false);
 }
 
+// The neighbors of one atom within rc, taken from its full list (radius 10.5 A
+// in the charge workloads, so one entry in five) by the L lanes of its group
+// and compacted into LDS, so that the Gaussians are evaluated by full lanes:
+// with the test inside the loop every wave ran them for nearly every entry.
+// body(h, j, r, species of j) is called by one lane for each hit h, in the
+// list's order, so the sums have one order; returns the number of hits.  The
+// group's lanes are consecutive threads of one wave; CAP hits are held at a
+// time.
+template <int L, int CAP, class Body>
+__device__ __forceinline__ int near_neighbors(int i, int n, int lane, const CellGeom &g,
+                                              const double4 *__restrict__ pos,
+                                              const int *__restrict__ nbr,
+                                              const int *__restrict__ nimg, int nf, double rc2,
+                                              int *s_j, float *s_r, Body &&body)
+{
+    constexpr int U = 4;   // entries in flight per lane
+    static_assert(CAP >= 2 * L * U, "room for a batch beside what is held");
+    const int shift = (threadIdx.x & 63) / L * L;
+    const unsigned long long mask = (1ull << L) - 1ull, below = (1ull << lane) - 1ull;
+    const double4 pi = i < n ? pos[i] : make_double4(0, 0, 0, 0);
+    int held = 0, done = 0;
+    auto flush = [&]() {
+        for (int h = lane; h < held; h += L) body(done + h, s_j[h] >> 2, s_r[h], s_j[h] & 3);
+        done += held;
+        held = 0;
+    };
+    int longest = nf;   // the ballots are the wave's: its groups run together
+#pragma unroll
+    for (int d = L; d < 64; d <<= 1) longest = max(longest, __shfl_xor(longest, d));
+    for (int t0 = 0; t0 < longest; t0 += L * U) {
+        int jv[U], iv[U];
+        double4 pv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int t = t0 + u * L + lane;
+            jv[u] = -1;
+            iv[u] = 0;
+            if (t < nf) {
+                jv[u] = nbr[(size_t)t * n + i];
+                iv[u] = nimg[(size_t)t * n + i];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) pv[u] = pos[max(jv[u], 0)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const double r2 = dot64(separation64(pi, pv[u], iv[u], g.v));
+            const bool hit = jv[u] >= 0 && r2 < rc2;
+            const unsigned long long b = (__ballot(hit) >> shift) & mask;
+            if (hit) {
+                const int at = held + __popcll(b & below);
+                s_j[at] = jv[u] << 2 | (int)pv[u].w;
+                s_r[at] = (float)sqrt(r2);
+            }
+            held += __popcll(b);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // one wave's LDS: in order
+        if (held > CAP - L * U) flush();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    flush();
+    return done;
+}
+
+// Descriptors, DESC_LANES lanes per atom.  24,576 atoms: 461 us with a thread
+// per atom and every entry tested inside the Gaussian loop, 85 us.  The hits
+// are kept for the corrector's stages if near is given (CORR_NEAR of them at
+// most; nnear holds the full number).
+constexpr int DESC_LANES = 8;
+constexpr int CORR_NEAR = 128;
 template <int NS>
 __global__ __launch_bounds__(256) void k_descriptors(int n, CellGeom g,
                                                      const double4 *__restrict__ pos,
@@ -51,29 +121,28 @@ __global__ __launch_bounds__(256) void k_descriptors(int n, CellGeom g,
                                                      const int *__restrict__ nimg,
                                                      const int *__restrict__ ncnt, DescParams dp,
                                                      float *__restrict__ feat,
-                                                     int *__restrict__ spec)
+                                                     int *__restrict__ spec,
+                                                     int2 *__restrict__ near,
+                                                     int *__restrict__ nnear)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    constexpr int L = DESC_LANES, CAP = 96;
+    __shared__ int s_j[256 / L][CAP];
+    __shared__ float s_r[256 / L][CAP];
+    const int i = (blockIdx.x * 256 + threadIdx.x) / L, lane = threadIdx.x % L;
+    const int a = threadIdx.x / L;
     float acc[NS][MLP_G];
 #pragma unroll
     for (int s = 0; s < NS; ++s)
 #pragma unroll
         for (int m = 0; m < MLP_G; ++m) acc[s][m] = 0.0f;
-    const double4 pi = pos[i];
     const double rc2 = (double)dp.rc * (double)dp.rc;
     const float pirc = 3.14159265358979f / dp.rc;
-    const int nf = ncnt[i];
-    for (int t = 0; t < nf; ++t) {
-        const int j = nbr[(size_t)t * n + i];
-        const int im = nimg[(size_t)t * n + i];
-        const double4 pj = pos[j];
-        const double3 d3 = separation64(pi, pj, im, g.v);
-        const double r2 = dot64(d3);
-        if (!(r2 < rc2)) continue;
-        const float r = (float)sqrt(r2);
+    const int hits = near_neighbors<L, CAP>(i, n, lane, g, pos, nbr, nimg, i < n ? ncnt[i] : 0,
+                                            rc2, s_j[a], s_r[a],
+                                            [&](int h, int j, float r, int sj) {
+        if (near && h < CORR_NEAR)
+            near[(size_t)i * CORR_NEAR + h] = make_int2(j << 2 | sj, __float_as_int(r));
         const float fc = 0.5f * (cosf(r * pirc) + 1.0f);
-        const int sj = (int)pj.w;
 #pragma unroll
         for (int m = 0; m < MLP_G; ++m) {
             const float dr = r - dp.mu[m];
@@ -85,7 +154,14 @@ __global__ __launch_bounds__(256) void k_descriptors(int n, CellGeom g,
                 acc[NS - 1][m] += (sj == 1) ? v : 0.0f;
             }
         }
-    }
+    });
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int m = 0; m < MLP_G; ++m)
+#pragma unroll
+            for (int w = L / 2; w > 0; w >>= 1) acc[s][m] += __shfl_xor(acc[s][m], w, L);
+    if (i >= n || lane != 0) return;
     float4 *o = reinterpret_cast<float4 *>(feat + (size_t)i * MLP_F);
 #pragma unroll
     for (int q = 0; q < MLP_F / 4; ++q) {
@@ -97,7 +173,8 @@ __global__ __launch_bounds__(256) void k_descriptors(int n, CellGeom g,
         }
         o[q] = make_float4(f[0], f[1], f[2], f[3]);
     }
-    spec[i] = (int)pi.w;
+    spec[i] = (int)pos[i].w;
+    if (near) nnear[i] = hits;
 }
 
 // normalized, BF16-rounded input pairs of one sample
@@ -473,54 +550,77 @@ __global__ __launch_bounds__(128) void k_corr_features(int n, CellGeom g,
     o[CORR_NC - 1] = di;
 }
 
-// One corrector stage, CORR_LANES lanes per atom (the atom's neighbor list
-// split over the lanes, partial sums reduced by cross-lane shuffles); the
-// stage's coefficients are staged in LDS and read per pair class.
+// One corrector stage, CORR_LANES lanes per atom (the atom's neighbors within
+// rc split over the lanes, partial sums reduced by cross-lane shuffles); the
+// stage's coefficients are staged in LDS and read per pair class.  The stages
+// of one warm start share the neighbors that k_descriptors found: read there,
+// or again from the full list by an atom with more than CORR_NEAR of them.
+// 24,576 atoms, 60 neighbors of 400 entries within rc: 99 us over the list
+// with the Gaussians inside the loop, 77 us compacted, 23 us from near.
 constexpr int CORR_LANES = 16;
-
 __global__ __launch_bounds__(256) void k_corr_stage(int n, CellGeom g,
                                                     const double4 *__restrict__ pos,
                                                     const int *__restrict__ nbr,
                                                     const int *__restrict__ nimg,
                                                     const int *__restrict__ ncnt, DescParams dp,
+                                                    const int2 *__restrict__ near,
+                                                    const int *__restrict__ nnear,
                                                     const double *__restrict__ coef,
                                                     const double *__restrict__ chi,
                                                     const double *__restrict__ prev,
                                                     double *__restrict__ q,
                                                     double *__restrict__ next)
 {
+    constexpr int L = CORR_LANES, CAP = 128, U = 4;
     __shared__ double sc[CORR_NC];
+    __shared__ int s_j[256 / L][CAP];
+    __shared__ float s_r[256 / L][CAP];
     for (int k = threadIdx.x; k < CORR_NC; k += blockDim.x) sc[k] = coef[k];
     __syncthreads();
-    const int i = (blockIdx.x * blockDim.x + threadIdx.x) / CORR_LANES;
-    const int lane = threadIdx.x % CORR_LANES;
+    const int i = (blockIdx.x * blockDim.x + threadIdx.x) / L;
+    const int lane = threadIdx.x % L, grp = threadIdx.x / L;
+    const int si = i < n ? (int)pos[i].w : 0;
+    const double rc2 = (double)dp.rc * (double)dp.rc;
+    const float pirc = 3.14159265358979f / dp.rc;
+    const double ci = i < n ? chi[i] : 0.0, di = i < n ? prev[i] : 0.0;
     double acc = 0.0;
-    if (i < n) {
-        const double4 pi = pos[i];
-        const int si = (int)pi.w;
-        const double rc2 = (double)dp.rc * (double)dp.rc;
-        const float pirc = 3.14159265358979f / dp.rc;
-        const double ci = chi[i], di = prev[i];
-        const int nf = ncnt[i];
-        for (int t = lane; t < nf; t += CORR_LANES) {
-            const int j = nbr[(size_t)t * n + i];
-            const int im = nimg[(size_t)t * n + i];
-            const double4 pj = pos[j];
-            const double r2 = dot64(separation64(pi, pj, im, g.v));
-            if (!(r2 < rc2)) continue;
-            float phi[CORR_G];
-            corr_basis((float)sqrt(r2), dp, pirc, phi);
-            const double *a = sc + (si + (int)pj.w) * CORR_G;
-            const double *b = a + 3 * CORR_G;
-            double wa = 0.0, wb = 0.0;
+    auto term = [&](float r, int sj, double cj, double dj) {
+        float phi[CORR_G];
+        corr_basis(r, dp, pirc, phi);
+        const double *a = sc + (si + sj) * CORR_G;
+        const double *b = a + 3 * CORR_G;
+        double wa = 0.0, wb = 0.0;
 #pragma unroll
-            for (int m = 0; m < CORR_G; ++m) {
-                wa += a[m] * (double)phi[m];
-                wb += b[m] * (double)phi[m];
+        for (int m = 0; m < CORR_G; ++m) {
+            wa += a[m] * (double)phi[m];
+            wb += b[m] * (double)phi[m];
+        }
+        acc += wa * (cj - ci) + wb * (dj - di);
+    };
+    const int hits = i < n ? nnear[i] : 0;
+    const bool kept = hits <= CORR_NEAR;
+    if (kept) {
+        const int2 *row = near + (size_t)i * CORR_NEAR;
+        for (int h0 = lane; h0 < hits; h0 += L * U) {
+            int2 e[U];
+            double cj[U], dj[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) e[u] = row[min(h0 + u * L, hits - 1)];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                cj[u] = chi[e[u].x >> 2];
+                dj[u] = prev[e[u].x >> 2];
             }
-            acc += wa * (chi[j] - ci) + wb * (prev[j] - di);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (h0 + u * L < hits) term(__int_as_float(e[u].y), e[u].x & 3, cj[u], dj[u]);
         }
     }
+    if (__any(!kept))
+        near_neighbors<L, CAP>(i, n, lane, g, pos, nbr, nimg, kept ? 0 : ncnt[i], rc2, s_j[grp],
+                               s_r[grp], [&](int, int j, float r, int sj) {
+            term(r, sj, chi[j], prev[j]);
+        });
     // every lane of the group takes part in the shuffles (no early return)
 #pragma unroll
     for (int w = CORR_LANES / 2; w > 0; w >>= 1) acc += __shfl_xor(acc, w, CORR_LANES);
@@ -576,20 +676,27 @@ void MlpState::release_all()
     ccoef.release();
     cprev.release();
     cnext.release();
+    near.release();
+    nnear.release();
     cfeat.release();
     corr_stages = 0;
 }
 
-void mlp_descriptors(System &S, const MlpState &m, hipStream_t st)
+void mlp_descriptors(System &S, MlpState &m, bool keep_near, hipStream_t st)
 {
     const int n = S.n;
-    const int blocks = div_up(n, 256);
+    if (keep_near) {
+        m.near.ensure((size_t)n * CORR_NEAR);
+        m.nnear.ensure(n);
+    }
+    int2 *near = keep_near ? m.near.p : nullptr;
+    const int blocks = (int)div_up((long)n * DESC_LANES, 256L);
     if (m.nspecies == 1)
         k_descriptors<1><<<blocks, 256, 0, st>>>(n, S.geom, S.pos.p, S.nbr.p, S.nimg.p, S.ncnt.p,
-                                                 m.dp, m.sfeat.p, m.sspec.p);
+                                                 m.dp, m.sfeat.p, m.sspec.p, near, m.nnear.p);
     else
         k_descriptors<2><<<blocks, 256, 0, st>>>(n, S.geom, S.pos.p, S.nbr.p, S.nimg.p, S.ncnt.p,
-                                                 m.dp, m.sfeat.p, m.sspec.p);
+                                                 m.dp, m.sfeat.p, m.sspec.p, near, m.nnear.p);
     HIP_TRY(hipGetLastError());
 }
 
@@ -664,7 +771,9 @@ void mlp_corrector_stage(System &S, const MlpState &m, const double *coef, const
                          const double *prev, double *next, hipStream_t st)
 {
     const long threads = (long)S.n * CORR_LANES;
-    k_corr_stage<<<(int)div_up(threads, 256L), 256, 0, st>>>(S.n, S.geom, S.pos.p, S.nbr.p, S.nimg.p,
-                                                   S.ncnt.p, m.dp, coef, chi, prev, S.q.p, next);
+    k_corr_stage<<<(int)div_up(threads, 256L), 256, 0, st>>>(S.n, S.geom, S.pos.p, S.nbr.p,
+                                                             S.nimg.p, S.ncnt.p, m.dp, m.near.p,
+                                                             m.nnear.p, coef, chi, prev, S.q.p,
+                                                             next);
     HIP_TRY(hipGetLastError());
 }
