@@ -57,36 +57,40 @@ __device__ __forceinline__ Leg load_leg(const double4 &pv, int j, int img,
 }
 
 // The angle a-v-b of one row (evaluate_energy_bond_bending and
-// evaluate_force_bond_bending, Potentials.f90:3196-3328), with
-// s1 = r_v - r_a, s2 = r_b - r_v: E = eps (cos^n - c0)^m and, with FORCE,
-// the forces f[0..2] on a, v, b.
+// evaluate_force_bond_bending, Potentials.f90:3196-3328) seen from leg a, with
+// da = r_a - r_v and db = r_b - r_v: E = eps (cos^n - c0)^m times both legs'
+// f_c and, with FORCE, the force on a, t.  The same for either leg in the
+// first place: the angle and its smoothing are symmetric in them.
 template <bool FORCE>
-__device__ __forceinline__ double bend_term(const BendTerm &P, const double3 &s1, double r1,
-                                            const double3 &s2, double r2, double3 *f)
+__device__ __forceinline__ double bend_term(const BendTerm &P, const double3 &da, double ra,
+                                            const double3 &db, double rb, double3 &t)
 {
-    const double3 t1 = make_double3(-s1.x, -s1.y, -s1.z);
-    const double r3 = t1.x * s2.x + t1.y * s2.y + t1.z * s2.z;
-    const double e = P.eps * bend_ipow(bend_ipow(r3 / (r1 * r2), P.n) - P.c0, P.m);
-    if (FORCE) {
-        const double k1 = r3 / (r1 * r1), k2 = r3 / (r2 * r2);
-        const double3 t3 = make_double3(s2.x - k1 * t1.x, s2.y - k1 * t1.y, s2.z - k1 * t1.z);
-        const double3 t4 = make_double3(t1.x - k2 * s2.x, t1.y - k2 * s2.y, t1.z - k2 * s2.z);
-        const double ratio = 1.0 / (r1 * r2);
-        const double cosplain = r3 * ratio;
-        const double cospower = bend_ipow(cosplain, P.n - 1);
-        const double r6 = P.eps * (double)(P.m * P.n) *
-                          bend_ipow(cospower * cosplain - P.c0, P.m - 1) * cospower;
-        f[0] = make_double3(-t3.x * ratio * r6, -t3.y * ratio * r6, -t3.z * ratio * r6);
-        f[1] = make_double3((t3.x + t4.x) * ratio * r6, (t3.y + t4.y) * ratio * r6,
-                            (t3.z + t4.z) * ratio * r6);
-        f[2] = make_double3(-t4.x * ratio * r6, -t4.y * ratio * r6, -t4.z * ratio * r6);
+    const double ira = recip64(ra), ratio = ira * recip64(rb);
+    const double r3 = da.x * db.x + da.y * db.y + da.z * db.z;
+    const double cosine = r3 * ratio;
+    double fa = 1.0, dfa = 0.0, fb = 1.0, dfb = 0.0;
+    if (P.smooth) {
+        smooth64(ra, P.cut, P.soft, &fa, &dfa);
+        smooth64(rb, P.cut, P.soft, &fb, &dfb);
     }
-    return e;
+    const double e = P.eps * bend_ipow(bend_ipow(cosine, P.n) - P.c0, P.m);
+    if (FORCE) {
+        const double cospower = bend_ipow(cosine, P.n - 1);
+        const double xm = bend_ipow(cospower * cosine - P.c0, P.m - 1);
+        // dE/dcos f_c f_c along -(d cos / d r_a), and f_c's own slope
+        const double k = ira * ira * r3;
+        const double c = ratio * P.eps * (double)(P.m * P.n) * xm * cospower * fa * fb;
+        const double s = dfa * ira * fb * e;
+        t = make_double3(-c * (db.x - k * da.x) - s * da.x, -c * (db.y - k * da.y) - s * da.y,
+                         -c * (db.z - k * da.z) - s * da.z);
+    }
+    return e * fa * fb;
 }
 
-// The short list of each vertex: its neighbors within the largest bend
-// cutoff, widened by 1e-10 relative so that a pair inside a cutoff seen from
-// either end is in both atoms' lists.
+// The short list of each vertex: its neighbors that are a leg of some row's
+// angle at the vertex, or it of theirs (species and cutoff, bend_leg2: the
+// same answer seen from either end, so a pair is in both atoms' lists).
+// Silica within 3.05 A: 3 legs an atom instead of 8 neighbors.
 template <class Geo>
 __global__ __launch_bounds__(BB) void k_bend_list(int n, Geo geo, const double4 *__restrict__ pos,
                                                   const int *__restrict__ nbr,
@@ -101,16 +105,29 @@ __global__ __launch_bounds__(BB) void k_bend_list(int n, Geo geo, const double4 
     const double4 pv = pos[v];
     const double *cv = geo.vec(v);
     const size_t N = (size_t)n;
-    const double bc2 = PM->bend_cut * PM->bend_cut * (1.0 + 1e-10);
+    const double *leg2 = PM->bend_leg2[(int)pv.w];
     const int nf = ncnt[v];
     int c = 0;
-    for (int t = 0; t < nf; ++t) {
-        const int j = nbr[(size_t)t * N + v], img = nimg[(size_t)t * N + v];
-        const double3 d = separation64(pv, pos[j], img, cv);
-        if (!(dot64(d) < bc2)) continue;
-        bsj[(size_t)c * N + v] = j;
-        bsimg[(size_t)c * N + v] = img;
-        ++c;
+    constexpr int U = 8;   // entries in flight
+    for (int t0 = 0; t0 < nf; t0 += U) {
+        int jv[U], iv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const size_t at = (size_t)min(t0 + u, nf - 1) * N + v;
+            jv[u] = nbr[at];
+            iv[u] = nimg[at];
+        }
+        double4 p[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) p[u] = pos[jv[u]];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (t0 + u >= nf) break;
+            if (!(dot64(separation64(pv, p[u], iv[u], cv)) < leg2[(int)p[u].w])) continue;
+            bsj[(size_t)c * N + v] = jv[u];
+            bsimg[(size_t)c * N + v] = iv[u];
+            ++c;
+        }
     }
     bscnt[v] = c;
 }
@@ -134,6 +151,14 @@ __global__ __launch_bounds__(BB) void k_bend_angles(int n, Geo geo, const double
     constexpr bool FORCE = MODE != PAIR_ENERGY;
     constexpr bool VIR = MODE == PAIR_FORCES;
     __shared__ double red[7][BB];
+    __shared__ BendTerm rows[PYSIC_MAXB];
+    {
+        const int *src = reinterpret_cast<const int *>(&PM->bend[0]);
+        int *dst = reinterpret_cast<int *>(&rows[0]);
+        const int words = PM->nbend * (int)(sizeof(BendTerm) / sizeof(int));
+        for (int w = threadIdx.x; w < words; w += BB) dst[w] = src[w];
+    }
+    __syncthreads();
     const int blk = xcd_block(gridDim.x);
     const int gid = blk * BB + threadIdx.x;
     // G * H consecutive lanes per vertex: lane l + G h takes the legs
@@ -169,44 +194,20 @@ __global__ __launch_bounds__(BB) void k_bend_angles(int n, Geo geo, const double
                 // the second leg is searched within atom 1's radius, which
                 // for (first, v) is the vertex's own largest potential cutoff
                 if (!vfirst && !(Ll.r < vmax)) continue;
-                const double3 s1 = make_double3(-Fl.d.x, -Fl.d.y, -Fl.d.z), s2 = Ll.d;
                 const double r1 = Fl.r, r2 = Ll.r;
-                for (int k = 0; k < nbend; ++k) {
-                    const BendTerm &P = PM->bend[k];
-                    if (P.e[0] != e0 || P.e[1] != e1 || P.e[2] != Ll.s) continue;
-                    if (!(P.cut > r1) || !(P.cut > r2) || P.vertex != sv) continue;
-                    double fc1 = 1.0, fc2 = 1.0;
-                    if (P.smooth) {
-                        fc1 = fc64(r1, P.cut, P.soft);
-                        fc2 = fc64(r2, P.cut, P.soft);
-                    }
-                    if (!FORCE) {
-                        const double ev = bend_term<false>(P, s1, r1, s2, r2, nullptr);
-                        e += 0.5 * (ev * fc1 * fc2 * (1.0 + 1.0 + 1.0) / 3.0);
-                        continue;
-                    }
-                    double3 f[3];
-                    const double ev = bend_term<true>(P, s1, r1, s2, r2, f);
-                    const double ff = fc1 * fc2;
+                // the lanes look for their row first and evaluate it together:
+                // a wave's vertices and orientations match different rows
+                for (int k = 0;; ++k) {
+                    while (k < nbend &&
+                           (rows[k].e[0] != e0 || rows[k].e[1] != e1 || rows[k].e[2] != Ll.s ||
+                            !(rows[k].cut > r1) || !(rows[k].cut > r2) || rows[k].vertex != sv))
+                        ++k;
+                    if (k >= nbend) break;
                     double3 t;
-                    if (ab) {  // this lane's leg is the first: f[0] and fc(r1)'s gradient
-                        double3 g1 = make_double3(0.0, 0.0, 0.0);
-                        if (P.smooth) {
-                            const double d1 = dfc64(r1, P.cut, P.soft) / r1;
-                            g1 = make_double3(s1.x * d1 * fc2 * ev, s1.y * d1 * fc2 * ev,
-                                              s1.z * d1 * fc2 * ev);
-                        }
-                        t = make_double3(f[0].x * ff + g1.x, f[0].y * ff + g1.y,
-                                         f[0].z * ff + g1.z);
-                    } else {  // the last: f[2] and fc(r2)'s gradient
-                        double3 g2 = make_double3(0.0, 0.0, 0.0);
-                        if (P.smooth && r2 != 0.0) {
-                            const double d2 = dfc64(r2, P.cut, P.soft) / r2;
-                            g2 = make_double3(s2.x * d2 * fc1 * ev, s2.y * d2 * fc1 * ev,
-                                              s2.z * d2 * fc1 * ev);
-                        }
-                        t = make_double3(f[2].x * ff - g2.x, f[2].y * ff - g2.y,
-                                         f[2].z * ff - g2.z);
+                    const double ev = bend_term<FORCE>(rows[k], A.d, A.r, B.d, B.r, t);
+                    if (!FORCE) {
+                        e += 0.5 * ev;
+                        continue;
                     }
                     fa.x += t.x;
                     fa.y += t.y;
@@ -311,12 +312,15 @@ __global__ __launch_bounds__(BB) void k_bend_gather(int n, const int *__restrict
 
 }  // namespace
 
-// lanes per vertex: 16 covers the legs of a 3 A cutoff in oxides with one
-// leg per lane (24,576 atoms of COMB SiO2: angles + gather 337 us with 4
-// lanes, 247 with 8, 196 with 16)
-constexpr int BG_LANES = 16;
-// and each leg's partners split over BG_PARTS lanes
-constexpr int BG_PARTS = 2;
+// lanes per vertex: the two to four legs of an oxide's vertex, one or two a
+// lane, and each leg's partners over BG_PARTS lanes.  24,576 atoms of COMB
+// silica, the angle kernel alone: 80 us with all neighbors within 3.05 A in
+// the lists (16 x 2 lanes) and each lane evaluating its rows as it met them,
+// 57 with the legs alone, 44 with the rows found first and evaluated together
+// (with the other two chains beside it 55; 8 x 4 lanes 47, 8 x 2 65, 4 x 2 80,
+// 2 x 4 87, and the same step time within 2% for all of them).
+constexpr int BG_LANES = 4;
+constexpr int BG_PARTS = 4;
 // lanes per atom in the gather: its slots split over 8 lanes
 constexpr int BG_GATHER_LANES = 8;
 

@@ -117,7 +117,7 @@ void System::release_all()
     DBuf<double4> *b4[] = {&pos, &pos2, &mom, &mom2, &frc, &frc2};
     for (auto *b : b4) b->release();
     DBuf<double> *bd[] = {&q, &q2, &cut, &cut2, &partial, &totals, &gpartial,
-                          &gtotals, &atom_ev, &cell_ev};
+                          &gtotals, &atom_ev, &cell_ev, &qhalf};
     for (auto *b : bd) b->release();
     DBuf<int> *bi[] = {&id, &id2, &key, &key2, &wrap, &wrap2, &perm, &cellcount, &cellstart, &cellfill, &scanblk,
                        &prevstart, &dirty, &dirty2, &scanloc, &srow,
@@ -339,7 +339,18 @@ void compile_model(pysic_ctx *h)
             B.cut = d[6];
             if (d[7] > 0.0 && d[7] < d[6]) { B.soft = d[7]; B.smooth = 1; }
             else { B.soft = d[6]; B.smooth = 0; }
-            P.bend_cut = std::max(P.bend_cut, d[6]);
+            const double leg2 = d[6] * d[6] * (1.0 + 1e-10);
+            auto leg = [&](int s) {
+                double &a = P.bend_leg2[B.vertex][s], &b = P.bend_leg2[s][B.vertex];
+                a = b = std::max(a, leg2);
+            };
+            // the vertex is target 0 or 1 of the row (the angle is found from
+            // the pair of the vertex and its first leg); the others are legs
+            if (B.vertex >= 0 && B.vertex < PYSIC_MAXS && d[6] > 0.0) {
+                if (e1 == B.vertex) leg(e2);
+                if (e2 == B.vertex) leg(e1);
+                if (e1 == B.vertex || e2 == B.vertex) leg(e3);
+            }
             P.has_pairs = 1;
         } else if (type == 10 || type == 11) {
             PYSIC_REQUIRE(group < 0, PYSIC_EINVAL,
@@ -402,6 +413,24 @@ void compile_model(pysic_ctx *h)
                         PYSIC_REQUIRE(P.ncf < PYSIC_MAXCF, PYSIC_EINVAL,
                                       "too many distinct charge-dependent pair factors "
                                       "(at most 16)");
+                        for (int a = 0; a < 2 && F.type != 14; ++a) {
+                            ChargeHalf H;
+                            std::memset(&H, 0, sizeof(H));
+                            H.type = F.type;
+                            if (F.type == 12) {
+                                const double v[5] = {Q.p[1 + 4 * a], Q.beta[a], Q.p[3 + 4 * a],
+                                                     Q.eta[a], Q.p[9 + a]};
+                                std::memcpy(H.p, v, sizeof(v));
+                            } else {
+                                std::memcpy(H.p, Q.p + 4 * a, 4 * sizeof(double));
+                            }
+                            int col = 0;
+                            while (col < P.nhalf &&
+                                   std::memcmp(&P.half[col], &H, sizeof(H)) != 0)
+                                ++col;
+                            if (col == P.nhalf) P.half[P.nhalf++] = H;
+                            P.hcol[P.ncf][a] = col;
+                        }
                         P.cf[P.ncf++] = Q;
                     }
                     F.toff = slot;
@@ -733,7 +762,7 @@ std::vector<const void *> graph_signature(pysic_ctx *h, bool rebuild)
             S.frc.p, S.flags.p, S.dmodel.p, S.cells.p, S.first_bin.p, S.cell_of.p, S.atom0.p,
             S.dpmodel.p, S.tables.p, S.gpartial.p, S.gtotals.p, S.totals.p, S.bsj.p,
             S.bsimg.p, S.bscnt.p, S.bG.p, S.dbmodel.p, S.osj.p, S.osimg.p, S.oscnt.p, S.oD.p,
-            S.oW.p, S.oown.p,
+            S.oW.p, S.oown.p, S.qhalf.p,
             (const void *)(long)S.cap, (const void *)(long)h->variant,
             (const void *)(long)S.site_grid, (const void *)(long)S.n, (const void *)(long)S.nbins,
             (const void *)(long)S.nb_method, (const void *)(long)(rebuild ? 1 : 0)};

@@ -75,6 +75,12 @@ struct ChargeFactor {
     double eta[2], beta[2];
     int orig, pad;
 };
+// One atom's part of a charge_exp or charge_abs factor, a function of its
+// charge alone: xi D(q) of charge_exp, f(q) of charge_abs.
+struct ChargeHalf {
+    int type, pad;        // 12 or 13
+    double p[5];          // 12: Rmax, beta, Qmax, eta, xi; 13: a, b, Q, n
+};
 struct GenPair {
     PairFactor f[PYSIC_MAXF];  // f[0] the potential, then its multipliers
     int nf;
@@ -117,8 +123,14 @@ struct PairModel {
     int needs_pick;       // a 'step' or charge factor: it depends on which atom the reference takes first
     int has_charge, ncf;  // charge-dependent factors (cf[0 .. ncf-1])
     ChargeFactor cf[PYSIC_MAXCF];
+    // the distinct halves of the factors, and which are those of factor c
+    int nhalf, pad_h;
+    int hcol[PYSIC_MAXCF][2];
+    ChargeHalf half[2 * PYSIC_MAXCF];
     int nbend, pad_b;     // bond_bend rows (bend[0 .. nbend-1])
-    double bend_cut;      // the largest bond_bend cutoff
+    // squared largest cutoff of the rows in which an atom of either species is
+    // a leg of an angle at one of the other, widened by 1e-10 relative; 0: none
+    double bend_leg2[PYSIC_MAXS][PYSIC_MAXS];
     // per species, the largest cutoff of the potentials whose first target
     // it is (the reference's max_potential_radius, Core.f90:1034-1125)
     double bend_maxpot[PYSIC_MAXS];
@@ -281,6 +293,56 @@ __device__ __forceinline__ double dfc64(double r, double hard, double soft)
     double f, df;
     smooth64(r, hard, soft, &f, &df);
     return df;
+}
+
+// The entries of one atom's full list that pass a test, taken by the L lanes
+// of its group (consecutive threads of one wave) and compacted into LDS, so
+// that the work on them is done by full lanes: with the test beside the work
+// in one loop, a wave does the work for nearly every entry as soon as one of
+// its 64 lanes has a hit.  test(position, image, j, hit) fills hit;
+// body(h, hit) is called by one lane for each hit h, in the list's order, so
+// sums have one order.  Returns the number of hits.  CAP of them are held at
+// a time, in held[] of the group.
+template <int L, int CAP, class T, class Test, class Body>
+__device__ __forceinline__ int lane_hits(int i, int n, int lane, const double4 *__restrict__ pos,
+                                         const int *__restrict__ nbr,
+                                         const int *__restrict__ nimg, int nf, T *held,
+                                         Test &&test, Body &&body)
+{
+    constexpr int U = 4;   // entries in flight per lane
+    static_assert(CAP >= L * U, "room for one batch");
+    const int shift = (threadIdx.x & 63) / L * L;
+    const unsigned long long mask = (1ull << L) - 1ull, below = (1ull << lane) - 1ull;
+    int done = 0, t0 = 0;
+    do {   // every condition here is the group's, not the lane's
+        int count = 0;
+        for (; t0 < nf && count <= CAP - L * U; t0 += L * U) {
+            int jv[U], iv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const size_t at = (size_t)min(t0 + u * L + lane, nf - 1) * n + i;
+                jv[u] = nbr[at];
+                iv[u] = nimg[at];
+            }
+            double4 pv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) pv[u] = pos[jv[u]];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                T hit;
+                const bool on = test(pv[u], iv[u], jv[u], hit) && t0 + u * L + lane < nf;
+                const unsigned long long b = (__ballot(on) >> shift) & mask;
+                if (on) held[count + __popcll(b & below)] = hit;
+                count += __popcll(b);
+            }
+        }
+        // one wave's LDS accesses complete in order; the compiler keeps them so
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        for (int h = lane; h < count; h += L) body(done + h, held[h]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        done += count;
+    } while (t0 < nf);
+    return done;
 }
 
 // x^y for the bond-order post-processing, where x >= 0: exp(y log x) for

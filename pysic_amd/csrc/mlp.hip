@@ -44,68 +44,23 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c)
                                            __builtin_bit_cast(bf16x2_t, b), c, false);
 }
 
-// The neighbors of one atom within rc, taken from its full list (radius 10.5 A
-// in the charge workloads, so one entry in five) by the L lanes of its group
-// and compacted into LDS, so that the Gaussians are evaluated by full lanes:
-// with the test inside the loop every wave ran them for nearly every entry.
-// body(h, j, r, species of j) is called by one lane for each hit h, in the
-// list's order, so the sums have one order; returns the number of hits.  The
-// group's lanes are consecutive threads of one wave; CAP hits are held at a
-// time.
+// The neighbors of one atom within rc, from its full list (radius 10.5 A in
+// the charge workloads: one entry in five), with the FP32 distances:
+// body(h, j, r, species of j), h < the number of them, which is returned.
 template <int L, int CAP, class Body>
 __device__ __forceinline__ int near_neighbors(int i, int n, int lane, const CellGeom &g,
                                               const double4 *__restrict__ pos,
                                               const int *__restrict__ nbr,
                                               const int *__restrict__ nimg, int nf, double rc2,
-                                              int *s_j, float *s_r, Body &&body)
+                                              int2 *held, Body &&body)
 {
-    constexpr int U = 4;   // entries in flight per lane
-    static_assert(CAP >= 2 * L * U, "room for a batch beside what is held");
-    const int shift = (threadIdx.x & 63) / L * L;
-    const unsigned long long mask = (1ull << L) - 1ull, below = (1ull << lane) - 1ull;
     const double4 pi = i < n ? pos[i] : make_double4(0, 0, 0, 0);
-    int held = 0, done = 0;
-    auto flush = [&]() {
-        for (int h = lane; h < held; h += L) body(done + h, s_j[h] >> 2, s_r[h], s_j[h] & 3);
-        done += held;
-        held = 0;
-    };
-    int longest = nf;   // the ballots are the wave's: its groups run together
-#pragma unroll
-    for (int d = L; d < 64; d <<= 1) longest = max(longest, __shfl_xor(longest, d));
-    for (int t0 = 0; t0 < longest; t0 += L * U) {
-        int jv[U], iv[U];
-        double4 pv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int t = t0 + u * L + lane;
-            jv[u] = -1;
-            iv[u] = 0;
-            if (t < nf) {
-                jv[u] = nbr[(size_t)t * n + i];
-                iv[u] = nimg[(size_t)t * n + i];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) pv[u] = pos[max(jv[u], 0)];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const double r2 = dot64(separation64(pi, pv[u], iv[u], g.v));
-            const bool hit = jv[u] >= 0 && r2 < rc2;
-            const unsigned long long b = (__ballot(hit) >> shift) & mask;
-            if (hit) {
-                const int at = held + __popcll(b & below);
-                s_j[at] = jv[u] << 2 | (int)pv[u].w;
-                s_r[at] = (float)sqrt(r2);
-            }
-            held += __popcll(b);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // one wave's LDS: in order
-        if (held > CAP - L * U) flush();
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    }
-    flush();
-    return done;
+    return lane_hits<L, CAP>(i, n, lane, pos, nbr, nimg, nf, held,
+                             [&](const double4 &pj, int im, int j, int2 &hit) {
+        const double r2 = dot64(separation64(pi, pj, im, g.v));
+        hit = make_int2(j << 2 | (int)pj.w, __float_as_int((float)sqrt(r2)));
+        return r2 < rc2;
+    }, [&](int h, const int2 &e) { body(h, e.x >> 2, __int_as_float(e.y), e.x & 3); });
 }
 
 // Descriptors, DESC_LANES lanes per atom.  24,576 atoms: 461 us with a thread
@@ -126,8 +81,7 @@ __global__ __launch_bounds__(256) void k_descriptors(int n, CellGeom g,
                                                      int *__restrict__ nnear)
 {
     constexpr int L = DESC_LANES, CAP = 96;
-    __shared__ int s_j[256 / L][CAP];
-    __shared__ float s_r[256 / L][CAP];
+    __shared__ int2 held[256 / L][CAP];
     const int i = (blockIdx.x * 256 + threadIdx.x) / L, lane = threadIdx.x % L;
     const int a = threadIdx.x / L;
     float acc[NS][MLP_G];
@@ -138,7 +92,7 @@ __global__ __launch_bounds__(256) void k_descriptors(int n, CellGeom g,
     const double rc2 = (double)dp.rc * (double)dp.rc;
     const float pirc = 3.14159265358979f / dp.rc;
     const int hits = near_neighbors<L, CAP>(i, n, lane, g, pos, nbr, nimg, i < n ? ncnt[i] : 0,
-                                            rc2, s_j[a], s_r[a],
+                                            rc2, held[a],
                                             [&](int h, int j, float r, int sj) {
         if (near && h < CORR_NEAR)
             near[(size_t)i * CORR_NEAR + h] = make_int2(j << 2 | sj, __float_as_int(r));
@@ -573,8 +527,7 @@ __global__ __launch_bounds__(256) void k_corr_stage(int n, CellGeom g,
 {
     constexpr int L = CORR_LANES, CAP = 128, U = 4;
     __shared__ double sc[CORR_NC];
-    __shared__ int s_j[256 / L][CAP];
-    __shared__ float s_r[256 / L][CAP];
+    __shared__ int2 held[256 / L][CAP];
     for (int k = threadIdx.x; k < CORR_NC; k += blockDim.x) sc[k] = coef[k];
     __syncthreads();
     const int i = (blockIdx.x * blockDim.x + threadIdx.x) / L;
@@ -617,8 +570,8 @@ __global__ __launch_bounds__(256) void k_corr_stage(int n, CellGeom g,
         }
     }
     if (__any(!kept))
-        near_neighbors<L, CAP>(i, n, lane, g, pos, nbr, nimg, kept ? 0 : ncnt[i], rc2, s_j[grp],
-                               s_r[grp], [&](int, int j, float r, int sj) {
+        near_neighbors<L, CAP>(i, n, lane, g, pos, nbr, nimg, kept ? 0 : ncnt[i], rc2, held[grp],
+                               [&](int, int j, float r, int sj) {
             term(r, sj, chi[j], prev[j]);
         });
     // every lane of the group takes part in the shuffles (no early return)

@@ -43,10 +43,48 @@ struct Radial {
 
 // The charges of a pair in the order the reference evaluates it (atom 1 the
 // atom pick takes first) and atom 1's species.
+// h: the atoms' charge halves (k_charge_halves), one column of n per half.
 struct QPair {
     double q1, q2;
     int s1;
+    int i1, i2;
+    const double *h;
+    size_t n;
 };
+
+// The charge-dependent functions of single atoms, once per evaluation: a
+// pair's factor then takes one exp or sqrt, where it took two powers per
+// factor and pair, and again from the pair's other end.  24,576 atoms of COMB
+// silica: 5 us for the six columns; the pair kernel goes from 57 to 35 us and
+// the bond-order pass from 89 to 51 with it and their full lanes.
+__global__ __launch_bounds__(PB) void k_charge_halves(int n, const PairModel *__restrict__ PM,
+                                                      const double *__restrict__ q,
+                                                      double *__restrict__ out)
+{
+    const int i = blockIdx.x * PB + threadIdx.x, col = blockIdx.y;
+    if (i >= n) return;
+    const ChargeHalf &H = PM->half[col];
+    double v;
+    if (H.type == 12) {
+        v = H.p[4] * (H.p[0] + pow(fabs(H.p[1] * (H.p[2] - q[i])), H.p[3]));
+    } else {
+        v = H.p[0] + H.p[1] * pow(fabs(q[i] - H.p[2]), H.p[3]);
+        if (v < 0.0) v = 0.0;
+    }
+    out[(size_t)col * n + i] = v;
+}
+__device__ __forceinline__ double charge_exp_value(const ChargeFactor &c, const int *col,
+                                                   const QPair &qp)
+{
+    const int a = qp.s1 != c.orig ? 1 : 0;
+    return c.p[0] * exp(0.5 * (qp.h[col[a] * qp.n + qp.i1] + qp.h[col[1 - a] * qp.n + qp.i2]));
+}
+__device__ __forceinline__ double charge_abs_value(const ChargeFactor &c, const int *col,
+                                                   const QPair &qp)
+{
+    const int a = qp.s1 != c.orig ? 1 : 0;
+    return sqrt(qp.h[col[a] * qp.n + qp.i1] * qp.h[col[1 - a] * qp.n + qp.i2]);
+}
 
 // charge_exp (evaluate_energy_charge_exp and _electronegativity_charge_exp,
 // Potentials.f90:3776-3836, 3847-3903): E = eps exp((xi1 D1 + xi2 D2) / 2),
@@ -63,12 +101,8 @@ __device__ __noinline__ double charge_exp(const ChargeFactor &c, const QPair &qp
     const double d2 = p[1 + 4 * b] + pow(fabs(d6), c.eta[b]);
     const double xi1 = p[9 + a], xi2 = p[9 + b];
     const double e = p[0] * exp(0.5 * (xi1 * d1 + xi2 * d2));
-    if (x) {
-        x[1] = e * xi2 * 0.5 * c.eta[b] * pow(fabs(d6), c.eta[b] - 1.0) * copysign(1.0, d6) *
-               c.beta[b];
-        x[0] = e * xi1 * 0.5 * c.eta[a] * pow(fabs(d5), c.eta[a] - 1.0) * copysign(1.0, d5) *
-               c.beta[a];
-    }
+    x[1] = e * xi2 * 0.5 * c.eta[b] * pow(fabs(d6), c.eta[b] - 1.0) * copysign(1.0, d6) * c.beta[b];
+    x[0] = e * xi1 * 0.5 * c.eta[a] * pow(fabs(d5), c.eta[a] - 1.0) * copysign(1.0, d5) * c.beta[a];
     return e;
 }
 
@@ -82,21 +116,19 @@ __device__ __noinline__ double charge_abs(const ChargeFactor &c, const QPair &qp
     const double *p = c.p;
     const double a1 = p[a], b1 = p[a + 1], Q1 = p[a + 2], n1 = p[a + 3];
     const double a2 = p[b], b2 = p[b + 1], Q2 = p[b + 2], n2 = p[b + 3];
-    if (x) {
-        const double abs1 = fabs(qp.q1 - Q1), abs2 = fabs(qp.q2 - Q2);
-        const double pow1 = pow(abs1, n1 - 1.0), pow2 = pow(abs2, n2 - 1.0);
-        double f1 = a1 + b1 * abs1 * pow1;
-        double f2 = a2 + b2 * abs2 * pow2;
-        const double dd1 = -n1 * pow1 * copysign(1.0, qp.q1 - Q1) * b1;
-        const double dd2 = -n2 * pow2 * copysign(1.0, qp.q2 - Q2) * b2;
-        double h = 0.5 / sqrt(f1 * f2);
-        if (f1 < 0.0) { f1 = 0.0; h = 0.0; }
-        if (f2 < 0.0) { f2 = 0.0; h = 0.0; }
-        x[0] = h * dd1 * f2;
-        x[1] = h * dd2 * f1;
-    }
-    double f1 = a1 + b1 * pow(fabs(qp.q1 - Q1), n1);
-    double f2 = a2 + b2 * pow(fabs(qp.q2 - Q2), n2);
+    const double abs1 = fabs(qp.q1 - Q1), abs2 = fabs(qp.q2 - Q2);
+    const double pow1 = pow(abs1, n1 - 1.0), pow2 = pow(abs2, n2 - 1.0);
+    double f1 = a1 + b1 * abs1 * pow1;
+    double f2 = a2 + b2 * abs2 * pow2;
+    const double dd1 = -n1 * pow1 * copysign(1.0, qp.q1 - Q1) * b1;
+    const double dd2 = -n2 * pow2 * copysign(1.0, qp.q2 - Q2) * b2;
+    double h = 0.5 / sqrt(f1 * f2);
+    if (f1 < 0.0) { f1 = 0.0; h = 0.0; }
+    if (f2 < 0.0) { f2 = 0.0; h = 0.0; }
+    x[0] = h * dd1 * f2;
+    x[1] = h * dd2 * f1;
+    f1 = a1 + b1 * pow(fabs(qp.q1 - Q1), n1);
+    f2 = a2 + b2 * pow(fabs(qp.q2 - Q2), n2);
     if (f1 < 0.0) f1 = 0.0;
     if (f2 < 0.0) f2 = 0.0;
     return sqrt(f1 * f2);
@@ -114,15 +146,19 @@ __device__ __forceinline__ double ipow(double x, int n)
 // charge_pair (evaluate_energy_charge_pair and
 // _electronegativity_charge_pair, Potentials.f90:4415-4506):
 // E = eps q1^n1 q2^n2 with integer exponents, swapped as for charge_exp.
+__device__ __forceinline__ double charge_pair_value(const ChargeFactor &c, const QPair &qp)
+{
+    const bool inv = qp.s1 != c.orig;
+    return c.p[0] * (ipow(qp.q1, (int)(inv ? c.p[2] : c.p[1])) *
+                     ipow(qp.q2, (int)(inv ? c.p[1] : c.p[2])));
+}
 __device__ __noinline__ double charge_pair(const ChargeFactor &c, const QPair &qp, double *x)
 {
     const bool inv = qp.s1 != c.orig;
     const int n1 = (int)(inv ? c.p[2] : c.p[1]), n2 = (int)(inv ? c.p[1] : c.p[2]);
-    if (x) {
-        x[0] = n1 > 0 ? -c.p[0] * (n1 * ipow(qp.q1, n1 - 1) * ipow(qp.q2, n2)) : 0.0;
-        x[1] = n2 > 0 ? -c.p[0] * (n2 * ipow(qp.q1, n1) * ipow(qp.q2, n2 - 1)) : 0.0;
-    }
-    return c.p[0] * (ipow(qp.q1, n1) * ipow(qp.q2, n2));
+    x[0] = n1 > 0 ? -c.p[0] * (n1 * ipow(qp.q1, n1 - 1) * ipow(qp.q2, n2)) : 0.0;
+    x[1] = n2 > 0 ? -c.p[0] * (n2 * ipow(qp.q1, n1) * ipow(qp.q2, n2 - 1)) : 0.0;
+    return charge_pair_value(c, qp);
 }
 
 // One factor at distance r > 0 (evaluate_energy_component and
@@ -131,7 +167,7 @@ __device__ __noinline__ double charge_pair(const ChargeFactor &c, const QPair &q
 // potential's cutoff (the spring's energy shift uses it).
 __device__ __forceinline__ Radial factor(const PairFactor &f, double r, double cut,
                                          const double2 *__restrict__ tab, bool need_force,
-                                         const ChargeFactor *cft, const QPair &qp)
+                                         const PairModel &PM, const QPair &qp)
 {
     Radial o{0.0, 0.0, 0.0};
     const double p0 = f.p[0], p1 = f.p[1], p2 = f.p[2], p3 = f.p[3];
@@ -211,13 +247,13 @@ __device__ __forceinline__ Radial factor(const PairFactor &f, double r, double c
         break;
     }
     case 12:  // charge_exp: no dependence on r (its force is the cutoff's)
-        o.v = charge_exp(cft[f.toff], qp, nullptr);
+        o.v = charge_exp_value(PM.cf[f.toff], PM.hcol[f.toff], qp);
         break;
     case 13:  // charge_abs
-        o.v = charge_abs(cft[f.toff], qp, nullptr);
+        o.v = charge_abs_value(PM.cf[f.toff], PM.hcol[f.toff], qp);
         break;
     case 14:  // charge_pair
-        o.v = charge_pair(cft[f.toff], qp, nullptr);
+        o.v = charge_pair_value(PM.cf[f.toff], qp);
         break;
     default:
         break;
@@ -233,14 +269,14 @@ __device__ __forceinline__ Radial factor(const PairFactor &f, double r, double c
 // re-evaluates each factor with its force.
 __device__ __forceinline__ Radial potential(const GenPair &T, double r,
                                             const double2 *__restrict__ tab, bool need_force,
-                                            const ChargeFactor *cft, const QPair &qp)
+                                            const PairModel &PM, const QPair &qp)
 {
     const int nf = T.nf;
-    if (nf == 1) return factor(T.f[0], r, T.cut, tab, need_force, cft, qp);
+    if (nf == 1) return factor(T.f[0], r, T.cut, tab, need_force, PM, qp);
     double e = 1.0, enz = 1.0;
     int zeros = 0;
     for (int k = 0; k < nf; ++k) {
-        const double v = factor(T.f[k], r, T.cut, tab, false, cft, qp).v;
+        const double v = factor(T.f[k], r, T.cut, tab, false, PM, qp).v;
         e = e * v;
         if (v != 0.0) enz = enz * v;
         else ++zeros;
@@ -250,7 +286,7 @@ __device__ __forceinline__ Radial potential(const GenPair &T, double r,
     for (int k = 0; k < nf; ++k) {
         // a charge-dependent factor has no r dependence: nothing to add
         if (T.f[k].type >= 12) continue;
-        const Radial q = factor(T.f[k], r, T.cut, tab, true, cft, qp);
+        const Radial q = factor(T.f[k], r, T.cut, tab, true, PM, qp);
         const double w = q.v != 0.0 ? e / q.v : (zeros == 1 ? enz : 0.0);
         out.g += w * q.g;
         out.c += w * q.c;
@@ -263,7 +299,7 @@ __device__ __forceinline__ Radial potential(const GenPair &T, double r,
 // prod_{j != k} E_j x_k where E_k = 0; factors without charge dependence
 // have x_k = 0.
 __device__ void potential_chi(const GenPair &T, double r, const double2 *__restrict__ tab,
-                              const ChargeFactor *cft, const QPair &qp, double *x)
+                              const PairModel &PM, const QPair &qp, double *x)
 {
     x[0] = x[1] = 0.0;
     double me[PYSIC_MAXF], mx[PYSIC_MAXF][2], e = 1.0;
@@ -271,10 +307,10 @@ __device__ void potential_chi(const GenPair &T, double r, const double2 *__restr
     for (int k = 0; k < nf; ++k) {
         const PairFactor &f = T.f[k];
         mx[k][0] = mx[k][1] = 0.0;
-        if (f.type == 12) me[k] = charge_exp(cft[f.toff], qp, mx[k]);
-        else if (f.type == 13) me[k] = charge_abs(cft[f.toff], qp, mx[k]);
-        else if (f.type == 14) me[k] = charge_pair(cft[f.toff], qp, mx[k]);
-        else me[k] = factor(f, r, T.cut, tab, false, cft, qp).v;
+        if (f.type == 12) me[k] = charge_exp(PM.cf[f.toff], qp, mx[k]);
+        else if (f.type == 13) me[k] = charge_abs(PM.cf[f.toff], qp, mx[k]);
+        else if (f.type == 14) me[k] = charge_pair(PM.cf[f.toff], qp, mx[k]);
+        else me[k] = factor(f, r, T.cut, tab, false, PM, qp).v;
     }
     if (nf == 1) {
         x[0] = mx[0][0];
@@ -380,10 +416,10 @@ __device__ __forceinline__ bool visit(const PairLds<0> &L, int si, int sj, doubl
         const GenPair &T = P.pair[si][sj][c];
         if (!(T.cut > r)) continue;
         if (!FORCE) {
-            const Radial q = potential(T, r, tab, false, P.cf, qp);
+            const Radial q = potential(T, r, tab, false, P, qp);
             v += T.smooth ? q.v * fc64(r, T.cut, T.soft) : q.v;
         } else if (r > 0.0) {  // the reference's forces vanish at r == 0
-            const Radial q = potential(T, r, tab, true, P.cf, qp);
+            const Radial q = potential(T, r, tab, true, P, qp);
             if (T.smooth) {
                 // f1 fc + v grad(fc), grad(fc) = fc' s / r
                 const double f = fc64(r, T.cut, T.soft), df = dfc64(r, T.cut, T.soft);
@@ -414,7 +450,8 @@ __device__ __forceinline__ bool visit(const PairLds<0> &L, int si, int sj, doubl
 // work (exp, pow and the products) is long enough that one thread per atom
 // leaves a system of some ten thousand atoms on a fraction of the chip
 // (24,576 atoms of COMB SiO2: 381 us with 1 lane, 209 with 2, 144 with 4,
-// 140 with 8).  Above that, one thread per atom already fills the chip, and
+// 140 with 8), and its lanes take the entries within the cutoffs, compacted
+// first (lane_hits).  Above that, one thread per atom already fills the chip, and
 // each extra block would stage the whole model into LDS once more.
 // The LJ kinds take 8, 4 or 2 lanes up to LJ_LANES_ATOMS / lanes atoms, 4
 // neighbors in flight each, for the same reason: 13,500 argon atoms are 211
@@ -438,6 +475,7 @@ __global__ __launch_bounds__(PB) void k_pairs(int n, Geo geo, const double4 *__r
                                               const PairModel *__restrict__ PM,
                                               const double2 *__restrict__ tab,
                                               const double *__restrict__ q,
+                                              const double *__restrict__ qh,
                                               double4 *__restrict__ frc, int accumulate,
                                               double4 *__restrict__ mom, double half_dt, int kick,
                                               double *__restrict__ partial)
@@ -447,6 +485,8 @@ __global__ __launch_bounds__(PB) void k_pairs(int n, Geo geo, const double4 *__r
     constexpr int NBU = KIND == 0 ? 2 : G == 1 ? PYSIC_PAIR_NBU : 4;
     __shared__ PairLds<KIND> lds;
     __shared__ double red[7][PB];
+    constexpr int HITS = 48;
+    __shared__ int2 held[KIND == 0 && G > 1 ? PB / G : 1][HITS];
     stage(lds, PM);
     __syncthreads();
     const int blk = xcd_block(gridDim.x);
@@ -477,9 +517,54 @@ __global__ __launch_bounds__(PB) void k_pairs(int n, Geo geo, const double4 *__r
         const double qi = charged ? q[i] : 0.0;
         LJPair one{};
         if constexpr (KIND == 2) one = PM->lj[0][0];
+        auto one_pair = [&](int j, int im, const double4 &pj) {
+            const double3 d = separation64(pi, pj, im, cv);
+            const double r2 = dot64(d);
+            double v, G2, C;
+            bool on;
+            if constexpr (KIND == 2) on = visit<FORCE>(one, r2, v, G2, C);
+            else if constexpr (KIND == 1) on = visit<FORCE>(lds.lj[si][(int)pj.w], r2, v, G2, C);
+            else {
+                QPair qp{};
+                if (charged) {
+                    const int sj = (int)pj.w;
+                    const double qj = q[j];
+                    if (pick_dev(idi, id[j], im)) qp = QPair{qi, qj, si, i, j, qh, (size_t)n};
+                    else qp = QPair{qj, qi, sj, j, i, qh, (size_t)n};
+                }
+                on = visit<FORCE>(lds, si, (int)pj.w, r2, v, G2, C, tab, qp);
+            }
+            if (!on) return;
+            if (!FORCE) {
+                e += 0.5 * v;
+            } else {
+                // atom i is the first atom when pick(i, j) holds: g_i = f1
+                // with s = r_ij; otherwise g_i = -f1 with s = -r_ij
+                double cs = C;
+                if (pick && C != 0.0 && !pick_dev(idi, id[j], im)) cs = -C;
+                const double gx = G2 * d.x + cs, gy = G2 * d.y + cs, gz = G2 * d.z + cs;
+                fx += gx; fy += gy; fz += gz;
+                if (VIR) {
+                    w0 -= 0.5 * d.x * gx;
+                    w1 -= 0.5 * d.y * gy;
+                    w2 -= 0.5 * d.z * gz;
+                    w3 -= 0.5 * d.y * gz;
+                    w4 -= 0.5 * d.x * gz;
+                    w5 -= 0.5 * d.x * gy;
+                }
+            }
+        };
         // list rows t0 .. t0 + NBU - 1 of atom i (column-major: row t at t n + i)
         const size_t stride = (size_t)n;
-        for (int t0 = lane * NBU; t0 < nf; t0 += G * NBU) {
+        if constexpr (KIND == 0 && G > 1) {
+            lane_hits<G, HITS>(i, n, lane, pos, nbr, nimg, nf, held[threadIdx.x / G],
+                               [&](const double4 &pj, int im, int j, int2 &hit) {
+                hit = make_int2(j, im);
+                const int sj = (int)pj.w;
+                return lds.pm.npair[si][sj] != 0 &&
+                       dot64(separation64(pi, pj, im, cv)) < lds.pm.cut2_hi[si][sj];
+            }, [&](int, const int2 &h) { one_pair(h.x, h.y, pos[h.x]); });
+        } else for (int t0 = lane * NBU; t0 < nf; t0 += G * NBU) {
             const int *pn = nbr + (size_t)t0 * stride + i, *pm = nimg + (size_t)t0 * stride + i;
             int jv[NBU], iv[NBU];
 #pragma unroll
@@ -497,41 +582,7 @@ __global__ __launch_bounds__(PB) void k_pairs(int n, Geo geo, const double4 *__r
 #pragma unroll
             for (int u = 0; u < NBU; ++u) {
                 if (t0 + u >= nf) break;
-                const double3 d = separation64(pi, pv[u], iv[u], cv);
-                const double r2 = dot64(d);
-                double v, G2, C;
-                bool on;
-                if constexpr (KIND == 2) on = visit<FORCE>(one, r2, v, G2, C);
-                else if constexpr (KIND == 1) on = visit<FORCE>(lds.lj[si][(int)pv[u].w], r2, v, G2, C);
-                else {
-                    QPair qp{0.0, 0.0, 0};
-                    if (charged) {
-                        const int j = jv[u], sj = (int)pv[u].w;
-                        const double qj = q[j];
-                        if (pick_dev(idi, id[j], iv[u])) qp = QPair{qi, qj, si};
-                        else qp = QPair{qj, qi, sj};
-                    }
-                    on = visit<FORCE>(lds, si, (int)pv[u].w, r2, v, G2, C, tab, qp);
-                }
-                if (!on) continue;
-                if (!FORCE) {
-                    e += 0.5 * v;
-                } else {
-                    // atom i is the first atom when pick(i, j) holds: g_i = f1
-                    // with s = r_ij; otherwise g_i = -f1 with s = -r_ij
-                    double cs = C;
-                    if (pick && C != 0.0 && !pick_dev(idi, id[jv[u]], iv[u])) cs = -C;
-                    const double gx = G2 * d.x + cs, gy = G2 * d.y + cs, gz = G2 * d.z + cs;
-                    fx += gx; fy += gy; fz += gz;
-                    if (VIR) {
-                        w0 -= 0.5 * d.x * gx;
-                        w1 -= 0.5 * d.y * gy;
-                        w2 -= 0.5 * d.z * gz;
-                        w3 -= 0.5 * d.y * gz;
-                        w4 -= 0.5 * d.x * gz;
-                        w5 -= 0.5 * d.x * gy;
-                    }
-                }
+                one_pair(jv[u], iv[u], pv[u]);
             }
         }
     }
@@ -635,12 +686,12 @@ __global__ __launch_bounds__(PB) void k_pair_chi(int n, Geo geo, const double4 *
             const double r = sqrt(r2);
             const bool first = pick_dev(idi, id[j], img);
             const double qj = q[j];
-            const QPair qp = first ? QPair{qi, qj, si} : QPair{qj, qi, sj};
+            const QPair qp = first ? QPair{qi, qj, si, i, j, nullptr, 0} : QPair{qj, qi, sj, j, i, nullptr, 0};
             for (int c = 0; c < np; ++c) {
                 const GenPair &T = P.pair[si][sj][c];
                 if (!(T.cut > r)) continue;
                 double xs[2];
-                potential_chi(T, r, tab, P.cf, qp, xs);
+                potential_chi(T, r, tab, P, qp, xs);
                 const double s = first ? xs[0] : xs[1];
                 x += T.smooth ? s * fc64(r, T.cut, T.soft) : s;
             }
@@ -660,7 +711,7 @@ void launch(System &S, const Geo &geo, int mode, bool accumulate, double half_dt
     const int acc = accumulate ? 1 : 0;
     auto args = [&](auto kern) {
         kern<<<nb, PB, 0, S.stream>>>(S.n, geo, S.pos.p, S.id.p, S.nbr.p, S.nimg.p, S.ncnt.p,
-                                      S.dpmodel.p, S.tables.p, S.q.p, S.frc.p, acc, S.mom.p,
+                                      S.dpmodel.p, S.tables.p, S.q.p, S.qhalf.p, S.frc.p, acc, S.mom.p,
                                       half_dt, kick, S.gpartial.p);
     };
     if (mode == PAIR_ENERGY) args(k_pairs<Geo, PAIR_ENERGY, KIND, G>);
@@ -815,12 +866,25 @@ __global__ __launch_bounds__(PB) void k_bop_list(int n, Geo geo, const double4 *
     const double r2max = radius * radius * (1.0 + 1e-10);
     const int nf = ncnt[v];
     int c = 0;
-    for (int t = 0; t < nf; ++t) {
-        const int j = nbr[(size_t)t * N + v], img = nimg[(size_t)t * N + v];
-        if (!(dot64(separation64(pv, pos[j], img, cv)) < r2max)) continue;
-        osj[(size_t)c * N + v] = j;
-        osimg[(size_t)c * N + v] = img;
-        ++c;
+    constexpr int U = 8;   // entries in flight
+    for (int t0 = 0; t0 < nf; t0 += U) {
+        int jv[U], iv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const size_t at = (size_t)min(t0 + u, nf - 1) * N + v;
+            jv[u] = nbr[at];
+            iv[u] = nimg[at];
+        }
+        double4 p[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) p[u] = pos[jv[u]];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (t0 + u >= nf || !(dot64(separation64(pv, p[u], iv[u], cv)) < r2max)) continue;
+            osj[(size_t)c * N + v] = jv[u];
+            osimg[(size_t)c * N + v] = iv[u];
+            ++c;
+        }
     }
     oscnt[v] = c;
 }
@@ -860,6 +924,40 @@ __device__ __forceinline__ void bop_stage(BopStage<G> &st, int i, int n, int lan
     __syncthreads();
 }
 
+// The slots of a block's PB / G atoms counted through: offs[a] is the first
+// of atom a's, offs[PB / G] their number.  Threads that take the slots of the
+// block in turn are all busy but for the last wave, where G lanes an atom
+// leave a wave at the longest of its lists (silica: 8 slots an atom, 11 at
+// most, two turns of a wave for nearly every one).
+template <int G>
+__device__ __forceinline__ void bop_offsets(int *offs, int first, int n,
+                                            const int *__restrict__ oscnt)
+{
+    constexpr int A = PB / G;
+    static_assert(A <= 64, "one wave counts");
+    const int a = threadIdx.x;
+    if (a < 64) {
+        int c = a < A && first + a < n ? oscnt[first + a] : 0;
+#pragma unroll
+        for (int d = 1; d < A; d <<= 1) {
+            const int o = __shfl_up(c, d);
+            if (a >= d) c += o;
+        }
+        if (a == 0) offs[0] = 0;
+        if (a < A) offs[a + 1] = c;
+    }
+}
+// The atom of slot p: the last a with offs[a] <= p (p < offs[A])
+template <int G>
+__device__ __forceinline__ int bop_owner(const int *offs, int p)
+{
+    int a = 0;
+#pragma unroll
+    for (int d = PB / G / 2; d > 0; d >>= 1)
+        if (offs[a + d] <= p) a += d;
+    return a;
+}
+
 // Entry u of atom i's list: r_k - r_i, its length, the species of k.
 template <int G>
 __device__ __forceinline__ void bop_entry(const BopStage<G> &st, int u, int i, int a, size_t N,
@@ -882,7 +980,10 @@ __device__ __forceinline__ void bop_entry(const BopStage<G> &st, int u, int i, i
     }
 }
 
-// Pass 1: G lanes per atom, lane l takes the partner slots l, l + G, ...
+// Pass 1: a block's PB / G atoms; its threads take the partner slots of all
+// of them in turn (for the electronegativities, which are summed per atom, G
+// lanes take those of each).  24,576 atoms of COMB silica: 89 us
+// with G lanes for each atom and the powers of the charges inside, 51 now.
 template <class Geo, int MODE, int G>
 __global__ __launch_bounds__(PB) void k_bop_pairs(int n, Geo geo, const double4 *__restrict__ pos,
                                                   const int *__restrict__ id,
@@ -890,6 +991,7 @@ __global__ __launch_bounds__(PB) void k_bop_pairs(int n, Geo geo, const double4 
                                                   const PairModel *__restrict__ PM,
                                                   const double2 *__restrict__ tab,
                                                   const double *__restrict__ q,
+                                                  const double *__restrict__ qh,
                                                   const int *__restrict__ osj,
                                                   const int *__restrict__ osimg,
                                                   const int *__restrict__ oscnt,
@@ -901,20 +1003,25 @@ __global__ __launch_bounds__(PB) void k_bop_pairs(int n, Geo geo, const double4 
     constexpr bool CHI = MODE == BOP_CHI;
     __shared__ double red[PB];
     __shared__ BopStage<G> stg;
+    __shared__ int offs[PB / G + 1];
     const int blk = xcd_block(gridDim.x);
-    const int gid = blk * PB + threadIdx.x;
-    const int i = gid / G, lane = gid % G, a = threadIdx.x / G;
+    const int first_i = blk * (PB / G);
+    const int gi = first_i + threadIdx.x / G, lane = threadIdx.x % G;
     const size_t N = (size_t)n;
-    bop_stage<G>(stg, i, n, lane, a, geo, pos, osj, osimg, oscnt);
+    if (!CHI) bop_offsets<G>(offs, first_i, n, oscnt);
+    bop_stage<G>(stg, gi, n, lane, threadIdx.x / G, geo, pos, osj, osimg, oscnt);
     double e = 0.0, own = 0.0;
-    if (i < n) {
-        const double4 pi = pos[i];
-        const int si = (int)pi.w, idi = id[i];
-        const double qi = q[i];
-        const double *cv = geo.vec(i);
-        const double mb = BM->maxbond[si];
-        const int c = oscnt[i];
-        for (int t = lane; t < c; t += G) {
+    const int end = CHI ? (gi < n ? oscnt[gi] : 0) : offs[PB / G];
+    for (int p = CHI ? lane : threadIdx.x; p < end; p += CHI ? G : PB) {
+        {
+            const int a = CHI ? threadIdx.x / G : bop_owner<G>(offs, p);
+            const int i = first_i + a, t = CHI ? p : p - offs[a];
+            const double4 pi = pos[i];
+            const int si = (int)pi.w, idi = id[i];
+            const double qi = q[i];
+            const double *cv = geo.vec(i);
+            const double mb = BM->maxbond[si];
+            const int c = oscnt[i];
             const int j = osj[(size_t)t * N + i], img = osimg[(size_t)t * N + i];
             double3 d;
             double r;
@@ -953,16 +1060,16 @@ __global__ __launch_bounds__(PB) void k_bop_pairs(int n, Geo geo, const double4 
                 const double bt = pp.valid ? bo_post(zeta, pp) : zeta;
                 const bool first = pick_dev(idi, id[j], img);
                 const double qj = q[j];
-                const QPair qp = first ? QPair{qi, qj, si} : QPair{qj, qi, sj};
+                const QPair qp = first ? QPair{qi, qj, si, i, j, qh, N} : QPair{qj, qi, sj, j, i, qh, N};
                 const double fc = T.smooth ? fc64(r, T.cut, T.soft) : 1.0;
                 if (CHI) {
                     // potential_chi gives -dV/dq in the pair's orientation
                     double xs[2];
-                    potential_chi(T, r, tab, PM->cf, qp, xs);
+                    potential_chi(T, r, tab, *PM, qp, xs);
                     own += -0.5 * fc * bt * (first ? xs[0] : xs[1]);
                     D.w = -0.5 * fc * bt * (first ? xs[1] : xs[0]);
                 } else {
-                    const Radial pv = potential(T, r, tab, FORCE, PM->cf, qp);
+                    const Radial pv = potential(T, r, tab, FORCE, *PM, qp);
                     e += 0.5 * fc * pv.v * bt;
                     if (FORCE) {
                         // d(f_c V)/dr_ij = (G f_c + V f_c' / r) d: central (a
@@ -984,7 +1091,7 @@ __global__ __launch_bounds__(PB) void k_bop_pairs(int n, Geo geo, const double4 
     if (CHI) {
 #pragma unroll
         for (int o = G / 2; o > 0; o >>= 1) own += __shfl_xor(own, o);
-        if (i < n && lane == 0) oown[i] = own;
+        if (gi < n && lane == 0) oown[gi] = own;
         return;
     }
     if (MODE == PAIR_FORCES_ONLY) return;
@@ -998,9 +1105,10 @@ __global__ __launch_bounds__(PB) void k_bop_pairs(int n, Geo geo, const double4 
     if (tid < 8) partial[(size_t)(blk0 + blk) * 8 + tid] = tid == 0 ? red[0] : 0.0;
 }
 
-// Pass 2: G lanes per atom, lane l takes the slots t = l, l + G, ... as the
+// Pass 2: the threads of a block take the slots t of its PB / G atoms as the
 // third atom of every other bond of the atom; then the virial
-// -sum_t r_it (x) dU_i/dr_it.
+// -sum_t r_it (x) dU_i/dr_it.  24,576 atoms of COMB silica: 47 us
+// with G lanes for each atom, 32 in turn.
 template <class Geo, int MODE, int G>
 __global__ __launch_bounds__(PB) void k_bop_third(int n, Geo geo, const double4 *__restrict__ pos,
                                                   const BopModel *__restrict__ BM,
@@ -1014,19 +1122,24 @@ __global__ __launch_bounds__(PB) void k_bop_third(int n, Geo geo, const double4 
     constexpr bool VIR = MODE == PAIR_FORCES;
     __shared__ double red[6][PB];
     __shared__ BopStage<G> stg;
+    __shared__ int offs[PB / G + 1];
     const int blk = xcd_block(gridDim.x);
-    const int gid = blk * PB + threadIdx.x;
-    const int i = gid / G, lane = gid % G, a = threadIdx.x / G;
+    const int first_i = blk * (PB / G);
     const size_t N = (size_t)n;
-    bop_stage<G>(stg, i, n, lane, a, geo, pos, osj, osimg, oscnt);
+    bop_offsets<G>(offs, first_i, n, oscnt);
+    bop_stage<G>(stg, first_i + threadIdx.x / G, n, threadIdx.x % G, threadIdx.x / G, geo, pos,
+                 osj, osimg, oscnt);
     double w0 = 0.0, w1 = 0.0, w2 = 0.0, w3 = 0.0, w4 = 0.0, w5 = 0.0;
-    if (i < n) {
-        const double4 pi = pos[i];
-        const int si = (int)pi.w;
-        const double *cv = geo.vec(i);
-        const double mb = BM->maxbond[si];
-        const int c = oscnt[i];
-        for (int t = lane; t < c; t += G) {
+    const int end = offs[PB / G];
+    for (int p = threadIdx.x; p < end; p += PB) {
+        {
+            const int a = bop_owner<G>(offs, p);
+            const int i = first_i + a, t = p - offs[a];
+            const double4 pi = pos[i];
+            const int si = (int)pi.w;
+            const double *cv = geo.vec(i);
+            const double mb = BM->maxbond[si];
+            const int c = oscnt[i];
             double3 s2;
             double r2;
             int sk;
@@ -1164,7 +1277,14 @@ void pr_eval(System &S, int mode, bool accumulate, double half_dt, int kick)
     // the pair kernel: on streams of their own they share the chip with it,
     // which one of them alone leaves half idle at these sizes.  Serially while
     // the kernels are timed, and for systems that fill the chip.  20 steps of
-    // 24,576 atoms of COMB SiO2 and their state: 7.97 -> 7.30 ms.
+    // 24,576 atoms of COMB SiO2 and their state: 5.92 -> 5.42 ms.
+    const int halves = S.pmodel.nhalf;
+    if (halves > 0) {
+        S.qhalf.ensure((size_t)halves * S.n);
+        k_charge_halves<<<dim3(div_up(S.n, PB), halves), PB, 0, S.stream>>>(S.n, S.dpmodel.p,
+                                                                            S.q.p, S.qhalf.p);
+        HIP_TRY(hipGetLastError());
+    }
     const bool side = (bb || ob) && !S.timer.on && S.n <= PAIR_LANES_MAX_ATOMS;
     if (side) {
         sys_fork(S, 0, bb > 0);
@@ -1262,7 +1382,7 @@ void bop_sites(System &S, int mode, int blk0, hipStream_t stream)
         using Geo = decltype(geo);
         auto one = [&](auto kern) {
             kern<<<nb, PB, 0, stream>>>(n, geo, S.pos.p, S.id.p, S.dbmodel.p, S.dpmodel.p,
-                                        S.tables.p, S.q.p, S.osj.p, S.osimg.p, S.oscnt.p, S.oD.p,
+                                        S.tables.p, S.q.p, S.qhalf.p, S.osj.p, S.osimg.p, S.oscnt.p, S.oD.p,
                                         S.oW.p, S.oown.p, S.gpartial.p, blk0);
         };
         auto two = [&](auto kern) {
@@ -1308,8 +1428,8 @@ void bop_chi(System &S, double *chi)
     bop_prepare(S, S.stream);
     with_geo(S, [&](auto geo) {
         k_bop_pairs<decltype(geo), BOP_CHI, BOP_LANES><<<nb, PB, 0, S.stream>>>(
-            n, geo, S.pos.p, S.id.p, S.dbmodel.p, S.dpmodel.p, S.tables.p, S.q.p, S.osj.p,
-            S.osimg.p, S.oscnt.p, S.oD.p, S.oW.p, S.oown.p, nullptr, 0);
+            n, geo, S.pos.p, S.id.p, S.dbmodel.p, S.dpmodel.p, S.tables.p, S.q.p, nullptr,
+            S.osj.p, S.osimg.p, S.oscnt.p, S.oD.p, S.oW.p, S.oown.p, nullptr, 0);
     });
     HIP_TRY(hipGetLastError());
     k_bop_gather<BOP_LANES, true><<<nb, PB, 0, S.stream>>>(n, S.osj.p, S.osimg.p, S.oscnt.p,

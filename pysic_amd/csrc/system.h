@@ -122,6 +122,7 @@ struct System {
     // pair potentials of pair.hip and their tables
     PairModel pmodel{};
     DBuf<PairModel> dpmodel;
+    DBuf<double> qhalf;         // charge halves [nhalf][n] of the current charges
     DBuf<double2> tables;       // 'tabulated' rows (value, derivative), all tables
     DBuf<double> gpartial;      // per-block energy + virial partials of pair.hip
     int gpartial_blocks = 0;
