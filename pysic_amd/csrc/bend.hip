@@ -11,8 +11,8 @@
 // when pick(v, a) holds (targets matched as (v, a, b)), else from (a, v)
 // (targets matched as (a, v, b)).
 //
-// Here each vertex v gets a short list of its neighbors within the largest
-// bend cutoff, then G lanes: each lane takes some of the legs and, for each,
+// Here each vertex v gets a short list of the neighbors that can take part
+// in an angle at it, or it at them, then G lanes: each lane takes some of the legs and, for each,
 // every angle it forms with another leg, oriented and matched against the
 // rows as the reference does it.  The force on a leg's atom is stored per
 // short-list slot and summed by that atom's own thread afterwards, with the

@@ -127,8 +127,8 @@ struct System {
     DBuf<double> gpartial;      // per-block energy + virial partials of pair.hip
     int gpartial_blocks = 0;
     DBuf<double> gtotals;       // reduced energy + virial (7 doubles)
-    // bond_bend: each vertex's neighbors within the largest bend cutoff
-    // (column-major, capacity cap, as the full lists) and the forces its
+    // bond_bend: each vertex's neighbors that can take part in its angles, or
+    // it in theirs (column-major, capacity cap, as the full lists) and the forces its
     // angles put on them
     DBuf<int> bsj, bsimg, bscnt;
     DBuf<double4> bG;
