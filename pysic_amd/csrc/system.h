@@ -101,6 +101,8 @@ struct System {
     int cap = 0;
     int nb_method = 0;          // 0 auto (= 5), 1 global scan, 2 LDS bricks, 3 bricks w/o LDS room,
                                 // 4 lane groups, 5 FP32-prefiltered scan
+    DBuf<int> nwrap;        // per atom: some list entry is in another image than 0
+    bool nwrap_on = false;  // nwrap belongs to the lists (else any entry may be)
     DBuf<int> nbr, nimg, ncnt;
     DBuf<int> flags;            // [0] max list length, [1] max short length, [2] wrap range, [3] unpaired bond
 

@@ -121,3 +121,39 @@ def test_relaxation_that_diverges_is_reported(eng, n):
     got, _, k, _ = eng.relax_charges(q0, v0, 2, 0.05, 1.0, 4.0, 1e-9)
     q, _, _, _, _ = _driven(eng, q0, v0, 2, 0.05, 4.0, 1e-9)
     assert k == 2 and rel_maxnorm(got, q) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [864, 137388])
+def test_image_words_follow_the_list_build(eng, n):
+    """The Lennard-Jones kernels skip the image words of waves whose entries
+    are all in the atom's own image, which only the lane-parallel build
+    records: after any order of builds, and after dynamics, the forces are
+    those of lists built atom by atom, bit for bit (up to 131,072 atoms the
+    lanes sum in the list's order, which is the same)."""
+    print("case: images n=%d" % n, flush=True)
+    m = round((n / 4) ** (1.0 / 3.0))
+    s = st.fcc((m, m, m), a=5.4, sigma=0.1, seed=6)
+    assert len(s) == 4 * m ** 3
+    n = len(s)
+    pd, _, _ = build_descriptors([Potential("LJ", symbols=[["Ar", "Ar"]], parameters=[0.01, 3.4],
+                                            cutoff=6.4)], {"Ar": 0})
+    st.maxwell_boltzmann(s, 60.0, 2)
+    eng.create_atoms(np.zeros(n, np.int32), s.positions, masses=s.masses, momenta=s.momenta)
+    eng.create_cell(s.cell, (True, True, True))
+    eng.set_potentials(pd)
+    eng.set_bond_order_factors(np.zeros((0, 14)))
+    eng.ewald_off()
+
+    def forces(method):
+        eng.set_neighbor_method(method)
+        eng.generate_neighbor_lists(np.full(n, 6.6))
+        return eng.forces()[0]
+    want = forces(1)
+    for method in (0, 1, 4, 0):
+        assert np.array_equal(forces(method), want)
+    for method in (0, 1, 0, 1):      # steps replayed from graphs, then lists of both kinds
+        forces(method)
+        eng.md_run(4, 0.5)
+        f = eng.forces()[0]
+        assert np.array_equal(forces(1), f) and np.array_equal(forces(0), f)
+    eng.set_neighbor_method(0)
