@@ -353,10 +353,10 @@ def ewald_benchmark(reps=3, ref_reps=(4, 4, 4)):
     nk = int(((k2 < EWALD_KC ** 2) & (k2 > 0)).sum())
     sk_us = tim.get("ewald_sk", (0.0, 1))
     sk_avg = sk_us[0] / max(sk_us[1], 1) / 1e3
-    # algorithmic work of one structure-factor pass: per (k, ion) one complex
-    # multiply-accumulate, 4 FMAs = 8 FP64 flops (the phase generation, one
-    # sincos per 16 k, is not counted)
-    flops = 8.0 * nk * n
+    # algorithmic work of one structure-factor pass over the mesh: each ion's
+    # charge goes to 16^3 mesh points, one FMA (2 FP64 flops) each; the
+    # transforms, placing the ions and their kernel values are not counted
+    flops = 2.0 * 16 ** 3 * n
     out = {"workload": "rocksalt 32^3 cells, 262,144 ions, sigma 0.08 A, Ewald rc 10 A "
                        "sigma 2.0443 A kc 2.5713 1/A (1e-6), FP64",
            "ions": n, "k_vectors_half_space": nk, "evaluation": "energy + forces + stress",
@@ -445,8 +445,9 @@ def lj_benchmark(steps=100, warmup=10, ref_cells=6, reference=True):
     pf_ms, pf_calls = tim.get("pair_forces", (0.0, 1))
     pf_s = pf_ms / max(pf_calls, 1) / 1e3
     # algorithmic bytes of one forces launch per atom: position 32, list
-    # entries 8 each (j + image), momentum read + write 64, force write 32
-    bytes_launch = (128.0 + 8.0 * n_list) * n
+    # entries 4 each (j; image words are read near the cell's faces only),
+    # momentum read + write 64, force write 32
+    bytes_launch = (128.0 + 4.0 * n_list) * n
     out = {"workload": "LJ argon fcc 64^3 cells, 1,048,576 atoms, rc 2.5 sigma = 8.51 A, "
                        "skin 0.5 A, lists rebuilt every 10 steps, VV dt = 2 fs, 80 K, FP64",
            "atoms": n, "list_entries_per_atom": round(n_list, 2), "steps": steps,
