@@ -1455,9 +1455,12 @@ void ewald_relax(System &S, const EwaldParams &P, EwaldState &E, double *rates, 
             if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         k_clear_stop<<<1, 64, 0, S.stream>>>(E.stop.p);
         auto queue = [&](int k) {
+            // the first step is taken on the loop's own condition, which the
+            // starting charges' error has no part in
+            const bool more = k < n_steps && (k > 0 || 2.0 * tolerance > tolerance);
             chi_eval(S, P, E, k > 0, k > 0);
             k_relax_tail<<<1, 1024, 0, S.stream>>>(n, E.chi.p, S.q.p, rates, E.scaler.p, k == 0,
-                                                   k < n_steps, dt, inv_mq, friction, future,
+                                                   more, dt, inv_mq, friction, future,
                                                    tolerance, E.stop.p, E.red.p, mail + (k & 1));
             HIP_TRY(hipGetLastError());
             HIP_TRY(hipEventRecord(E.seen[k & 1], S.stream));

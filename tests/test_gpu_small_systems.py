@@ -111,6 +111,23 @@ def test_relaxation_steps_and_stops(eng, n):
         assert rel_maxnorm(got, q) <= 1e-12 and np.abs(rate - v).max() <= 1e-12
 
 
+@pytest.mark.parametrize("tol", [0.0, -1e-9, float("nan"), float("inf")])
+@pytest.mark.parametrize("n", [2, 8192, 8193])
+def test_relaxation_that_is_not_entered(eng, n, tol):
+    """The loop is entered while twice the tolerance is above the tolerance:
+    with one that is zero, negative, infinite or not a number nothing moves."""
+    print("case: relaxation n=%d tolerance %r" % (n, tol), flush=True)
+    q0, v0 = _relaxation_case(eng, n)
+    got, rate, k, e = eng.relax_charges(q0, v0, 5, 0.05, 1.0, 4.0, tol)
+    assert k == 0
+    assert np.array_equal(got, q0) and np.array_equal(rate, v0)
+    assert np.array_equal(e, 2.0 * tol, equal_nan=True)
+    # and the device's own copies are the caller's as well
+    x = eng.electronegativities()
+    eng.update_charges(q0)
+    assert np.array_equal(eng.electronegativities(), x)
+
+
 @pytest.mark.parametrize("n", [1023, 8193])
 def test_relaxation_that_diverges_is_reported(eng, n):
     print("case: diverging relaxation n=%d" % n, flush=True)
