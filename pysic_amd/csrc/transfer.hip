@@ -41,7 +41,9 @@ constexpr size_t KEEP_BLOCKS = 16, KEEP_SLOTS = 2 * HostLink::PAIRS;
 static_assert(MAIL_WORDS * sizeof(double) <= 1024, "the mail fits its part of the block");
 
 // What is kept, for all systems and threads of the process.  Pinned portably:
-// any device may use it next.
+// any device may use it next.  Coherent by its own flag, whatever the process
+// sets as the default: the host reads rows and error words after an event,
+// which need not flush a device's caches to memory of the other kind.
 struct Pinned {
     std::mutex m;
     long users = 0;
@@ -50,7 +52,7 @@ struct Pinned {
     static char *fresh(size_t bytes)
     {
         char *p = nullptr;
-        HIP_TRY(hipHostMalloc((void **)&p, bytes, hipHostMallocPortable));
+        HIP_TRY(hipHostMalloc((void **)&p, bytes, hipHostMallocPortable | hipHostMallocCoherent));
         return p;
     }
     char *take(std::vector<char *> &v, size_t bytes)

@@ -2,7 +2,11 @@
 bit for bit, in the caller's order, at the sizes where the way changes (the
 small slots hold 10,922 rows of 3 or 32,768 scalars; the large ones 131,072
 rows of 3 or 393,216 scalars, in chunks over several threads), and with
-several handles moving data at once."""
+several handles moving data at once, and whatever the process sets as the
+default kind of pinned memory."""
+import os
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -75,3 +79,33 @@ def test_handles_on_several_threads():
     for t in threads:
         t.join()
     assert not failed, failed
+
+
+@pytest.mark.parametrize("coherent", ["0", "1"])
+def test_default_kind_of_pinned_memory(coherent):
+    """The rows of the large downloads and the errors that end a relaxation
+    are read after events: they need coherent memory, also in a process
+    whose default is the other kind."""
+    code = """
+import numpy as np
+import test_gpu_small_systems as small
+import test_gpu_transfer as t
+t.roundtrip(1000003, 3)
+print("rows arrive", flush=True)
+eng = small.Engine(0)
+q0, v0 = small._relaxation_case(eng, 1500)
+q, v, steps, err, errs = small._driven(eng, q0, v0, 200, 0.05, 4.0, 1e-6)
+for _ in range(3):
+    got, rate, k, e = eng.relax_charges(q0, v0, 200, 0.05, 1.0, 4.0, 1e-6)
+    assert k == steps and 3 < k < 200, (k, steps)
+    assert abs(e - err) <= 1e-3 * abs(err) and np.abs(got - q).max() <= 1e-10
+eng.close()
+print("errors arrive", flush=True)
+"""
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = "import sys; sys.path[:0] = [%r, %r]\nfrom pysic_amd.engine import Engine\n" % (
+        here, os.path.dirname(here)) + code.replace("small.Engine", "Engine")
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=110,
+                         env=dict(os.environ, HIP_HOST_COHERENT=coherent))
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert "errors arrive" in out.stdout
