@@ -18,8 +18,10 @@ struct EwaldParams {
 struct MeshState {
     int n[3] = {0, 0, 0}, K[3] = {0, 0, 0}, nb[3] = {0, 0, 0}, nbins = 0, nepart = 0;
     int fmt[3], fst[3], imt[3], ist[3];   // tiles and steps of the transforms, per axis
-    DBuf<double> ftab[3], itab[3];        // their operand tables
-    DBuf<double> dec, coef;               // kernel transforms, k-vector coefficients
+    bool tables = false;                  // tab is that of n and K
+    DBuf<double> tab;                     // operand tables, reciprocal kernel transforms
+    size_t fat[3], iat[3], dat;           // where in tab: forward, inverse, transforms
+    DBuf<double> coef;                    // k-vector coefficients
     DBuf<double> bufa, bufb, oct;         // mesh, half-transformed mesh, octant
     DBuf<int> count, fill, start, bin, claim, order;
     DBuf<int4> at;                        // window origin and slot, tile order

@@ -1075,10 +1075,11 @@ void prepare(System &S, const EwaldParams &P, EwaldState &E)
         E.nk = (int)kv.size();
         E.kvec.ensure(kv.size());
         E.sk.ensure(kv.size());
-        if (!kv.empty())
+        if (!kv.empty()) {
             HIP_TRY(hipMemcpyAsync(E.kvec.p, kv.data(), sizeof(double4) * kv.size(),
                                    hipMemcpyHostToDevice, S.stream));
-        HIP_TRY(hipStreamSynchronize(S.stream));   // before the host vectors go
+            HIP_TRY(hipStreamSynchronize(S.stream));   // before the host vectors go
+        }
         E.dirty = false;
     }
     // scaler in the current atom order
