@@ -71,11 +71,13 @@ struct EwaldState {
     int skchunks = 0;
 };
 
-// Pairs of an ion and a k-vector from which the mesh is the faster way: both
-// ways take the same time for about 6,000 ions at 1e-6 accuracy (mesh.hip).
+// Pairs of an ion and a k-vector from which the mesh may be the faster way: both
+// take the same time for 4,096 ions at 1e-6 accuracy (energy + forces 0.51 ms
+// direct, 0.53 mesh; 8,000 ions 0.67 and 0.57).
 constexpr double MESH_MIN_PAIRS = 1e8;
-// Whether a system's reciprocal sums should go over the mesh.
-bool mesh_suits(int natoms, const EwaldParams &P, const CellGeom &c, double volume);
+// Whether the system's reciprocal sums should go over the mesh; counts where the
+// ions are (in M's sort buffers, and waits) if its sizes do not settle it.
+bool mesh_suits(System &S, const EwaldParams &P, MeshState &M, const double *f, double volume);
 // Sizes, tables and coefficients; b: reciprocal vectors (rows).
 void mesh_plan(System &S, const EwaldParams &P, MeshState &M, const double *b, double inv_eps_2v);
 // Sorts the atoms by tile and forms their kernel values; f: inverse cell rows.

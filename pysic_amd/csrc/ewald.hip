@@ -1011,7 +1011,6 @@ void prepare(System &S, const EwaldParams &P, EwaldState &E)
     if (E.dirty) {
         E.sk_valid = false;
         E.planned_n = n;
-        E.mesh_on = mesh_suits(n, P, S.geom, E.volume);
         // k-vectors in the reference's loop order (Potentials.f90:1526-1548)
         const double pi = 4.0 * std::atan(1.0);
         double rcl[9];
@@ -1023,6 +1022,7 @@ void prepare(System &S, const EwaldParams &P, EwaldState &E)
         }
         PYSIC_REQUIRE(P.K[0] < 1024 && P.K[1] < 1024 && P.K[2] < 1024, PYSIC_EINVAL,
                       "at most 1023 reciprocal cells along each axis");
+        E.mesh_on = mesh_suits(S, P, E.mesh, E.f, E.volume);
         if (E.mesh_on) mesh_plan(S, P, E.mesh, E.b, c.inv_eps_2v);
         double kc2 = P.kc * P.kc;
         std::vector<double4> kv;
@@ -1114,7 +1114,12 @@ void structure_factors(System &S, EwaldState &E, bool placed = false)
     if (E.mesh_on) {
         hipEvent_t ev;
         S.timer.begin("ewald_sk", S.stream, &ev);
-        if (!placed) mesh_place(S, E.mesh, E.f);
+        if (!placed) {
+            hipEvent_t at;
+            S.timer.begin("ewald_mesh_place", S.stream, &at);
+            mesh_place(S, E.mesh, E.f);
+            S.timer.end("ewald_mesh_place", S.stream, at);
+        }
         mesh_structure(S, E.mesh, E.f, E.scaler.p);
         S.timer.end("ewald_sk", S.stream, ev);
         return;

@@ -21,9 +21,8 @@
 // Measured, energy + forces of 262,144 ions, 852,533 k-vectors, mesh 304^3:
 // the reciprocal part takes 2.2 ms where the direct sums take 125 ms; one
 // electronegativity evaluation of 24,576 ions (mesh 128 x 120 x 120) 0.16 ms
-// against 0.84 ms.  The direct sums stay below 1e8 pairs of an ion and a
-// k-vector, where their few launches cost less (energy + forces of 4,096
-// ions: 0.51 ms direct, 0.53 ms mesh; of 8,000: 0.67 and 0.57).
+// against 0.84 ms.  The direct sums stay where they cost less (mesh_suits):
+// few ions or k-vectors, and ions crowded into few mesh tiles.
 //
 //  k_mesh_bin/scan/fill/order  counting sort of the atoms by mesh tile
 //  k_mesh_weights              kernel values (and derivatives) per atom, axis
@@ -186,8 +185,17 @@ __global__ __launch_bounds__(MB) void k_mesh_weights(int n, MeshGeo g,
     }
 }
 
-// The atoms whose windows meet tile (tx, ty, tz): those of the 2 x 3 x 3
-// bins ending at it.  Lane s < 18 holds bin s; base[s] is the first stream
+// Bin s of the 2 x 3 x 3 that end at tile (tx, ty, tz).
+__device__ __forceinline__ int stream_bin(const MeshGeo &g, int tx, int ty, int tz, int s)
+{
+    int bx = tx - (s & 1), by = ty - (s >> 1) % 3, bz = tz - (s >> 1) / 3;
+    bx += bx < 0 ? g.nb[0] : 0;
+    by += by < 0 ? g.nb[1] : 0;
+    bz += bz < 0 ? g.nb[2] : 0;
+    return bx + g.nb[0] * (by + g.nb[1] * bz);
+}
+
+// The atoms whose windows meet tile (tx, ty, tz): those of its 18 bins.  Lane s < 18 holds bin s; base[s] is the first stream
 // position of bin s, base[18] the total.
 __device__ __forceinline__ void tile_stream(const MeshGeo &g, int tx, int ty, int tz,
                                             const int *__restrict__ start, int *first, int *base)
@@ -195,11 +203,7 @@ __device__ __forceinline__ void tile_stream(const MeshGeo &g, int tx, int ty, in
     const int s = threadIdx.x;
     int len = 0, a = 0;
     if (s < SLOTS) {
-        int bx = tx - (s & 1), by = ty - (s >> 1) % 3, bz = tz - (s >> 1) / 3;
-        bx += bx < 0 ? g.nb[0] : 0;
-        by += by < 0 ? g.nb[1] : 0;
-        bz += bz < 0 ? g.nb[2] : 0;
-        const int b = bx + g.nb[0] * (by + g.nb[1] * bz);
+        const int b = stream_bin(g, tx, ty, tz, s);
         a = start[b];
         len = start[b + 1] - a;
     }
@@ -787,6 +791,22 @@ __global__ __launch_bounds__(MB) void k_mesh_finish(int n, MeshGeo g,
     if (threadIdx.x < 6) bpart[(size_t)blockIdx.x * 8 + threadIdx.x] = red[0][threadIdx.x];
 }
 
+// The most ions that one tile meets (those of its 18 bins), into peak.
+__global__ __launch_bounds__(MB) void k_mesh_crowd(MeshGeo g, int nbins,
+                                                   const int *__restrict__ count,
+                                                   int *__restrict__ peak)
+{
+    const int t = blockIdx.x * MB + threadIdx.x;
+    int sum = 0;
+    if (t < nbins) {
+        const int tx = t % g.nb[0], ty = t / g.nb[0] % g.nb[1], tz = t / (g.nb[0] * g.nb[1]);
+        for (int s = 0; s < SLOTS; ++s) sum += count[stream_bin(g, tx, ty, tz, s)];
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) sum = max(sum, __shfl_xor(sum, d));
+    if ((threadIdx.x & 63) == 0) atomicMax(peak, sum);
+}
+
 __global__ void k_mesh_zero(int m, int *__restrict__ a)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -796,6 +816,14 @@ __global__ void k_mesh_zero(int m, int *__restrict__ a)
 // ---- host side ----------------------------------------------------------------
 
 int round_up(int x, int m) { return (x + m - 1) / m * m; }
+
+// mesh points of axis d for k-vectors up to K: whole tiles, and enough of them
+// that a window meets none twice
+int mesh_points(int K, int d)
+{
+    const int least[3] = {2 * TX, 3 * TY, 3 * TZ}, tile[3] = {TX, TY, TZ};
+    return round_up(std::max(4 * K + 4, least[d]), tile[d]);
+}
 
 // ints that k_mesh_scan reads for nbins counts: whole int4 for 1024 threads
 int scan_room(int nbins) { return round_up(nbins, 4096); }
@@ -943,23 +971,59 @@ void transform(System &S, const MeshState &M, int axis, bool forward, int arrays
 
 }  // namespace
 
-bool mesh_suits(int natoms, const EwaldParams &P, const CellGeom &c, double volume)
+// The choice is by cost, both sides' times (µs) of S(k) and one pass over the
+// atoms as sums of what they grow with.  Fitted to 90 systems of 100 to 262,144
+// ions and K = 6 to 74 in cubes, slabs and rods: within 20% of most of what was
+// measured, within 30% of all.
+//   direct: launches, k-vectors, pairs, ions (phases);
+//   mesh:   launches, points (the transforms), and the ions: a tile is one
+//           wave's, so the longest chain of a tile or, with tiles for the whole
+//           chip, all ions.
+// Measured, direct and mesh: 262,144 ions, K = 20: 3755 and 2022 µs; K = 14
+// (18,400 ions a tile): 1771 and 4876; 64,000 in an eighth of a cell, K = 14:
+// 484 and 7552; in a cell of 304^3 points 500 ions 425 and 675, 2,000 904 and
+// 715.  Below MESH_MIN_PAIRS neither is ahead by more than a launch or two.
+bool mesh_suits(System &S, const EwaldParams &P, MeshState &M, const double *f, double volume)
 {
     // k-vectors of the half space: half a sphere's worth, at most the box
-    const double pi = 4.0 * std::atan(1.0);
+    const double pi = 4.0 * std::atan(1.0), n = S.n;
+    const int tile[3] = {TX, TY, TZ};
+    MeshGeo g;
     double box = 1.0, points = 1.0, lowest = P.kc;
     for (int d = 0; d < 3; ++d) {
+        g.n[d] = mesh_points(P.K[d], d);
+        g.nb[d] = g.n[d] / tile[d];
         box *= d == 2 ? P.K[d] + 1 : 2 * P.K[d] + 1;
-        points *= round_up(std::max(4 * P.K[d] + 4, 32), TX);
-        const double *v = c.v + 3 * d;
+        points *= g.n[d];
+        const double *v = S.geom.v + 3 * d;
         const double len = std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
         lowest = std::min(lowest, 2.0 * pi * P.K[d] / len);
     }
+    for (int c = 0; c < 9; ++c) g.f[c] = f[c];
     const double nk = std::min(box, volume * P.kc * P.kc * P.kc / (12.0 * pi * pi));
-    // The kernel's aliasing error grows to 3e-12 of a term at the mesh's band
-    // edge (it is 1e-16 at small k), so the sum has to have decayed there.
+    // The kernel's aliasing error grows to 2e-11 of a term at the mesh's band
+    // edge (it is 6e-17 at half of it), so the sum has to have decayed there.
     const bool decayed = std::exp(-0.5 * P.sigma * P.sigma * lowest * lowest) <= 1e-4;
-    return decayed && (double)natoms * nk >= MESH_MIN_PAIRS && points <= 268435456.0;
+    if (!decayed || !(n * nk >= MESH_MIN_PAIRS) || points > 268435456.0) return false;
+    const double direct = 75.0 + 2e-4 * nk + 4.2e-7 * n * nk + 5e-3 * n;
+    auto mesh = [&](double met) {   // ions that the most crowded tile meets
+        return 60.0 + 2e-5 * points + std::max(0.25 * met, 3.3e-3 * n);
+    };
+    const int nbins = g.nb[0] * g.nb[1] * g.nb[2];
+    if (mesh(SLOTS * n / nbins) >= direct) return false;
+    // where the ions are decides, counted once for each plan
+    M.bin.ensure(S.n);
+    M.count.ensure(scan_room(nbins));
+    M.start.ensure(scan_room(nbins) + 1);
+    k_mesh_zero<<<div_up(nbins, 256), 256, 0, S.stream>>>(nbins, M.count.p);
+    k_mesh_zero<<<1, 64, 0, S.stream>>>(1, M.start.p);
+    k_mesh_bin<<<div_up(S.n, MB), MB, 0, S.stream>>>(S.n, g, S.pos.p, M.bin.p, M.count.p);
+    k_mesh_crowd<<<div_up(nbins, MB), MB, 0, S.stream>>>(g, nbins, M.count.p, M.start.p);
+    HIP_TRY(hipGetLastError());
+    int met = 0;
+    HIP_TRY(hipMemcpyAsync(&met, M.start.p, sizeof(int), hipMemcpyDeviceToHost, S.stream));
+    HIP_TRY(hipStreamSynchronize(S.stream));
+    return mesh(met) < direct;
 }
 
 // The operand tables and kernel transforms of M.n and M.K, in one upload: equal
@@ -1001,15 +1065,15 @@ static void mesh_tables(System &S, MeshState &M)
 
 void mesh_plan(System &S, const EwaldParams &P, MeshState &M, const double *b, double inv_eps_2v)
 {
-    const int least[3] = {2 * TX, 3 * TY, 3 * TZ}, tile[3] = {TX, TY, TZ};
+    const int tile[3] = {TX, TY, TZ};
     // A new cell with the same k-vector counts (each step of a relaxation of
     // the cell) keeps the tables and runs k_mesh_coef alone.  Energy and forces
-    // in a new cell, 8,000 ions: 1.44 ms with the tables formed again, 0.52 so
+    // in a new cell, 8,000 ions: 1.44 ms with the tables formed again, 0.55 so
     // (1.24 by the direct sums before; in the same cell 0.45).
     bool same = M.tables;
     M.tables = false;
     for (int d = 0; d < 3; ++d) {
-        const int n = round_up(std::max(4 * P.K[d] + 4, least[d]), tile[d]);
+        const int n = mesh_points(P.K[d], d);
         same = same && M.K[d] == P.K[d] && M.n[d] == n;
         M.K[d] = P.K[d];
         M.n[d] = n;

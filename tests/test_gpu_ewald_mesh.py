@@ -1,5 +1,6 @@
 """GPU parity of the reciprocal sums over the mesh (mesh.hip), which take over
-from the ion-by-ion sums at 1e8 pairs of an ion and a k-vector.
+from the ion-by-ion sums where they cost less, and the choice between the two
+(read back from the kernel families that were timed).
 
 Reference: the oracle for everything but the reciprocal terms (it is given no
 reciprocal cells), plus the reciprocal sums term by term in numpy's FP64
@@ -91,7 +92,23 @@ CASES = [
     dict(n=3001, cell=(40.0, 40.0, 40.0), part=(0.3, 0.35, 0.4), kc=4.6, seed=4),
     # a flat cell: the smallest mesh an axis can have (24 points)
     dict(n=8000, cell=(68.0, 64.0, 7.0), kc=5.0, seed=5),
+    # some 45 ions in each tile of a corner, none in the others
+    dict(n=12000, cell=(60.0, 60.0, 60.0), part=(0.3, 0.35, 0.4), kc=4.6, seed=6),
+    # the sum has barely decayed at the mesh's band edge: 1.0e-4 there
+    dict(n=3000, cell=(36.0, 36.0, 36.0), kc=5.0, seed=7, sigma=4.292 / 5.0),
 ]
+# everything in one corner of a smaller cell: the crowded tiles cost more
+DIRECT = {3}
+
+
+def went_over_the_mesh(eng, call):
+    """Whether the reciprocal sums of call() went over the mesh."""
+    eng.timing(True)
+    call()
+    families = eng.timing_read()
+    eng.timing(False)
+    assert "ewald_sk" in families
+    return "ewald_mesh_place" in families
 
 
 @pytest.mark.parametrize("k", range(len(CASES)))
@@ -99,7 +116,7 @@ def test_mesh_matches_term_by_term(oracle, k):
     from pysic_amd.engine import Engine
     case = CASES[k]
     pos, q, cell, scaler = ions(case)
-    n, kc, sigma, rc = len(pos), case["kc"], 1.2, 3.0
+    n, kc, sigma, rc = len(pos), case["kc"], case.get("sigma", 1.2), 3.0
     K = kcells(cell, kc)
     print("mesh case %d: n=%d K=%s" % (k, n, K), flush=True)
     sp = np.zeros(n, np.int32)
@@ -141,6 +158,7 @@ def test_mesh_matches_term_by_term(oracle, k):
     moved = pos + np.random.default_rng(9).normal(0.0, 0.02, pos.shape)
     eng.update_coordinates(moved)
     compare(moved, "fex")
+    assert went_over_the_mesh(eng, eng.electronegativities) == (k not in DIRECT)
     eng.close()
 
 
@@ -176,6 +194,7 @@ def test_relaxation_steps_over_the_mesh():
         f = force()
         v = (v + 0.5 * f * dt) / (1 + 0.5 * fr * dt)
     assert rel_maxnorm(got, q) <= TOL and rel_maxnorm(rate, v) <= TOL
+    assert went_over_the_mesh(eng, eng.electronegativities)
     eng.close()
 
 
@@ -208,7 +227,7 @@ def test_tables_follow_the_cell():
     q = np.random.default_rng(5).choice([-1.0, 1.0], n)
     cube = np.eye(3) * 36.0
     strain = np.array([[1.001, 0.002, 0.0], [0.0, 0.999, 0.001], [0.0, 0.0, 1.0005]])
-    eng, seen = None, set()
+    eng, seen, way = None, set(), set()
     for k, cell in enumerate((cube, cube @ strain, cube @ strain @ strain, np.diag([60.0, 30.0, 15.0]),
                               np.diag([30.0, 15.0, 60.0]), cube * 0.9, cube)):
         pos = u @ cell
@@ -225,15 +244,17 @@ def test_tables_follow_the_cell():
         for a, b in zip(eng.forces(), fresh.forces()):
             assert np.array_equal(a, b)
         assert np.array_equal(eng.electronegativities(), fresh.electronegativities())
+        way.add(went_over_the_mesh(eng, eng.electronegativities))
         fresh.close()
     assert len(seen) == 4   # the strained cubes have the cube's counts
+    assert way == {True}
     eng.close()
 
 
 def test_first_evaluation_in_a_new_cell_is_quick():
     """A strained cell with the same k-vector counts, as every step of a cell
     relaxation brings: its first evaluation takes at most 0.4 ms more than a
-    repeated one (8,000 ions: 0.07; forming the tables again took 1.0)."""
+    repeated one (8,000 ions: 0.12; forming the tables again took 1.0)."""
     import time
     from pysic_amd import structures as st
     s = st.rocksalt((10, 10, 10), sigma=0.08, seed=3)
@@ -251,7 +272,78 @@ def test_first_evaluation_in_a_new_cell_is_quick():
         eng.energy()
         eng.forces()
         times[new].append(time.perf_counter() - t)
+    assert went_over_the_mesh(eng, eng.electronegativities)
     extra = 1e6 * (np.median(times[True][2:]) - np.median(times[False][2:]))
     print("a new cell: %.0f us more" % extra, flush=True)
     assert extra <= 400.0
+    eng.close()
+
+
+# the choice: (ions, cell edges, part of the cell they fill, k_c, sigma, mesh)
+CHOICE = [
+    (8000, (56.4,) * 3, (1, 1, 1), 2.5713, 2.0443, True),
+    (4096, (45.1,) * 3, (1, 1, 1), 2.5713, 2.0443, False),     # few pairs
+    (500, (180.5,) * 3, (0.25, 0.25, 0.05), 2.5713, 2.0443, False),   # mesh for few ions
+    (4000, (100.0,) * 3, (1, 1, 0.2), 2.5713, 2.0443, True),   # a slab worth its mesh
+    (262144, (180.5,) * 3, (1, 1, 1), 0.5, 10.0, False),       # a thousand ions a tile
+    (32000, (200.0,) * 3, (0.2, 0.2, 0.2), 1.3, 3.6, False),   # a particle: crowded tiles
+    (32000, (200.0,) * 3, (1, 1, 1), 1.3, 3.6, True),          # the same ions spread out
+    (8000, (56.4,) * 3, (1, 1, 1), 2.5713, 1.6, False),        # not decayed: 2e-4
+]
+
+
+def _ions_of(n, edge, part):
+    rng = np.random.default_rng(n)
+    m = int(np.ceil(n ** (1 / 3) - 1e-9))
+    site = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    u = (site + 0.5 + 0.3 * (rng.random((n, 3)) - 0.5)) / m * np.array(part)
+    return u * np.array(edge), rng.choice([-1.0, 1.0], n)
+
+
+@pytest.mark.parametrize("k", range(len(CHOICE)))
+def test_the_cheaper_way_is_taken(k):
+    n, edge, part, kc, sigma, mesh = CHOICE[k]
+    print("choice %d: n=%d" % (k, n), flush=True)
+    pos, q = _ions_of(n, edge, part)
+    eng = _engine(pos, q, np.diag(edge), kc, sigma, 5.0)
+    assert went_over_the_mesh(eng, eng.electronegativities) == mesh
+    eng.close()
+
+
+def test_one_handle_changes_its_way(oracle):
+    """Through new cells and atom counts from the direct sums to the mesh and
+    back, each time what a new handle gives, bit for bit; the reciprocal parts
+    of a mesh and a direct evaluation against the sums term by term."""
+    steps = [(2000, 30.0, False), (3000, 36.0, True), (2999, 36.0, True), (3000, 30.0, False),
+             (1500, 36.0, False), (3000, 36.0, True)]
+    eng = None
+    for n, edge, mesh in steps:
+        print("step n=%d edge=%g" % (n, edge), flush=True)
+        pos, q = _ions_of(n, (edge,) * 3, (1, 1, 1))
+        cell = np.eye(3) * edge
+        fresh = _engine(pos, q, cell, 5.0)
+        if eng is None:
+            eng = _engine(pos, q, cell, 5.0)
+        elif n != eng_n:
+            eng.create_atoms(np.zeros(n, np.int32), pos, charges=q)
+            _new_cell(eng, pos, cell, 5.0)
+        else:
+            eng.update_charges(q)
+            _new_cell(eng, pos, cell, 5.0)
+        eng_n = n
+        for e in (eng, fresh):   # both from their own sorted order
+            e.generate_neighbor_lists(np.full(n, 3.2))
+        got = eng.energy(), eng.forces()[0], eng.electronegativities()
+        want = fresh.energy(), fresh.forces()[0], fresh.electronegativities()
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
+        assert went_over_the_mesh(eng, eng.electronegativities) == mesh
+        nl = oracle.neighbor_list(pos, cell, [1, 1, 1], np.full(n, 3.2))
+        args = (np.zeros(n, np.int32), pos, q, cell, nl, np.zeros((0, 12)), None,
+                [1, 3.0, 5.0, 0, 0, 0, 1.2, EPS], None)
+        er, fr, _, field = reciprocal(pos, q, cell, kcells(cell, 5.0), 5.0, 1.2)
+        f, _ = oracle.evaluate("forces", *args)
+        assert abs(got[0] - oracle.evaluate("energy", *args) - er) <= TOL * abs(got[0])
+        assert rel_maxnorm(got[1], f + fr) <= TOL
+        assert rel_maxnorm(got[2], oracle.evaluate("enegs", *args) - field) <= TOL
+        fresh.close()
     eng.close()
