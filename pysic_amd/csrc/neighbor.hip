@@ -247,10 +247,13 @@ __global__ void k_scan_blocks(int nb, int *__restrict__ blk, int *__restrict__ o
 }
 
 // The whole scan in one block, for at most SCAN_ONE bins, where the pair above
-// is two launches of little work (2,000 bins: 7.5 -> 4.5 us).  The arrays are
+// is two launches of little work (2,000 bins: 7.5 -> 4.5 us).  Above, the block
+// is one compute unit's work where the pair's are the chip's: an MD step with
+// the pair and with the block, 8,000 bins 43.5 and 42.3 us, 9,261 44.6 and 45.6,
+// 29,791 59.9 and 76.9, 64,000 91 and 130.  The arrays are
 // padded to whole int4 per thread; the block totals that bin_start adds are
 // zeros here.
-constexpr int SCAN_ONE = 1 << 16;
+constexpr int SCAN_ONE = 1 << 13;
 __global__ __launch_bounds__(1024) void k_scan_one(int per4, int4 *__restrict__ in,
                                                    int4 *__restrict__ out,
                                                    int4 *__restrict__ fill, int nblk,

@@ -62,3 +62,56 @@ def test_lists_are_the_per_atom_scans(oracle, k):
         eng.close()
     for x, y in zip(got[0], got[1]):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("bins", [(16, 16, 32), (16, 17, 32), (32, 32, 16), (64, 32, 33)])
+def test_lists_around_the_one_block_scan(oracle, bins):
+    """The bins' scan is one block's work up to 8,192 of them."""
+    from pysic_amd.engine import Engine
+    n, rc = 6000, 2.5
+    print("case: %d bins" % np.prod(bins), flush=True)
+    cell = np.diag((np.array(bins) + 0.5) * rc)
+    pos = np.random.default_rng(sum(bins)).random((n, 3)) @ cell
+    eng = Engine(0)
+    eng.create_atoms(np.zeros(n, np.int32), pos)
+    eng.create_cell(cell)
+    eng.set_potentials(np.zeros((0, 12)))
+    eng.set_bond_order_factors(np.zeros((0, 14)))
+    eng.ewald_off()
+    for k in range(3):   # the third build follows two sorts with atoms changing bins
+        p = pos + 1.3 * k
+        eng.update_coordinates(p)
+        eng.generate_neighbor_lists(np.full(n, rc))
+        assert_same_pairs(eng, oracle.neighbor_list(p, cell, [1, 1, 1], np.full(n, rc)))
+    eng.close()
+
+
+def test_the_scan_of_many_bins_uses_the_chip():
+    """A step of 140,608 atoms (64,000 bins) is no longer than one of 262,144
+    (122,500 bins): in one block the scan alone took 40 of its 130 us."""
+    import time
+    from pysic_amd import structures as st
+    from pysic_amd.engine import Engine
+    from helpers import tersoff_descriptors
+    pd, bd = tersoff_descriptors()
+    step = {}
+    for reps in ((26, 26, 26), (32, 32, 32)):
+        s = st.maxwell_boltzmann(st.diamond_si(reps, sigma=0.1, seed=1), 600.0, 2)
+        n = len(s)
+        print("case: step of %d atoms" % n, flush=True)
+        eng = Engine(0)
+        eng.create_atoms(np.zeros(n, np.int32), s.positions, masses=s.masses, momenta=s.momenta)
+        eng.create_cell(s.cell)
+        eng.set_potentials(pd)
+        eng.set_bond_order_factors(bd)
+        eng.ewald_off()
+        eng.generate_neighbor_lists(np.full(n, 3.5))
+        times = []
+        for _ in range(9):
+            t = time.perf_counter()
+            eng.md_run(40, 0.02, rebuild=1)
+            times.append(time.perf_counter() - t)
+        step[n] = np.median(times[2:]) / 40
+        eng.close()
+    print({n: round(1e6 * t, 1) for n, t in step.items()}, flush=True)
+    assert step[140608] < step[262144]
