@@ -182,8 +182,11 @@ const char *pysic_kernel_variant_name(int variant);
 int pysic_set_neighbor_capacity(pysic_ctx *h, int cap);
 /* neighbor scan: 0 auto, 1 per-atom scan from global memory, 2 LDS-staged
  * bricks, 3 bricks with no LDS room (the global-memory fallback of 2),
- * 4 lane-parallel scan over x-contiguous bin columns, 5 per-atom scan with an
- * FP32 prefilter and the exact FP64 test on survivors (0 selects 5) */
+ * 4 lane-parallel scan with an FP32 prefilter and the exact FP64 test on
+ * survivors, 5 per-atom scan with the same tests where bins hold few atoms,
+ * else as 4.  0 selects 4 for one cell of less than 2^17 atoms or of more
+ * than 10/3 atoms a bin, else 5; cells thinner than the cutoff always take 4.
+ * The lists are the same by any of them. */
 int pysic_set_neighbor_method(pysic_ctx *h, int method);
 int pysic_timing(pysic_ctx *h, int on);
 /* per kernel family: name, accumulated ms, launch count; returns the count */

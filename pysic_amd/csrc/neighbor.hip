@@ -1349,14 +1349,17 @@ void nb_build_lists(System &S)
     // at any size, is the lane-parallel scan.  Sparse bins (silicon at 3.5 A):
     // 64,000 atoms 23 us against 34 with a thread per atom, 140,608 43 against
     // 38, 1,048,576 271 against 125.  Dense bins: 262,144 ions at 10.5 A 737
-    // against 1915, 1,048,576 argon atoms at 9.0 A 1303 against 1830.
+    // against 1915, 1,048,576 argon atoms at 9.0 A 1303 against 1830; method 5
+    // asked for takes it there too (16,384 argon atoms 34 us against 840 with a
+    // thread per atom, 397,808 478 against 2034).
     // a cell thinner than the cutoff: the lane-parallel scan that searches
     // several bins on each side
     const bool thin = S.ncells == 0 && (g.reach[0] > 1 || g.reach[1] > 1 || g.reach[2] > 1);
     const bool sparse = apb * 3.0 <= 10.0;
-    const int method =
-        ((S.nb_method == 0 && S.ncells == 0 && (n < (1 << 17) || !sparse)) || thin) ? 4
-                                                                                    : S.nb_method;
+    const bool lanes = S.ncells == 0 && (S.nb_method == 0   ? n < (1 << 17) || !sparse
+                                         : S.nb_method == 5 ? !sparse
+                                                            : false);
+    const int method = lanes || thin ? 4 : S.nb_method;
     bool brick = method == 2 || method == 3;
     hipEvent_t ev;
     S.timer.begin("neighbors", st, &ev);

@@ -99,8 +99,8 @@ struct System {
 
     // neighbor lists (column-major: entry e of atom i at e*n + i)
     int cap = 0;
-    int nb_method = 0;          // 0 auto (= 5), 1 global scan, 2 LDS bricks, 3 bricks w/o LDS room,
-                                // 4 lane groups, 5 FP32-prefiltered scan
+    int nb_method = 0;          // 0 auto (4 or 5), 1 global scan, 2 LDS bricks, 3 bricks w/o LDS
+                                // room, 4 lane groups, 5 FP32-prefiltered scan
     DBuf<int> nwrap;        // per atom: some list entry is in another image than 0
     bool nwrap_on = false;  // nwrap belongs to the lists (else any entry may be)
     DBuf<int> nbr, nimg, ncnt;

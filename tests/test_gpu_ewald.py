@@ -87,13 +87,13 @@ def test_rocksalt_8x8x8_rc10(eng, oracle):
     check(eng, oracle, sp, s.positions, s.charges, s.cell, np.zeros((0, 10)), ew)
 
 
-def test_dense_bin_neighbor_scan(eng, oracle):
-    """The neighbor scan taken for large dense cells (Ewald and LJ lists):
-    the per-atom FP32-prefiltered scan with its wave-uniform stencil union
-    (method 5; picked by default from 2^17 atoms).  Rocksalt 8^3 at
-    rc + skin = 10.5 A has 4 bins per axis and 64 ions per bin, which selects
-    the dense instance.  The sorted (i, j, offset) set must equal the
-    oracle's bit for bit, and E, F, W and chi must agree to 1e-9."""
+@pytest.mark.parametrize("method", [0, 5])
+def test_dense_bin_neighbor_scan(eng, oracle, method):
+    """The neighbor scan of dense bins (Ewald and LJ lists): 16 lanes an atom
+    take the candidates of its 27 bins, by default and where the per-atom
+    prefiltered scan is asked for.  Rocksalt 8^3 at rc + skin = 10.5 A has 4
+    bins per axis and 64 ions per bin.  The sorted (i, j, offset) set must
+    equal the oracle's bit for bit, and E, F, W and chi must agree to 1e-9."""
     s = st.rocksalt((8, 8, 8), sigma=0.08, seed=15)
     rc, sigma, kc = 10.0, 2.04430, 2.5713
     K = kcells(s.cell, kc)
@@ -101,8 +101,8 @@ def test_dense_bin_neighbor_scan(eng, oracle):
     sp = (s.charges < 0).astype(np.int32)
     L = np.linalg.norm(s.cell, axis=1)
     bins = np.floor(L / (rc + 0.5))
-    assert bins.min() >= 3 and len(s) / bins.prod() >= 6  # the dense instance's condition
-    eng.set_neighbor_method(5)
+    assert bins.min() >= 3 and 3 * len(s) / bins.prod() > 10  # the dense bins' condition
+    eng.set_neighbor_method(method)
     try:
         check(eng, oracle, sp, s.positions, s.charges, s.cell, np.zeros((0, 10)), ew)
         # a triclinic replica: bins and wrapped images along sheared axes

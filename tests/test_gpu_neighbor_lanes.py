@@ -1,5 +1,5 @@
-"""The lane-parallel neighbor scan of one cell below 2^17 atoms (and any size where bins are dense; its 27 bins
-as one stream) against the per-atom scan: the same lists entry by entry, in
+"""The lane-parallel neighbor scan of one cell below 2^17 atoms and of any size
+where bins are dense (its 27 bins as one stream) against the per-atom scan: the same lists entry by entry, in
 the same order, and the oracle's as sets.  Cells of one, two and more bins an
 axis, open axes with atoms outside the box, atoms several cells away, sparse
 and dense bins (8 and 16 lanes an atom), and per-atom radii."""
@@ -115,3 +115,36 @@ def test_the_scan_of_many_bins_uses_the_chip():
         eng.close()
     print({n: round(1e6 * t, 1) for n, t in step.items()}, flush=True)
     assert step[140608] < step[262144]
+
+
+@pytest.mark.parametrize("pbc", [(1, 1, 1), (0, 0, 0)])
+def test_dense_bins_are_not_one_threads_work(pbc):
+    """Where bins are dense, the per-atom prefiltered scan asked for by its
+    number is the lane-parallel one: the default's lists, entry by entry, in
+    the default's time (a thread per atom takes 10 to 20 times as long)."""
+    from pysic_amd import structures as st
+    from pysic_amd.engine import Engine
+    s = st.fcc((16, 16, 16), a=5.26, sigma=0.05, seed=1)
+    n = len(s)
+    times, lists = {}, {}
+    for method in (0, 5):
+        print("case: method %d pbc %s" % (method, pbc), flush=True)
+        eng = Engine(0)
+        eng.create_atoms(np.zeros(n, np.int32), s.positions)
+        eng.create_cell(s.cell, pbc)
+        eng.set_potentials(np.zeros((0, 12)))
+        eng.set_bond_order_factors(np.zeros((0, 14)))
+        eng.ewald_off()
+        eng.set_neighbor_method(method)
+        eng.generate_neighbor_lists(np.full(n, 9.0))
+        lists[method] = eng.neighbor_lists()
+        eng.timing(True)
+        for _ in range(10):
+            eng.generate_neighbor_lists(np.full(n, 9.0))
+        ms, calls = eng.timing_read()["neighbors"]
+        times[method] = ms / calls
+        eng.close()
+    for x, y in zip(lists[0], lists[5]):
+        assert np.array_equal(x, y)
+    print(times, flush=True)
+    assert times[5] < 3.0 * times[0]
