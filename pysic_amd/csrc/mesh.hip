@@ -10,10 +10,13 @@
 // the direct sum's (same set, same cutoff test), so nothing is truncated
 // but the kernel's tail: with a window of W = 16 points, a mesh of at least
 // 4 K + 4 points per axis and the kernel
-//   phi(x) = exp(beta (sqrt(1 - (2x/W)^2) - 1)), beta = 2.45 W
+//   phi(x) = exp(beta (sqrt(1 - (2x/W)^2) - 1)), beta = 2.55 W
 // (Barnett, Magland & af Klinteberg, SIAM J. Sci. Comput. 41, 2019), the
-// error against extended precision equals the direct FP64 sum's (1,000 and
-// 2,744 ions: forces 8.9e-15 and 1.2e-14 against 1.0e-14 and 1.4e-14).
+// error against extended precision is the direct FP64 sum's: reciprocal forces
+// of disordered ions, 2,500 of K = 28 1.8e-15 against 1.2 to 1.7e-15, 1,200 of
+// K = 47 3.6e-15 against 3.5e-15; electronegativities 6e-16 against 8e-16.
+// A smaller beta leaves a larger tail, which the forces of the long waves show,
+// n / k of it (2.45 W: 5.3e-15 and 5e-15); a larger one costs the band edge.
 //
 // Everything is FP64 and free of atomics on values: each mesh tile sums its
 // atoms in a fixed order, each atom sums its tiles in a fixed order.
@@ -44,7 +47,7 @@ namespace {
 typedef double mfma_d4 __attribute__((ext_vector_type(4)));
 
 constexpr int W = 16;                       // window points per axis
-constexpr double BETA = 2.45 * W;
+constexpr double BETA = 2.55 * W;
 constexpr int TX = 16, TY = 8, TZ = 8;      // mesh tile of one wave
 constexpr int SLOTS = 18;                   // tiles an atom can meet: 2 x 3 x 3
 constexpr int MB = 256;
@@ -153,8 +156,8 @@ __global__ __launch_bounds__(64) void k_mesh_order(const int *__restrict__ start
 // each axis: w[a * 48 + 16 d + o].  The distance to the first window point
 // is one fma, so it carries no error of the mesh coordinate's size, and the
 // exponent is written without the cancellation of sqrt - 1.  The derivative
-// has an integrable 1/sqrt edge where phi is e^-beta = 9e-18; the root is
-// held at 1e-2 there, which changes dphi by less than 1e-14.
+// has an integrable 1/sqrt edge where phi is e^-beta = 2e-18; the root is
+// held at 1e-2 there, which changes dphi by some 1e-15.
 // at[a] = (window origin on the mesh, slot).
 template <bool D>
 __global__ __launch_bounds__(MB) void k_mesh_weights(int n, MeshGeo g,
@@ -817,12 +820,23 @@ __global__ void k_mesh_zero(int m, int *__restrict__ a)
 
 int round_up(int x, int m) { return (x + m - 1) / m * m; }
 
-// mesh points of axis d for k-vectors up to K: whole tiles, and enough of them
-// that a window meets none twice
-int mesh_points(int K, int d)
+// What the sum has decayed to at the band edge of axis d.
+double band_decay(const CellGeom &c, const EwaldParams &P, int d)
+{
+    const double *v = c.v + 3 * d;
+    const double len = std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+    const double k = std::min(P.kc, 8.0 * std::atan(1.0) * P.K[d] / len);
+    return std::exp(-0.5 * P.sigma * P.sigma * k * k);
+}
+
+// Mesh points of axis d: 4 K + 4, where aliasing leaves 3e-10 of a term at the
+// band edge (2e-17 at half of it), if the sum has decayed to 3e-6 there, else
+// 4.5 K + 4, where it leaves 6e-12.
+int mesh_points(const CellGeom &c, const EwaldParams &P, int d)
 {
     const int least[3] = {2 * TX, 3 * TY, 3 * TZ}, tile[3] = {TX, TY, TZ};
-    return round_up(std::max(4 * K + 4, least[d]), tile[d]);
+    const int K = P.K[d], n = band_decay(c, P, d) <= 3e-6 ? 4 * K + 4 : (9 * K + 1) / 2 + 4;
+    return round_up(std::max(n, least[d]), tile[d]);
 }
 
 // ints that k_mesh_scan reads for nbins counts: whole int4 for 1024 threads
@@ -989,22 +1003,18 @@ bool mesh_suits(System &S, const EwaldParams &P, MeshState &M, const double *f, 
     const double pi = 4.0 * std::atan(1.0), n = S.n;
     const int tile[3] = {TX, TY, TZ};
     MeshGeo g;
-    double box = 1.0, points = 1.0, lowest = P.kc;
+    double box = 1.0, points = 1.0, decay = 0.0;
     for (int d = 0; d < 3; ++d) {
-        g.n[d] = mesh_points(P.K[d], d);
+        g.n[d] = mesh_points(S.geom, P, d);
         g.nb[d] = g.n[d] / tile[d];
         box *= d == 2 ? P.K[d] + 1 : 2 * P.K[d] + 1;
         points *= g.n[d];
-        const double *v = S.geom.v + 3 * d;
-        const double len = std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-        lowest = std::min(lowest, 2.0 * pi * P.K[d] / len);
+        decay = std::max(decay, band_decay(S.geom, P, d));
     }
     for (int c = 0; c < 9; ++c) g.f[c] = f[c];
     const double nk = std::min(box, volume * P.kc * P.kc * P.kc / (12.0 * pi * pi));
-    // The kernel's aliasing error grows to 2e-11 of a term at the mesh's band
-    // edge (it is 6e-17 at half of it), so the sum has to have decayed there.
-    const bool decayed = std::exp(-0.5 * P.sigma * P.sigma * lowest * lowest) <= 1e-4;
-    if (!decayed || !(n * nk >= MESH_MIN_PAIRS) || points > 268435456.0) return false;
+    // (what has not decayed at the band edge would need a finer mesh yet)
+    if (decay > 1e-4 || !(n * nk >= MESH_MIN_PAIRS) || points > 268435456.0) return false;
     const double direct = 75.0 + 2e-4 * nk + 4.2e-7 * n * nk + 5e-3 * n;
     auto mesh = [&](double met) {   // ions that the most crowded tile meets
         return 60.0 + 2e-5 * points + std::max(0.25 * met, 3.3e-3 * n);
@@ -1073,7 +1083,7 @@ void mesh_plan(System &S, const EwaldParams &P, MeshState &M, const double *b, d
     bool same = M.tables;
     M.tables = false;
     for (int d = 0; d < 3; ++d) {
-        const int n = mesh_points(P.K[d], d);
+        const int n = mesh_points(S.geom, P, d);
         same = same && M.K[d] == P.K[d] && M.n[d] == n;
         M.K[d] = P.K[d];
         M.n[d] = n;

@@ -218,6 +218,48 @@ def _new_cell(eng, pos, cell, kc, sigma=1.2, rc=3.0):
     eng.generate_neighbor_lists(np.full(len(pos), rc + 0.2))
 
 
+def test_forces_of_long_waves():
+    """Forces of disordered ions whose sum has decayed far inside the mesh's
+    band, so that the longest waves carry them, against the same terms in
+    extended precision.  Bound: along one axis of n = 120 points the derivative
+    of the wave k = 1 is off by 1.1e-15 of it by the kernel's tail (2.6e-18 in
+    its transform) and by n / (2 pi) / 2 eps / 2 = 1.0e-15 by the rounding of
+    products that cancel: 1.5e-15; the other two components of its gradient,
+    which vanish, by as much: sqrt(3) of it, 2.6e-15, for the longest wave and
+    less for the others.  (A kernel of a tail of 1.8e-17 gave 8.4e-15.)"""
+    n, edge, kc = 3000, 36.0, 5.0
+    pos, q = _ions_of(n, (edge,) * 3, (1, 1, 1))
+    q -= q.mean()
+    sigma = 27.0 / kc     # 1e-18 at a third of the band
+    eng = _engine(pos, q, np.eye(3) * edge, kc, sigma, 1e-3)
+    f = eng.forces()[0]
+    assert went_over_the_mesh(eng, eng.electronegativities)
+    eng.close()
+    ld = np.longdouble
+    pi, K = 4 * np.arctan(ld(1)), 10
+    b = 2 * pi / ld(edge)
+    k = [np.arange(-K, K + 1), np.arange(-K, K + 1), np.arange(0, K + 1)]
+    ex = []
+    for a in range(3):
+        turn = (pos[:, a].astype(ld) / ld(edge))[:, None] * k[a]
+        ex.append(np.exp(2j * pi * (turn - np.rint(turn))))
+    want = np.zeros((n, 3), ld)
+    for x, k1 in enumerate(k[0]):
+        k2 = b * b * (k1 * k1 + k[1][:, None] ** 2 + k[2][None] ** 2)
+        on = k2 > 0
+        c = np.where(on, np.where(k[2] == 0, 1, 2)[None] * np.exp(-ld(sigma) ** 2 * k2 / 2) /
+                     np.where(on, k2, 1), 0) / (2 * ld(edge) ** 3 * ld(EPS))
+        e12 = ex[0][:, x:x + 1] * ex[1]
+        z = 2 * c * np.einsum("ij,ik->jk", q[:, None] * e12, ex[2])
+        at = np.einsum("ik,jk->ij", ex[2].conj(), z) * e12.conj()
+        at3 = np.einsum("ik,jk->ij", ex[2].conj() * (k[2] * b), z) * e12.conj()
+        for d, y in enumerate((at.sum(1) * (k1 * b), (at * (k[1] * b)).sum(1), at3.sum(1))):
+            want[:, d] -= q * (y * -1j).real
+    error = float(np.sqrt(((f - want) ** 2).sum() / (want ** 2).sum()))
+    print("long waves: relative error %.2e" % error, flush=True)
+    assert error <= 2.6e-15
+
+
 def test_tables_follow_the_cell():
     """The transforms' tables are kept while the k-vector counts stay and
     shared by equal axes: over a strain, new counts, axes of other lengths and
