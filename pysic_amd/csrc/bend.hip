@@ -329,15 +329,20 @@ int bend_blocks(const System &S)
     return S.pmodel.nbend > 0 ? div_up(S.n * BG_LANES * BG_PARTS, BB) : 0;
 }
 
+void bend_room(System &S)
+{
+    const size_t cap = (size_t)S.cap * S.n;
+    S.bsj.ensure(cap);
+    S.bsimg.ensure(cap);
+    S.bscnt.ensure(S.n);
+    S.bG.ensure(cap);
+}
+
 // up to the gather: short lists, each vertex's angles, their partials
 void bend_sites(System &S, int mode, int blk0, hipStream_t stream)
 {
     const int n = S.n, nb = div_up(n, BB), na = bend_blocks(S);
-    const size_t cap = (size_t)S.cap * n;
-    S.bsj.ensure(cap);
-    S.bsimg.ensure(cap);
-    S.bscnt.ensure(n);
-    S.bG.ensure(cap);
+    bend_room(S);
     with_geo(S, [&](auto geo) {
         using Geo = decltype(geo);
         k_bend_list<Geo><<<nb, BB, 0, stream>>>(n, geo, S.pos.p, S.nbr.p, S.nimg.p, S.ncnt.p,

@@ -1292,6 +1292,10 @@ void pr_eval(System &S, int mode, bool accumulate, double half_dt, int kick)
     }
     const bool side = (bb || ob) && !S.timer.on && S.n <= PAIR_LANES_MAX_ATOMS;
     if (side) {
+        // all memory before the fork: an allocation that fails after it would
+        // leave a side stream at work that nothing waits for
+        if (ob) bop_room(S);
+        if (bb) bend_room(S);
         sys_fork(S, 0, bb > 0);
         sys_fork(S, 1, ob > 0);
         if (ob) bop_sites(S, mode, nb + bb, S.side[1]);   // the longest chain first
@@ -1360,16 +1364,21 @@ int bop_blocks(const System &S, int mode)
     return mode == PAIR_ENERGY ? nb : 2 * nb;
 }
 
+void bop_room(System &S)
+{
+    const size_t cap = (size_t)S.cap * S.n;
+    S.osj.ensure(cap);
+    S.osimg.ensure(cap);
+    S.oscnt.ensure(S.n);
+    S.oD.ensure(cap);
+    S.oW.ensure(cap);
+    S.oown.ensure(S.n);
+}
+
 static void bop_prepare(System &S, hipStream_t stream)
 {
     const int n = S.n;
-    const size_t cap = (size_t)S.cap * n;
-    S.osj.ensure(cap);
-    S.osimg.ensure(cap);
-    S.oscnt.ensure(n);
-    S.oD.ensure(cap);
-    S.oW.ensure(cap);
-    S.oown.ensure(n);
+    bop_room(S);
     with_geo(S, [&](auto geo) {
         k_bop_list<decltype(geo)><<<div_up(n, PB), PB, 0, stream>>>(
             n, geo, S.pos.p, S.nbr.p, S.nimg.p, S.ncnt.p, S.bmodel.radius, S.osj.p, S.osimg.p,

@@ -222,13 +222,15 @@ void pr_chi(System &S, double *chi);
 // [blk0, blk0 + blocks), forces added into frc (then p += half_dt F if kick)
 void bend_eval(System &S, int mode, int blk0, double half_dt, int kick);
 // the same in two parts: everything up to the gather on any stream, the gather
-// (forces and kick) on the main one
+// (forces and kick) on the main one; room: the first part's memory, ahead of it
+void bend_room(System &S);
 void bend_sites(System &S, int mode, int blk0, hipStream_t stream);
 void bend_gather(System &S, int mode, double half_dt, int kick);
 int bend_blocks(const System &S);
 // bond-order-scaled pair potentials: the same contract as bend_eval, and
 // their share of chi
 void bop_eval(System &S, int mode, int blk0, double half_dt, int kick);
+void bop_room(System &S);
 void bop_sites(System &S, int mode, int blk0, hipStream_t stream);
 void bop_gather(System &S, int mode, double half_dt, int kick);
 int bop_blocks(const System &S, int mode);
