@@ -143,16 +143,23 @@ void System::release_all()
         side[k] = nullptr;
         forked[k] = joined[k] = nullptr;
     }
+    evaluations = 0;
     order_valid = false;
     bins_clean = false;
+}
+
+void sys_sides(System &S)
+{
+    for (int k = 0; k < 2; ++k) {
+        for (hipEvent_t *e : {&S.forked[k], &S.joined[k]})
+            if (!*e) HIP_TRY(hipEventCreateWithFlags(e, hipEventDisableTiming));
+        if (!S.side[k]) HIP_TRY(hipStreamCreate(&S.side[k]));
+    }
 }
 
 void sys_fork(System &S, int k, bool on)
 {
     if (!on) return;
-    if (!S.side[k]) HIP_TRY(hipStreamCreate(&S.side[k]));
-    for (hipEvent_t *e : {&S.forked[k], &S.joined[k]})
-        if (!*e) HIP_TRY(hipEventCreateWithFlags(e, hipEventDisableTiming));
     HIP_TRY(hipEventRecord(S.forked[k], S.stream));
     HIP_TRY(hipStreamWaitEvent(S.side[k], S.forked[k], 0));
 }
@@ -679,7 +686,10 @@ void local_forces(pysic_ctx *h)
     const bool gen = has_gen(S);
     if (S.model.has_pairs) tersoff_checked(h, SITE_FORCES);
     else if (!gen) k_zero4<<<div_up(S.n, 256), 256, 0, S.stream>>>(S.n, S.frc.p);
-    if (gen) pr_eval(S, PAIR_FORCES, S.model.has_pairs != 0);
+    if (gen) {
+        pr_sides(S, 1);
+        pr_eval(S, PAIR_FORCES, S.model.has_pairs != 0);
+    }
 }
 
 // The forces of a velocity-Verlet step (no virial), with the second
@@ -1259,6 +1269,7 @@ int pysic_calculate_energy(pysic_ctx *h, double *energy)
         e += r.t[0];
     }
     if (has_gen(S)) {
+        pr_sides(S, 1);
         pr_eval(S, PAIR_ENERGY, false);
         sys_post_report(S, false, true);
         HIP_TRY(hipStreamSynchronize(S.stream));
@@ -1469,6 +1480,7 @@ int pysic_md_run(pysic_ctx *h, int nsteps, double dt, int rebuild, double *energ
     HIP_TRY(hipMemsetAsync(S.flags.p, 0, sizeof(int) * 4, S.stream));
     DBuf<double> ebuf;
     if (energies) ebuf.ensure(nsteps > 0 ? nsteps : 1);
+    if (has_gen(S)) pr_sides(S, nsteps);
     if (!h->forces_valid) local_forces(h);
     HIP_TRY(hipMemsetAsync(S.flags.p, 0, sizeof(int) * 4, S.stream));
     const double half = 0.5 * dt;

@@ -29,6 +29,7 @@
 // evaluated only when the model has a step factor.
 #include "system.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -1263,6 +1264,16 @@ __global__ __launch_bounds__(PB) void k_bop_gather(int n, const int *__restrict_
 
 }  // namespace
 
+// The side streams of pr_eval are made once a handle has shown that it is used
+// again, by its third evaluation or by dynamics: a new handle's energy and
+// forces of 768 COMB atoms take 1.06 ms without them and 1.19 to 1.26 with.
+void pr_sides(System &S, int count)
+{
+    S.evaluations += std::min(count, 3);
+    if (S.side[1] || S.evaluations < 3 || S.n > PAIR_LANES_MAX_ATOMS) return;
+    if (S.pmodel.nbend > 0 || S.bmodel.on) sys_sides(S);
+}
+
 void pr_eval(System &S, int mode, bool accumulate, double half_dt, int kick)
 {
     PYSIC_REQUIRE(S.dpmodel.p && S.tables.p, PYSIC_ESTATE, "pair model not compiled");
@@ -1290,7 +1301,7 @@ void pr_eval(System &S, int mode, bool accumulate, double half_dt, int kick)
                                                                             S.q.p, S.qhalf.p);
         HIP_TRY(hipGetLastError());
     }
-    const bool side = (bb || ob) && !S.timer.on && S.n <= PAIR_LANES_MAX_ATOMS;
+    const bool side = (bb || ob) && S.side[1] && !S.timer.on && S.n <= PAIR_LANES_MAX_ATOMS;
     if (side) {
         // all memory before the fork: an allocation that fails after it would
         // leave a side stream at work that nothing waits for

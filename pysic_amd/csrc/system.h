@@ -66,6 +66,7 @@ struct System {
     // streams for work beside the main stream's, always joined back into it
     // within the call that forked them (graph capture follows the events)
     hipStream_t side[2] = {nullptr, nullptr};
+    int evaluations = 0;        // asked of the general pair model (pr_sides)
     hipEvent_t forked[2] = {nullptr, nullptr}, joined[2] = {nullptr, nullptr};
     int device = 0;
     HostLink link;
@@ -218,6 +219,8 @@ enum { PAIR_ENERGY = 0, PAIR_FORCES = 1, PAIR_FORCES_ONLY = 2 };
 void pr_eval(System &S, int mode, bool accumulate, double half_dt = 0.0, int kick = 0);
 // chi += the charge-dependent pair terms' -dE/dq (nothing without them)
 void pr_chi(System &S, double *chi);
+// ahead of `count` evaluations outside a capture: whether they use side streams
+void pr_sides(System &S, int count);
 // bond_bend angles: energy / virial partials into gpartial blocks
 // [blk0, blk0 + blocks), forces added into frc (then p += half_dt F if kick)
 void bend_eval(System &S, int mode, int blk0, double half_dt, int kick);
@@ -256,6 +259,8 @@ double *sys_mail(System &S);
 void sys_post_report(System &S, bool tersoff, bool general);
 Report sys_read_report(System &S);
 
+// makes the side streams and their events (never under capture)
+void sys_sides(System &S);
 // side stream k waits for what the main stream holds now; the main stream
 // waits for what side stream k holds now (nothing if !on)
 void sys_fork(System &S, int k, bool on);

@@ -80,3 +80,46 @@ def test_angle_legs(eng, oracle, rows):
                        parameters=[1.0 + k, 1.8 + 0.2 * k, 1 + k % 2, 2])
              for k, r in enumerate(rows)]
     check(eng, oracle, s, model, 4.0, np.zeros(len(s)))
+
+
+def test_streams_beside_the_main_one():
+    """A handle's third evaluation, or its dynamics, put the angles and the
+    bond-order pairs on streams of their own: the same bits before and after,
+    and with the kernels timed, where all is serial again."""
+    from pysic_amd.engine import Engine
+    s = st.amorphous_sio2(200, 2.2, seed=8)
+    st.maxwell_boltzmann(s, 300.0, 5)
+    q = comb_charges(s.symbols, 9)
+    n = len(s)
+    pd, bd, _ = build_descriptors(comb_sio2(), {"O": 0, "Si": 1})
+    sp = np.array([("O", "Si").index(x) for x in s.symbols], np.int32)
+
+    def handle():
+        e = Engine(0)
+        e.create_atoms(sp, s.positions, masses=s.masses, charges=q, momenta=s.momenta)
+        e.create_cell(s.cell, (True, True, True))
+        e.set_potentials(pd)
+        e.set_bond_order_factors(bd)
+        e.ewald_off()
+        e.set_neighbor_capacity(48)
+        e.generate_neighbor_lists(np.full(n, 3.55))
+        return e
+
+    a, b = handle(), handle()
+    first = a.energy(), a.forces()                       # serial
+    for timed in (False, False, True, False):            # streams
+        a.timing(timed)
+        again = a.energy(), a.forces()
+        assert again[0] == first[0]
+        assert all(np.array_equal(x, y) for x, y in zip(again[1], first[1]))
+    # dynamics of a handle that has evaluated and of one that has not
+    for e in (a, b):
+        e.md_run(6, 0.02, rebuild=1)
+    for x, y in zip(a.state(), b.state()):
+        assert np.array_equal(x, y)
+    for e in (a, b):
+        e.md_run(5, 0.02, rebuild=2)                     # eager steps
+    for x, y in zip(a.state(), b.state()):
+        assert np.array_equal(x, y)
+    a.close()
+    b.close()
