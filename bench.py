@@ -150,7 +150,8 @@ def qeq_benchmark(model_path, reps=2):
            "network_only": started(w0, 0),
            "network_only_over_cold": round(w0[0] / c[0], 4),
            "ms_per_relaxation_step": round(c[0] / c[1] * 1e3, 3),
-           "kernels_us_per_step": {k: round(v[0] / max(v[1], 1) * 1e3, 1) for k, v in tim.items()},
+           "kernels_us_per_step": {k: round(v[0] / max(v[1], 1) * 1e3, 1) for k, v in tim.items()
+                                   if k != "ewald_mesh_place"},  # once a relaxation
            "model": {k: pred.meta.get(k) for k in ("configs", "atoms_per_config", "val_rmse",
                                                     "val_maxerr", "epochs")},
            "corrector": pred.meta.get("corrector")}
@@ -351,8 +352,9 @@ def ewald_benchmark(reps=3, ref_reps=(4, 4, 4)):
     kv = g @ rec
     k2 = (kv ** 2).sum(axis=1)
     nk = int(((k2 < EWALD_KC ** 2) & (k2 > 0)).sum())
+    # one pass with the placing of the ions, a family of its own
     sk_us = tim.get("ewald_sk", (0.0, 1))
-    sk_avg = sk_us[0] / max(sk_us[1], 1) / 1e3
+    sk_avg = (sk_us[0] + tim.get("ewald_mesh_place", (0.0, 0))[0]) / max(sk_us[1], 1) / 1e3
     # algorithmic work of one structure-factor pass over the mesh: each ion's
     # charge goes to 16^3 mesh points, one FMA (2 FP64 flops) each; the
     # transforms, placing the ions and their kernel values are not counted
